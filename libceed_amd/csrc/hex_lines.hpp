@@ -15,6 +15,15 @@
 // z-contractions and the pointwise operator stay in registers on the
 // (x, y) columns, as in the column-slab kernel.
 //
+// kGeo: on a trilinear geometry the factors are not read but recomputed from
+// the element's map (hex_geo.hpp).  With the 48 bytes per point gone (1.30 of
+// the 1.49 GB of an apply at p=4, 8M DoFs) what bounds the kernel is its own
+// issue rate and the latency between its barriers, so whole wavefronts of
+// elements (geo_default_epb) and the in-place slabs count: MI355X, FP64
+// diffusion, 8M DoFs, ms per apply, stored factors / recomputed / recomputed
+// with the lines in place: p=2 0.621 / 0.462 / 0.445, p=4 0.357 / 0.254 /
+// 0.222, p=6 0.252 / 0.229 / 0.180, p=8 0.283 / 0.231 / 0.199.
+//
 // Thread t of an element's Q*Q threads plays these roles:
 //   column (qx, qy) = (t % Q, t / Q)                     z-contractions, pointwise D
 //   node column (x, y) = (t % Q, t / Q), x, y < P      gather E, scatter E^T (coalesced)
@@ -22,13 +31,16 @@
 //   y-line (qx, z) = (t % Q, t / Q), t < Q*P              B_y, B_y^T
 //   x-line (qy, qz) and y-line (qx, qz) = (t % Q, t / Q)  the collocated derivatives
 // Slabs are [z][y][x] with strides (Q*Q, Q, 1), padded at Q = 7, 8 against LDS
-// bank conflicts (line_row_stride, line_plane_stride); mass needs two per element,
-// diffusion three (the y-derivative transpose waits in registers for a barrier
-// and then takes the slab the x-derivative transpose has read: one barrier more
-// than four slabs, and a quarter less LDS, so more workgroups fit a CU).
+// bank conflicts (line_row_stride, line_plane_stride).  A line's thread reads
+// all of it before it writes and no other thread touches it in that phase, so
+// lines are contracted in place: mass needs one slab per element, diffusion
+// two (the y-lines of the derivative are read before and written after the
+// barrier that ends the x-lines' reads), against two and three with separate
+// source and target, and eleven barriers against thirteen.
 #pragma once
 
 #include "hex_fused.hpp"
+#include "hex_geo.hpp"
 
 namespace mi355 {
 
@@ -63,6 +75,15 @@ __device__ __forceinline__ double pair_swap(double x) {
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
+// Slabs per element: the line kernel contracts its lines in place (mass one,
+// diffusion two, and a third where the z-derivatives wait in LDS:
+// line_dz_in_lds); the shared pipeline below (line_element) goes back and forth.
+__host__ __device__ constexpr bool line_dz_in_lds(int Q, int ncomp, int qf, int sb, bool geo) {
+  return !geo && qf != kQfMass && ncomp == 1 && sb == 8 && Q >= 10;
+}
+__host__ __device__ constexpr int line_kernel_slabs(int Q, int ncomp, int qf, int sb, bool geo) {
+  return qf == kQfMass ? 1 : line_dz_in_lds(Q, ncomp, qf, sb, geo) ? 3 : 2;
+}
 template <int QF>
 struct LineSlabs {
   static constexpr int kSlabs = QF == kQfMass ? 2 : 3;
@@ -84,10 +105,20 @@ __host__ __device__ constexpr int line_row_stride(int Q, int sb) { return sb == 
 __host__ __device__ constexpr int line_plane_stride(int Q, int sb) { return Q == 8 ? (sb == 8 ? 72 : 73) : Q == 7 && sb == 8 ? 58 : Q * Q; }
 __host__ __device__ constexpr int line_slab_entries(int Q, int sb) { return Q * line_plane_stride(Q, sb); }
 
-template <int P, int Q, int QF, typename T>
-__host__ __device__ constexpr int hex_lines_lds_entries(int epb) {
-  return epb * LineSlabs<QF>::kSlabs * line_slab_entries(Q, (int)sizeof(T));
+// LDS bytes of a workgroup of epb elements: the slabs and, where the factors
+// are recomputed, the elements' trilinear maps behind them
+__host__ __device__ constexpr size_t line_lds_bytes(int Q, int ncomp, int qf, int sb, bool geo, int epb) {
+  const size_t slabs = (size_t)sb * epb * line_kernel_slabs(Q, ncomp, qf, sb, geo) * line_slab_entries(Q, sb);
+  return geo ? ((slabs + 15) & ~(size_t)15) + sizeof(double) * kGeoStride * (size_t)epb : slabs;
 }
+
+// Where the factors are recomputed (kGeo): once per element into the registers
+// the stored ones would be loaded into, or point by point in every component.
+// One component: at the point, the registers are worth more.  Three: once
+// where 6 Q doubles fit beside the pipeline (Q <= 7, and FP32), per component
+// above (MI355X, 4M DoFs, ms per apply, once / per component: FP64 Q=4 0.214 /
+// 0.239, Q=6 0.098 / 0.106, Q=8 0.110 / 0.104, Q=10 0.149 / 0.133).
+__host__ __device__ constexpr bool line_geo_once(int Q, int ncomp, int sb) { return ncomp > 1 && (Q <= 7 || sb == 4); }
 
 // The column's geometric factors (QC values at each of its Q points) and how
 // they are loaded: all loads issued at once and shared by the components, at
@@ -429,22 +460,25 @@ __device__ __forceinline__ void line_element(T *S0, T *S1, T *S2, int t, bool ac
 // (MI355X, 8M nodes: 0.779-0.789 vs 0.826-0.830 ms per apply).  Measured and
 // not kept: 3-component FP32 at P = 6, Q = 7 (5 waves, no spills) 4% slower;
 // FP64 3-component at P = 5, Q = 6 (4 waves, 8 VGPRs spilled) 7% slower.
-template <int P, int Q, int NCOMP, int QF, typename T>
+template <int P, int Q, int NCOMP, int QF, typename T, bool kGeo>
 constexpr int lines_min_waves() {
-  return sizeof(T) == 8 && QF == kQfDiffusion && NCOMP == 3 && P == 4 && Q == 5 ? 4 : 1;
+  return !kGeo && sizeof(T) == 8 && QF == kQfDiffusion && NCOMP == 3 && P == 4 && Q == 5 ? 4 : 1;
 }
-template <int P, int Q, int NCOMP, int QF, typename T, bool kSeg = false>
-__global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T>())) hex_apply_lines_kernel(int64_t elem_begin, int64_t elem_end, int scatter,
+template <int P, int Q, int NCOMP, int QF, typename T, bool kSeg = false, bool kGeo = false>
+__global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo>())) hex_apply_lines_kernel(int64_t elem_begin, int64_t elem_end, int scatter,
                                                                const int32_t *__restrict__ offsets, int32_t comp_stride,
                                                                const T *__restrict__ q_data, const T *__restrict__ mats,
                                                                const T *__restrict__ u, T *__restrict__ v, T *__restrict__ evec,
                                                                const int32_t *__restrict__ tpos,
                                                                const int32_t *__restrict__ elem_sys, const int32_t *__restrict__ sys_active,
-                                                               const int32_t *__restrict__ seg_start) {
+                                                               const int32_t *__restrict__ seg_start, const double *__restrict__ geo,
+                                                               const double *__restrict__ geo_pts) {
   constexpr int NT = Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QC = QfTraits<QF>::kComps;
   constexpr int SR = line_row_stride(Q, sizeof(T)), SP = line_plane_stride(Q, sizeof(T)), SLAB = Q * SP;
   static_assert(SR >= Q && SP >= Q * SR, "slab rows and planes must not overlap");
-  constexpr int NS = LineSlabs<QF>::kSlabs;
+  constexpr int NS = line_kernel_slabs(Q, NCOMP, QF, sizeof(T), kGeo);
+  constexpr bool kDzLds = line_dz_in_lds(Q, NCOMP, QF, sizeof(T), kGeo);
+  constexpr bool kOnce = line_geo_once(Q, NCOMP, sizeof(T));
   // from Q = 7 one phase's matrix entries no longer fit the SGPRs: load them
   // per output row (or column) instead of per phase
   constexpr bool kRowWise = Q >= 7;
@@ -453,10 +487,12 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T>())) 
 
   const int epb = blockDim.x / NT;
   const int le = threadIdx.x / NT, t = threadIdx.x - le * NT;
-  T        *S0 = reinterpret_cast<T *>(lds_raw) + (size_t)le * NS * SLAB;
-  T        *S1 = S0 + SLAB;
-  T        *S2 = S1 + SLAB;  // diffusion only
+  T        *X = reinterpret_cast<T *>(lds_raw) + (size_t)le * NS * SLAB;
+  T        *Y = X + SLAB;  // diffusion only
+  T        *Z = Y + SLAB;  // kDzLds only
   auto      at = [](int z, int y, int x) { return z * SP + y * SR + x; };
+  // kGeo: the element's trilinear map behind the slabs
+  double *sgeo = reinterpret_cast<double *>(lds_raw + (((size_t)epb * NS * SLAB * sizeof(T) + 15) & ~(size_t)15)) + le * kGeoStride;
 
   // the workgroup's elements: epb consecutive packed elements, or (kSeg)
   // segment elem_begin + chunk, whose consecutive elements share x-faces
@@ -467,7 +503,7 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T>())) 
   const bool    live  = le < epb && (kSeg ? le < slen : e < elem_end) && (!elem_sys || sys_active[elem_sys[e]]);
   if (elem_sys && !__syncthreads_or(live)) return;  // every element of the workgroup is frozen (uniform exit)
 
-  const int  cx = t % Q, cy = t / Q;  // column
+  const int  cx = t % Q, cy = t / Q;  // column; also the x-line (qy = cx, qz = cy) and the y-line (qx = cx, qz = cy)
   const int  ny = t % P, nz = t / P;  // x-line of nodes
   const bool xline = t < P * P;
   // E and E^T run on the node columns (cx, cy < P), like the column layout, so
@@ -478,78 +514,79 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T>())) 
 #pragma unroll
     for (int z = 0; z < P; z++) off[z] = offsets[e * P3 + (z * P + cy) * P + cx];
   }
-  // the column's geometric factors, all loads issued at once and shared by the
-  // components: at the element start (in flight during E and the
-  // interpolation), or for scalar FP64 diffusion from Q = 9 just before the
-  // pointwise operator, where 6Q doubles held through the whole element cost
-  // a wave per SIMD (191 -> 137 VGPRs at Q = 9; measured on MI355X, 8M DoFs:
-  // p=7 26.6 -> 27.6 GDoF/s, p=8 26.2 -> 27.5; later loads lose at Q <= 8
-  // and in FP32, where the exposed latency costs more than the occupancy gains)
-  constexpr bool kQdEarly = QF == kQfMass || NCOMP > 1 || Q < 9 || sizeof(T) < 8;
-  // paired 16-byte loads with the early loads of FP64 scalar diffusion, Q even
-  // (interleaved A/B on MI355X, 8M DoFs: p=4 +0.7% with colours, +3.7% with
-  // the map, p=6 +0-4% with the split; with the late loads at Q = 10 the swap
-  // in the pointwise loop cost 15%; FP32 pairs of 8-byte loads were 3-5% slower)
-  constexpr bool kPairQd = kQdEarly && sizeof(T) == 8 && QF == kQfDiffusion && NCOMP == 1 && Q % 2 == 0;
-  constexpr int  QH      = QC / 2;
-  const T       *qd       = q_data + (live ? e : 0) * (int64_t)QC * Q3 + (cy * Q + cx);
-  T              sq[kPairQd ? 1 : Q][QC];
-  line_v2<T>     sp[kPairQd ? Q : 1][kPairQd ? QH : 1];
-  auto           load_q = [&]() {
-    if constexpr (kPairQd) {  // 16-byte aligned: Q even, so (cy * Q + cx - odd) and every stride are even
-      const T *pb = q_data + (live ? e : 0) * (int64_t)QC * Q3 + (cy * Q + (cx & ~1)) + ((cx & 1) ? QH : 0) * Q3;
+  // the column's geometric factors (LineQData; kGeo: recomputed at the
+  // pointwise operator from the element's map, staged in LDS here)
+  LineQData<Q, NCOMP, QF, T> qd;
+  constexpr bool             kEarly = LineQData<Q, NCOMP, QF, T>::kEarly;
+  const T                   *qe     = q_data + (live ? e : 0) * (int64_t)QC * Q3;
+  double                     xi = 0, eta = 0, wxy = 0;
+  T                          kappa[kGeo && QF == kQfDiffusionKappa ? Q : 1];
+  if constexpr (kGeo && kOnce) {
+    GeoColumn k;
+    k.load(geo + (live ? e : 0) * kGeoStride, geo_pts[cx], geo_pts[cy]);
+    wxy = geo_pts[Q + cy] * geo_pts[Q + cx];
+    const auto gp = phase_ptr(geo_pts);
 #pragma unroll
-      for (int qz = 0; qz < Q; qz++)
+    for (int qz = 0; qz < Q; qz++) {
+      double g6[6];
+      __builtin_amdgcn_sched_barrier(0);
+      geo_poisson(k, gp[qz], gp[Q + qz] * wxy, g6);
 #pragma unroll
-        for (int kk = 0; kk < QH; kk++) sp[qz][kk] = __builtin_nontemporal_load((const line_v2<T> *)(pb + kk * Q3 + qz * Q * Q));
-    } else {
-#pragma unroll
-      for (int qz = 0; qz < Q; qz++)
-#pragma unroll
-        for (int k = 0; k < QC; k++) sq[qz][k] = __builtin_nontemporal_load(&qd[k * Q3 + qz * Q * Q]);
+      for (int i = 0; i < 6; i++) qd.sq[qz][i] = (T)g6[i];
     }
-  };
-  if constexpr (kQdEarly) load_q();
+  } else if constexpr (kGeo) {
+    for (int i = t; i < kGeoStride; i += NT) sgeo[i] = geo[(live ? e : 0) * kGeoStride + i];
+    xi  = geo_pts[cx];
+    eta = geo_pts[cy];
+    wxy = geo_pts[Q + cy] * geo_pts[Q + cx];
+    if constexpr (QF == kQfDiffusionKappa) {
+#pragma unroll
+      for (int qz = 0; qz < Q; qz++) kappa[qz] = __builtin_nontemporal_load(&qe[6 * Q3 + (qz * Q + cy) * Q + cx]);
+    }
+  } else if constexpr (kEarly) {
+    qd.load(qe, cx, cy);
+  }
 
+  // A line contraction in place needs no second slab and no synchronisation:
+  // the line's thread reads all of it before it writes, and owns it.
   for (int comp = 0; comp < NCOMP; comp++) {
     const int64_t coff = (int64_t)comp * comp_stride;
-    if (comp > 0) __syncthreads();  // the previous component's last phase still reads S0
-    // ---- E: the node column gathers its P nodes into S0
+    if (comp > 0) __syncthreads();  // the previous component's E^T still reads X
+    // ---- E: the node column gathers its P nodes into X
     if (node) {
 #pragma unroll
-      for (int z = 0; z < P; z++) S0[at(z, cy, cx)] = u[(off[z] >> 1) + coff];
+      for (int z = 0; z < P; z++) X[at(z, cy, cx)] = u[(off[z] >> 1) + coff];
     }
     __syncthreads();
-    // ---- B_x: x-line (ny, nz) of nodes, Q interpolated values into S1
+    // ---- B_x on the x-line (ny, nz) of nodes, in place
     if (xline) {
       const auto gB = phase_ptr(mats);
-      T        in[P];
+      T          in[P];
 #pragma unroll
-      for (int x = 0; x < P; x++) in[x] = S0[at(nz, ny, x)];
+      for (int x = 0; x < P; x++) in[x] = X[at(nz, ny, x)];
 #pragma unroll
       for (int qx = 0; qx < Q; qx++) {
         const auto m = kRowWise ? phase_ptr(mats + qx * P) : gB + qx * P;
-        T s = 0;
+        T          s = 0;
 #pragma unroll
         for (int b = 0; b < P; b++) s += m[b] * in[b];
-        S1[at(nz, ny, qx)] = s;
+        X[at(nz, ny, qx)] = s;
       }
     }
     __syncthreads();
-    // ---- B_y: y-line (qx, z), z < P
+    // ---- B_y on the y-line (qx = cx, z = cy < P), in place
     if (t < Q * P) {
       const auto gB = phase_ptr(mats);
-      const int qx = t % Q, z = t / Q;
-      T         in[P];
+      T          in[P];
 #pragma unroll
-      for (int b = 0; b < P; b++) in[b] = S1[at(z, b, qx)];
+      for (int b = 0; b < P; b++) in[b] = X[at(cy, b, cx)];
 #pragma unroll
       for (int qy = 0; qy < Q; qy++) {
         const auto m = kRowWise ? phase_ptr(mats + qy * P) : gB + qy * P;
-        T s = 0;
+        T          s = 0;
 #pragma unroll
         for (int b = 0; b < P; b++) s += m[b] * in[b];
-        S0[at(z, qy, qx)] = s;
+        X[at(cy, qy, cx)] = s;
       }
     }
     __syncthreads();
@@ -557,156 +594,155 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T>())) 
     T uq[Q];
     {
       const auto gB = phase_ptr(mats);
-      T        col[P];
+      T          col[P];
 #pragma unroll
-      for (int b = 0; b < P; b++) col[b] = S0[at(b, cy, cx)];
+      for (int b = 0; b < P; b++) col[b] = X[at(b, cy, cx)];
 #pragma unroll
       for (int qz = 0; qz < Q; qz++) {
         const auto m = kRowWise ? phase_ptr(mats + qz * P) : gB + qz * P;
-        T s = 0;
+        T          s = 0;
 #pragma unroll
         for (int b = 0; b < P; b++) s += m[b] * col[b];
         uq[qz] = s;
       }
     }
     if constexpr (QF == kQfMass) {
-      // ---- D, then B_z^T back into the column's own S0 entries (read only by this thread)
-      const auto gB = phase_ptr(mats);
+      // ---- D, then B_z^T back into the column's own entries
 #pragma unroll
-      for (int qz = 0; qz < Q; qz++) uq[qz] *= live ? sq[qz][0] : T(0);
+      for (int qz = 0; qz < Q; qz++) {
+        T s[QC];
+        qd.point(qz, cx, s);
+        uq[qz] *= s[0];
+      }
+      const auto gB = phase_ptr(mats);
 #pragma unroll
       for (int b = 0; b < P; b++) {
         const auto m = kRowWise ? phase_ptr(mats + b) : gB + b;
-        T s = 0;
+        T          s = 0;
 #pragma unroll
         for (int qz = 0; qz < Q; qz++) s += m[qz * P] * uq[qz];
-        S0[at(b, cy, cx)] = s;
+        X[at(b, cy, cx)] = s;
       }
     } else {
-      // ---- collocated derivatives: z on the column, x and y by lines through S1
-      const auto gD = phase_ptr(mats + Q * P);
-      T        dz[Q];
+      // ---- collocated derivatives: z on the column; x by x-lines of X into Y,
+      // y by y-lines of X in place once every x-line has been read
+      T dz[Q];
+      {
+        const auto gD = phase_ptr(mats + Q * P);
 #pragma unroll
-      for (int qz = 0; qz < Q; qz++) {
-        const auto m = kRowWise ? phase_ptr(mats + Q * P + qz * Q) : gD + qz * Q;
-        T s = 0;
+        for (int qz = 0; qz < Q; qz++) {
+          const auto m = kRowWise ? phase_ptr(mats + Q * P + qz * Q) : gD + qz * Q;
+          T          s = 0;
 #pragma unroll
-        for (int c = 0; c < Q; c++) s += m[c] * uq[c];
-        dz[qz] = s;
-        S1[at(qz, cy, cx)] = uq[qz];
+          for (int c = 0; c < Q; c++) s += m[c] * uq[c];
+          dz[qz]            = s;
+          X[at(qz, cy, cx)] = uq[qz];
+        }
       }
       __syncthreads();
       {
-        const auto gD = phase_ptr(mats + Q * P);
-        const int a = t % Q, qz = t / Q;  // x-line (qy = a, qz) and y-line (qx = a, qz)
-        T         in[Q];
+        T in[Q];
 #pragma unroll
-        for (int c = 0; c < Q; c++) in[c] = S1[at(qz, a, c)];
+        for (int c = 0; c < Q; c++) in[c] = X[at(cy, cx, c)];
+        {
+          const auto gD = phase_ptr(mats + Q * P);
 #pragma unroll
-        for (int qx = 0; qx < Q; qx++) {
-          const auto m = kRowWise ? phase_ptr(mats + Q * P + qx * Q) : gD + qx * Q;
-          T s = 0;
+          for (int qx = 0; qx < Q; qx++) {
+            const auto m = kRowWise ? phase_ptr(mats + Q * P + qx * Q) : gD + qx * Q;
+            T          s = 0;
 #pragma unroll
-          for (int c = 0; c < Q; c++) s += m[c] * in[c];
-          S2[at(qz, a, qx)] = s;
+            for (int c = 0; c < Q; c++) s += m[c] * in[c];
+            Y[at(cy, cx, qx)] = s;
+          }
         }
 #pragma unroll
-        for (int c = 0; c < Q; c++) in[c] = S1[at(qz, c, a)];
+        for (int c = 0; c < Q; c++) in[c] = X[at(cy, c, cx)];
+        __syncthreads();
+        const auto gD = phase_ptr(mats + Q * P);
 #pragma unroll
         for (int qy = 0; qy < Q; qy++) {
           const auto m = kRowWise ? phase_ptr(mats + Q * P + qy * Q) : gD + qy * Q;
-          T s = 0;
+          T          s = 0;
 #pragma unroll
           for (int c = 0; c < Q; c++) s += m[c] * in[c];
-          S0[at(qz, qy, a)] = s;
+          X[at(cy, qy, cx)] = s;
         }
       }
       __syncthreads();
-      // ---- pointwise (Poisson3DApply, times kappa for the kappa-weighted operator) on the column
-      // From Q = 10 the column's z-derivatives wait in S1 (free until D_x^T
-      // below; only this thread's entries) rather than in registers beside
-      // the late q_data loads (interleaved A/B on MI355X, 8M DoFs: p=8 0.283
-      // vs 0.293 ms; at Q = 9, p=7, 0.280 vs 0.274, so not there).
-      constexpr bool kDzLds = !kQdEarly && Q >= 10;
+      // ---- pointwise (Poisson3DApply, times kappa for the kappa-weighted operator) on the column, in place
+      // From Q = 10 the column's z-derivatives wait in a third slab (only this
+      // thread's entries) rather than in registers beside the late q_data
+      // loads (interleaved A/B on MI355X, 8M DoFs: p=8 0.283 vs 0.293 ms; at
+      // Q = 9, p=7, 0.280 vs 0.274, so not there).
       if constexpr (kDzLds) {
 #pragma unroll
-        for (int qz = 0; qz < Q; qz++) S1[at(qz, cy, cx)] = dz[qz];
+        for (int qz = 0; qz < Q; qz++) Z[at(qz, cy, cx)] = dz[qz];
       }
-      if constexpr (!kQdEarly) load_q();
+      if constexpr (!kGeo && !kEarly) qd.load(qe, cx, cy);
+      GeoColumn  k;
+      const auto gp = phase_ptr(geo_pts);
+      if constexpr (kGeo && !kOnce) k.load(sgeo, xi, eta);
       T vz[Q];
 #pragma unroll
       for (int qz = 0; qz < Q; qz++) {
-        T vx, vy, vzz;
-        if constexpr (kPairQd) {  // this column's half from the own load, the other half from the partner lane
-          const bool odd = cx & 1;
-          T          s6[QC];
+        T s[QC], vx, vy, vzz;
+        if constexpr (kGeo && !kOnce) {
+          double g6[6];
+          __builtin_amdgcn_sched_barrier(0);  // one point's factors at a time in registers (Q = 6: 92 VGPRs against 99, five waves per SIMD)
+          geo_poisson(k, gp[qz], gp[Q + qz] * wxy, g6);
 #pragma unroll
-          for (int kk = 0; kk < QH; kk++) {
-            const line_v2<T> d = sp[qz][kk];
-            const T       keep = odd ? d.y : d.x, got = pair_swap(odd ? d.x : d.y);
-            s6[kk]             = odd ? got : keep;
-            s6[QH + kk]        = odd ? keep : got;
-          }
-          poisson_regs<T>(s6, S2[at(qz, cy, cx)], S0[at(qz, cy, cx)], dz[qz], vx, vy, vzz);
+          for (int i = 0; i < 6; i++) s[i] = (T)g6[i];
+          if constexpr (QF == kQfDiffusionKappa) s[6] = kappa[qz];
         } else {
-          poisson_regs<T>(sq[qz], S2[at(qz, cy, cx)], S0[at(qz, cy, cx)], kDzLds ? S1[at(qz, cy, cx)] : dz[qz], vx, vy, vzz);
+          qd.point(qz, cx, s);
         }
+        poisson_regs<T>(s, Y[at(qz, cy, cx)], X[at(qz, cy, cx)], kDzLds ? Z[at(qz, cy, cx)] : dz[qz], vx, vy, vzz);
         if constexpr (QF == kQfDiffusionKappa) {
-          vx *= sq[qz][6];
-          vy *= sq[qz][6];
-          vzz *= sq[qz][6];
+          vx *= s[6];
+          vy *= s[6];
+          vzz *= s[6];
         }
-        if (!live) vx = vy = vzz = 0;
-        S2[at(qz, cy, cx)] = vx;
-        S0[at(qz, cy, cx)] = vy;
-        vz[qz]             = vzz;
+        Y[at(qz, cy, cx)] = vx;
+        X[at(qz, cy, cx)] = vy;
+        vz[qz]            = vzz;
       }
       __syncthreads();
-      // ---- D_x^T by x-lines into S1; D_y^T by y-lines, held in registers
-      // until every x-line has read S2, then written over it
+      // ---- D_x^T by x-lines of Y, D_y^T by y-lines of X, both in place
       {
-        const int a = t % Q, qz = t / Q;
-        T         ty[Q];
+        T in[Q];
         {
           const auto gD = phase_ptr(mats + Q * P);
-          T          in[Q];
 #pragma unroll
-          for (int c = 0; c < Q; c++) in[c] = S2[at(qz, a, c)];
+          for (int c = 0; c < Q; c++) in[c] = Y[at(cy, cx, c)];
 #pragma unroll
           for (int qx = 0; qx < Q; qx++) {
             const auto m = kRowWise ? phase_ptr(mats + Q * P + qx) : gD + qx;
-            T s = 0;
+            T          s = 0;
 #pragma unroll
             for (int c = 0; c < Q; c++) s += m[c * Q] * in[c];
-            S1[at(qz, a, qx)] = s;
+            Y[at(cy, cx, qx)] = s;
           }
         }
-        {
-          const auto gD = phase_ptr(mats + Q * P);
-          T          in[Q];
+        const auto gD = phase_ptr(mats + Q * P);
 #pragma unroll
-          for (int c = 0; c < Q; c++) in[c] = S0[at(qz, c, a)];
+        for (int c = 0; c < Q; c++) in[c] = X[at(cy, c, cx)];
 #pragma unroll
-          for (int qy = 0; qy < Q; qy++) {
-            const auto m = kRowWise ? phase_ptr(mats + Q * P + qy) : gD + qy;
-            T s = 0;
+        for (int qy = 0; qy < Q; qy++) {
+          const auto m = kRowWise ? phase_ptr(mats + Q * P + qy) : gD + qy;
+          T          s = 0;
 #pragma unroll
-            for (int c = 0; c < Q; c++) s += m[c * Q] * in[c];
-            ty[qy] = s;
-          }
+          for (int c = 0; c < Q; c++) s += m[c * Q] * in[c];
+          X[at(cy, qy, cx)] = s;
         }
-        __syncthreads();
-#pragma unroll
-        for (int qy = 0; qy < Q; qy++) S2[at(qz, qy, a)] = ty[qy];
       }
       __syncthreads();
-      // ---- sum of the three transposes on the column, then B_z^T into S0
+      // ---- sum of the three transposes on the column, then B_z^T into X
       const auto gDz = phase_ptr(mats + Q * P);
-      T        w[Q];
+      T          w[Q];
 #pragma unroll
       for (int qz = 0; qz < Q; qz++) {
         const auto m = kRowWise ? phase_ptr(mats + Q * P + qz) : gDz + qz;
-        T s = S1[at(qz, cy, cx)] + S2[at(qz, cy, cx)];
+        T          s = Y[at(qz, cy, cx)] + X[at(qz, cy, cx)];
 #pragma unroll
         for (int c = 0; c < Q; c++) s += m[c * Q] * vz[c];
         w[qz] = s;
@@ -715,43 +751,42 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T>())) 
 #pragma unroll
       for (int b = 0; b < P; b++) {
         const auto m = kRowWise ? phase_ptr(mats + b) : gBz + b;
-        T s = 0;
+        T          s = 0;
 #pragma unroll
         for (int qz = 0; qz < Q; qz++) s += m[qz * P] * w[qz];
-        S0[at(b, cy, cx)] = s;
+        X[at(b, cy, cx)] = s;
       }
     }
     __syncthreads();
-    // ---- B_y^T: y-line (qx, z), z < P, into S1
+    // ---- B_y^T on the y-line (qx = cx, z = cy < P), in place
     if (t < Q * P) {
       const auto gB = phase_ptr(mats);
-      const int qx = t % Q, z = t / Q;
-      T         in[Q];
+      T          in[Q];
 #pragma unroll
-      for (int a = 0; a < Q; a++) in[a] = S0[at(z, a, qx)];
+      for (int a = 0; a < Q; a++) in[a] = X[at(cy, a, cx)];
 #pragma unroll
       for (int y = 0; y < P; y++) {
         const auto m = kRowWise ? phase_ptr(mats + y) : gB + y;
-        T s = 0;
+        T          s = 0;
 #pragma unroll
         for (int a = 0; a < Q; a++) s += m[a * P] * in[a];
-        S1[at(z, y, qx)] = s;
+        X[at(cy, y, cx)] = s;
       }
     }
     __syncthreads();
-    // ---- B_x^T: x-line (ny, nz) of nodes, into S0 (last read by B_y^T)
+    // ---- B_x^T on the x-line (ny, nz) of nodes, in place
     if (xline) {
       const auto gB = phase_ptr(mats);
-      T        in[Q];
+      T          in[Q];
 #pragma unroll
-      for (int a = 0; a < Q; a++) in[a] = S1[at(nz, ny, a)];
+      for (int a = 0; a < Q; a++) in[a] = X[at(nz, ny, a)];
 #pragma unroll
       for (int x = 0; x < P; x++) {
-        const auto m = kRowWise ? phase_ptr(mats + x) : gB + x;
-        T acc = 0;
+        const auto m   = kRowWise ? phase_ptr(mats + x) : gB + x;
+        T          acc = 0;
 #pragma unroll
         for (int a = 0; a < Q; a++) acc += m[a * P] * in[a];
-        S0[at(nz, ny, x)] = acc;
+        X[at(nz, ny, x)] = acc;
       }
     }
     __syncthreads();
@@ -759,7 +794,7 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T>())) 
     if (node) {
       T s[P];
 #pragma unroll
-      for (int z = 0; z < P; z++) s[z] = S0[at(z, cy, cx)];
+      for (int z = 0; z < P; z++) s[z] = X[at(z, cy, cx)];
       if (!kSeg && scatter == kScatterEvec) {  // tpos gives each contribution's slot in the E-vector sorted by L entry
         int32_t pos[P];
 #pragma unroll
@@ -777,12 +812,12 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T>())) 
         }
       } else {
         // segments: the face x = P-1 also holds the next element's x = 0 face
-        // (its S0 is final after the barrier above), added after the own value;
+        // (its X is final after the barrier above), added after the own value;
         // the next element's threads of that face write nothing
         bool write = true;
         if constexpr (kSeg) {
           if (cx == P - 1 && le + 1 < slen) {
-            const T *Sn = S0 + NS * SLAB;
+            const T *Sn = X + NS * SLAB;
 #pragma unroll
             for (int z = 0; z < P; z++) s[z] += Sn[at(z, cy, 0)];
           }

@@ -16,6 +16,8 @@ struct CeedMi355Operator_private;
 
 namespace mi355 {
 
+// the line kernel with recomputed geometric factors over elements [b, e) of a plan (hex_geo_*.hip)
+using GeoLinesFn = void (*)(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, hipStream_t s);
 using ApplyFn = int (*)(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s);
 // v (=|+=) E^T evec by the plan's transpose map (operator_hex.hip)
 int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, hipStream_t s);
@@ -33,6 +35,8 @@ int brick_evec(const CeedMi355Operator_private *op, const void *evec, void *v, i
 // Kernel launcher for one (P, Q, num_comp, QF, scalar type); nullptr when no instantiation exists.
 ApplyFn pick_apply_f64(int P, int Q, int num_comp, int qf);
 ApplyFn pick_apply_f32(int P, int Q, int num_comp, int qf);
+GeoLinesFn pick_geo_f64(int P, int Q, int num_comp, int qf);
+GeoLinesFn pick_geo_f32(int P, int Q, int num_comp, int qf);
 // Thread layouts of the fused kernel: z-columns with x/y contractions read
 // point by point from LDS (hex_apply_kernel), whole 1D lines per thread for
 // the x/y contractions (hex_apply_lines_kernel), or a thread per quadrature
@@ -50,8 +54,12 @@ constexpr int kMaxLdsBytes = 160 * 1024, kDefaultLdsBytes = 64 * 1024;
 constexpr int max_threads(int) { return 256; }
 // Default elements per workgroup: for line-layout diffusion a table of measured
 // choices per Q, otherwise as many as fit 256 threads and kDefaultLdsBytes of LDS.
-int default_epb(int P, int Q, int qf, int scalar_bytes, int layout);
-int lds_bytes(int P, int Q, int qf, int epb, int scalar_bytes, int layout);
+int default_epb(int P, int Q, int qf, int num_comp, int scalar_bytes, int layout);
+// Whether a plan of this kind recomputes trilinear geometric factors in the
+// line kernel, and its elements per workgroup then (operator_hex.hip).
+bool geo_pays(int Q, int qf, int num_comp, int scalar_bytes);
+int  geo_default_epb(int Q);
+int lds_bytes(int P, int Q, int qf, int num_comp, int epb, int scalar_bytes, int layout);
 // Threads and LDS bytes of the brick kernel's workgroup for a brick of ns
 // slots (shape[0] * shape[1] * shape[2]); the kernel's own formulas in
 // hex_brick.hpp, for plan set-up on the host.
@@ -104,6 +112,7 @@ struct CeedMi355Operator_private {
   int64_t l_size;
   int     epb;
   int     layout     = 0;      // mi355::kLayoutColumns or kLayoutLines
+  bool    own_launch = false;  // layout and epb were set by the caller or the environment: kept when the factors change kind
   bool    covers_all = false;  // every L entry is reached by some element: Apply needs no zero fill
   int     scatter    = 0;      // CEED_MI355_PLAN_* E^T mode: 0 transpose map, COLOR, SPLIT, ATOMIC, BRICK, SEGMENT
   // transpose offset map (scatter == 0): contribution (elem, comp, node) is
@@ -161,6 +170,12 @@ struct CeedMi355Operator_private {
   void                *d_mats    = nullptr;  // B (Q x P) then D (Q x Q), plan scalar type
   void                *d_qdata   = nullptr;  // [elem][q_comp][Q^3], packed order
   mi355::ApplyFn       apply     = nullptr;
+  // trilinear geometry: the map's coefficients [elem][kGeoStride] in packed
+  // order and the 1D points and weights (2 Q doubles); geo_valid: d_qdata
+  // holds the factors of this geometry, which geo_lines may recompute
+  double              *d_geo = nullptr, *d_geo_pts = nullptr;
+  bool                 geo_valid = false;
+  mi355::GeoLinesFn    geo_lines = nullptr;
   CeedMi355JitKernel  *jit       = nullptr;  // kQfJit plans: the compiled kernel and the QFunction context
 };
 
@@ -172,8 +187,8 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
   const int    epb    = op->epb;
   const bool   lines  = op->layout == kLayoutLines;
   const bool   points = op->layout == kLayoutPoints;
-  const size_t lds    = sizeof(T) * (size_t)(lines ? hex_lines_lds_entries<P, Q, QF, T>(epb)
-                                                   : points ? hex_points_lds_entries<P, Q, QF>(epb) : hex_lds_entries<P, Q, QF>(epb));
+  const size_t lds    = lines ? line_lds_bytes(Q, NC, QF, sizeof(T), false, epb)
+                              : sizeof(T) * (size_t)(points ? hex_points_lds_entries<P, Q, QF>(epb) : hex_lds_entries<P, Q, QF>(epb));
   if (op->scatter == CEED_MI355_PLAN_BRICK) {
     if (op->num_bricks == 0) return CEED_MI355_SUCCESS;
     const int ns = op->brick_shape[0] * op->brick_shape[1] * op->brick_shape[2];
@@ -190,7 +205,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
         if (e <= b) continue;
         hex_apply_lines_kernel<P, Q, NC, QF, T, true><<<(unsigned)(e - b), epb * nt, lds, s>>>(
             b, e, overwrite ? kScatterOverwrite : kScatterAdd, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats,
-            (const T *)u, (T *)v, nullptr, nullptr, op->d_elem_sys, op->d_sys_active, op->d_seg_start);
+            (const T *)u, (T *)v, nullptr, nullptr, op->d_elem_sys, op->d_sys_active, op->d_seg_start, nullptr, nullptr);
       }
       MI355_LAUNCH_CHECK();
       return CEED_MI355_SUCCESS;
@@ -205,6 +220,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
     const int err = fill_zero(op, target, s);
     if (err) return err;
   }
+  const bool geo = lines && op->geo_valid && op->geo_lines && line_lds_bytes(Q, NC, QF, sizeof(T), true, epb) <= (size_t)kMaxLdsBytes;
   for (size_t c = 0; c + 1 < op->color_start.size(); c++) {
     const int64_t b = op->color_start[c], e = op->color_start[c + 1];
     if (e <= b) continue;
@@ -212,10 +228,11 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
     const int     scatter = tmap ? kScatterEvec
                                  : split ? kScatterSplit
                                          : (op->scatter == CEED_MI355_PLAN_ATOMIC ? kScatterAtomic : (overwrite ? kScatterOverwrite : kScatterAdd));
-    if (lines)
+    if (geo) op->geo_lines(op, b, e, scatter, u, target, s);
+    else if (lines)
       hex_apply_lines_kernel<P, Q, NC, QF, T><<<(unsigned)grid, epb * nt, lds, s>>>(
           b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, target, (T *)op->d_evec,
-          op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr);
+          op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, nullptr, nullptr);
     else if (points) {
       if constexpr (Q * Q * Q <= 256)
         hex_apply_points_kernel<P, Q, NC, QF, T><<<(unsigned)grid, epb * Q * Q * Q, lds, s>>>(
@@ -232,6 +249,31 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
   if (tmap) return transpose_gather(op, v, overwrite, s);
   if (split) return split_finish(op, v, overwrite, s);
   return CEED_MI355_SUCCESS;
+}
+
+template <int P, int Q, int NC, int QF, typename T>
+void launch_geo_lines(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, hipStream_t s) {
+  const int64_t epb = op->epb, grid = (e - b + epb - 1) / epb;
+  hex_apply_lines_kernel<P, Q, NC, QF, T, false, true><<<(unsigned)grid, (unsigned)(epb * Q * Q), line_lds_bytes(Q, NC, QF, sizeof(T), true, (int)epb), s>>>(
+      b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec,
+      op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, op->d_geo, op->d_geo_pts);
+}
+
+// Dispatch over the instantiated (P, Q) pairs: P = 2..9, Q in {P, P+1}.
+template <typename T>
+GeoLinesFn pick_geo(int P, int Q, int nc, int qf) {
+#define MI355_CASE_PQ(PP, QQ)                                                                                                  \
+  if (P == PP && Q == QQ) {                                                                                                    \
+    if (qf == kQfDiffusion)                                                                                                    \
+      return nc == 1 ? launch_geo_lines<PP, QQ, 1, kQfDiffusion, T> : (nc == 3 ? launch_geo_lines<PP, QQ, 3, kQfDiffusion, T> : nullptr); \
+    if (qf == kQfDiffusionKappa) return nc == 1 ? launch_geo_lines<PP, QQ, 1, kQfDiffusionKappa, T> : nullptr;                 \
+    return nullptr;                                                                                                            \
+  }
+  MI355_CASE_PQ(2, 2) MI355_CASE_PQ(2, 3) MI355_CASE_PQ(3, 3) MI355_CASE_PQ(3, 4) MI355_CASE_PQ(4, 4) MI355_CASE_PQ(4, 5)
+  MI355_CASE_PQ(5, 5) MI355_CASE_PQ(5, 6) MI355_CASE_PQ(6, 6) MI355_CASE_PQ(6, 7) MI355_CASE_PQ(7, 7) MI355_CASE_PQ(7, 8)
+  MI355_CASE_PQ(8, 8) MI355_CASE_PQ(8, 9) MI355_CASE_PQ(9, 9) MI355_CASE_PQ(9, 10)
+#undef MI355_CASE_PQ
+  return nullptr;
 }
 
 // Dispatch over the instantiated (P, Q) pairs: P = 2..9, Q in {P, P+1}.

@@ -1,10 +1,12 @@
 // Fused hex operator plans: element colouring, colour-ordered data layout,
 // geometric factors on the GPU, and the apply entry points.
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -15,8 +17,9 @@
 namespace mi355 {
 void collocated_grad(int P, int Q, const double *interp, const double *grad, double *collo);
 
-int lds_bytes(int P, int Q, int qf, int epb, int scalar_bytes, int layout) {
-  if (layout == kLayoutLines) return scalar_bytes * epb * (qf == kQfMass ? 2 : 3) * line_slab_entries(Q, scalar_bytes);
+int lds_bytes(int P, int Q, int qf, int num_comp, int epb, int scalar_bytes, int layout) {
+  if (layout == kLayoutLines && qf == kQfJit) return scalar_bytes * epb * 3 * Q * Q * Q;
+  if (layout == kLayoutLines) return (int)line_lds_bytes(Q, num_comp, qf, scalar_bytes, false, epb);
   if (layout == kLayoutPoints) return scalar_bytes * (Q * P + Q * Q + epb * (qf == kQfMass ? 3 : 4) * Q * Q * Q);
   const int slabs = qf == kQfMass ? 2 : 3;
   return scalar_bytes * (Q * P + Q * Q + epb * slabs * Q * Q * Q);
@@ -35,19 +38,47 @@ int64_t brick_lds_bytes(int P, int Q, int qf, int scalar_bytes, const int *shape
   return (int64_t)scalar_bytes * ns * (qf == kQfMass ? 2 : 3) * Q * Q * Q + 4 * nb;
 }
 
-int default_epb(int P, int Q, int qf, int scalar_bytes, int layout) {
+// Recomputing pays for diffusion, where it replaces 6 values per point: at
+// every order in FP64 with one component (1.4-1.9x).  Exceptions, all
+// measured on MI355X at 4M DoFs (ms per apply, stored / recomputed): mass
+// replaces one value (p=2 0.135 / 0.161, p=4 0.068 / 0.065, p=6 0.057 /
+// 0.058); FP32 reads half the bytes but computes the factors in FP64 all the
+// same, which costs as much as it saves at Q = 8 (0.071 / 0.073) and Q = 10
+// (0.088 / 0.092), not at Q = 7 (0.092 / 0.084) or Q = 9 (0.088 / 0.081),
+// whose stored layouts fill the wavefronts less well; three components share
+// one read of the factors (Q = 4: 0.210 / 0.214; Q = 3 0.654 / 0.620, Q = 5
+// 0.128 / 0.112, Q = 8 0.119 / 0.104).
+bool geo_pays(int Q, int qf, int num_comp, int scalar_bytes) {
+  if (qf != kQfDiffusion && qf != kQfDiffusionKappa) return false;
+  if (scalar_bytes == 4 && num_comp == 1) return Q != 8 && Q != 10;
+  return num_comp == 1 || Q != 4;
+}
+
+// Elements per workgroup with recomputed factors: the count of at most 256
+// threads that leaves the fewest lanes of its wavefronts idle (Q = 3 63 of 64,
+// 4 64, 5 125 of 128, 6 252 of 256, 7 245 of 256, 9 243 of 256, 10 200 of 256)
+// with no more wavefronts than that takes, the fastest measured at Q = 3..7
+// and 9 (8M DoFs, p=4: 0.222 ms, the next best, 5, 0.234); whole
+// wavefronts at Q = 2 and 8 share the barriers best at 128 and 256 threads
+// (p=6: 4 elements 0.182 ms, 1 element 0.197).
+int geo_default_epb(int Q) {
+  static const int table[11] = {0, 0, 32, 7, 4, 5, 7, 5, 4, 3, 2};
+  return Q >= 2 && Q <= 10 ? table[Q] : 1;
+}
+
+int default_epb(int P, int Q, int qf, int num_comp, int scalar_bytes, int layout) {
   if (layout == kLayoutLines && qf != kQfMass && Q >= 2 && Q <= 10) {
     // diffusion in the line layout: the autotuner's choices for FP64 at ~8M
     // DoFs on MI355X (Q = 2..10); within a few percent of the best for FP32
     static const int table[11] = {0, 0, 8, 6, 4, 2, 3, 1, 4, 3, 2};
     int              epb = table[Q];
-    while (epb > 1 && (epb * Q * Q > 256 || lds_bytes(P, Q, qf, epb, scalar_bytes, layout) > kMaxLdsBytes)) epb--;
+    while (epb > 1 && (epb * Q * Q > 256 || lds_bytes(P, Q, qf, num_comp, epb, scalar_bytes, layout) > kMaxLdsBytes)) epb--;
     return epb;
   }
   // as many elements as fit 256 threads and the default LDS budget
   int epb = 256 / layout_threads(Q, layout);
   if (epb < 1) epb = 1;
-  while (epb > 1 && lds_bytes(P, Q, qf, epb, scalar_bytes, layout) > kDefaultLdsBytes) epb--;
+  while (epb > 1 && lds_bytes(P, Q, qf, num_comp, epb, scalar_bytes, layout) > kDefaultLdsBytes) epb--;
   return epb;
 }
 }  // namespace mi355
@@ -189,6 +220,61 @@ int launch_build(int build, int64_t num_elem, int PM, const int32_t *mesh_offset
   return CEED_MI355_SUCCESS;
 }
 
+// The trilinear map of every element (hex_geo.hpp) from its 8 vertices.  Each
+// coefficient takes its differences before its sums, so that the cancellation
+// between neighbouring vertices happens on the coordinates themselves.
+__global__ void __launch_bounds__(256) geo_coefficients(int64_t num_elem, const int32_t *__restrict__ mesh_offsets, int32_t mesh_comp_stride,
+                                                        const double *__restrict__ coords, double *__restrict__ geo) {
+  const int64_t n = num_elem * 3;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t e = i / 3;
+    const int     d = (int)(i - e * 3);
+    double        x[8];
+    for (int k = 0; k < 8; k++) x[k] = coords[mesh_offsets[e * 8 + k] + (int64_t)d * mesh_comp_stride];
+    double *g = geo + e * mi355::kGeoStride + d;
+    const double x0 = x[1] - x[0], x1 = x[3] - x[2], x2 = x[5] - x[4], x3 = x[7] - x[6];  // differences along xi
+    const double y0 = x[2] - x[0], y1 = x[3] - x[1], y2 = x[6] - x[4], y3 = x[7] - x[5];  // along eta
+    const double z0 = x[4] - x[0], z1 = x[5] - x[1], z2 = x[6] - x[2], z3 = x[7] - x[3];  // along zeta
+    g[0]  = 0.125 * ((x0 + x1) + (x2 + x3));
+    g[3]  = 0.125 * ((y0 + y1) + (y2 + y3));
+    g[6]  = 0.125 * ((z0 + z1) + (z2 + z3));
+    g[9]  = 0.125 * ((x1 - x0) + (x3 - x2));
+    g[12] = 0.125 * ((x2 - x0) + (x3 - x1));
+    g[15] = 0.125 * ((y2 - y0) + (y3 - y1));
+    g[18] = 0.125 * ((x3 - x2) - (x1 - x0));
+    g[21] = 0;
+  }
+}
+
+// The plan's stored factors of a trilinear geometry: a thread per quadrature point
+template <typename T>
+__global__ void __launch_bounds__(256) geo_qdata(int64_t num_elem, int Q, int qf_mass, int64_t elem_stride, const double *__restrict__ geo,
+                                                 const double *__restrict__ pts, T *__restrict__ q_data) {
+  const int64_t q3 = (int64_t)Q * Q * Q, n = num_elem * q3;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t e = i / q3;
+    const int     r = (int)(i - e * q3), qx = r % Q, qy = (r / Q) % Q, qz = r / (Q * Q);
+    mi355::GeoColumn c;
+    c.load(geo + e * mi355::kGeoStride, pts[qx], pts[qy]);
+    const double w = pts[Q + qz] * (pts[Q + qy] * pts[Q + qx]);
+    T           *o = q_data + e * elem_stride + r;
+    if (qf_mass) {
+      o[0] = (T)mi355::geo_mass(c, pts[qz], w);
+    } else {
+      double s[6];
+      mi355::geo_poisson(c, pts[qz], w, s);
+      for (int k = 0; k < 6; k++) o[k * q3] = (T)s[k];
+    }
+  }
+}
+
+// Whether a mesh basis of two nodes is the linear one, (1 -+ xi)/2 at every point with slopes -+1/2
+bool linear_mesh_basis(int Q, const double *B, const double *G) {
+  for (int q = 0; q < Q; q++)
+    if (!(std::fabs(B[2 * q] + B[2 * q + 1] - 1) <= 1e-14 && std::fabs(G[2 * q] + 0.5) <= 1e-14 && std::fabs(G[2 * q + 1] - 0.5) <= 1e-14)) return false;
+  return true;
+}
+
 template <typename TOUT>
 int dispatch_build(int Q, int build, int64_t num_elem, int PM, const int32_t *mo, int32_t mcs, const double *coords, const double *mats,
                    int64_t st, TOUT *q_data, hipStream_t s) {
@@ -234,12 +320,12 @@ int color_elements(const int32_t *offsets, int64_t num_elem, int es, int nc, int
 }
 
 // Autotuner results: (thread layout, elements per workgroup) by (P, Q,
-// num_comp, pointwise operator, scalar type, E^T mode).
+// num_comp, pointwise operator, scalar type, E^T mode, recomputed factors).
 std::mutex                                                          g_tune_mutex;
-std::map<std::tuple<int, int, int, int, int, int>, std::pair<int, int>> g_tuned;
+std::map<std::tuple<int, int, int, int, int, int, bool>, std::pair<int, int>> g_tuned;
 
-std::tuple<int, int, int, int, int, int> tune_key(const CeedMi355Operator op) {
-  return std::make_tuple(op->P, op->Q, op->num_comp, op->qf, op->scalar_type, op->scatter);
+std::tuple<int, int, int, int, int, int, bool> tune_key(const CeedMi355Operator op) {
+  return std::make_tuple(op->P, op->Q, op->num_comp, op->qf, op->scalar_type, op->scatter, op->geo_valid);
 }
 
 bool tuned_launch(const CeedMi355Operator op, int *layout, int *epb) {
@@ -258,9 +344,25 @@ bool layout_exists(int Q, int qf, int layout) {
 }
 
 bool admissible(int P, int Q, int qf, int num_comp, int scalar_bytes, int layout, int epb) {
-  (void)num_comp;
   return layout_exists(Q, qf, layout) && epb >= 1 && epb * mi355::layout_threads(Q, layout) <= mi355::max_threads(layout) &&
-         mi355::lds_bytes(P, Q, qf, epb, scalar_bytes, layout) <= mi355::kMaxLdsBytes;
+         mi355::lds_bytes(P, Q, qf, num_comp, epb, scalar_bytes, layout) <= mi355::kMaxLdsBytes;
+}
+
+int plan_default_epb(const CeedMi355Operator op, int layout) {
+  if (layout == mi355::kLayoutLines && op->geo_valid) return mi355::geo_default_epb(op->Q);
+  return mi355::default_epb(op->P, op->Q, op->qf, op->num_comp, op->scalar_bytes, layout);
+}
+
+// The factors of the plan are from now on a trilinear geometry's (valid) or
+// the caller's; a launch nobody chose follows.
+void set_geo_valid(CeedMi355Operator op, bool valid) {
+  if (op->geo_valid == valid) return;
+  op->geo_valid = valid;
+  if (op->own_launch || op->scatter == CEED_MI355_PLAN_SEGMENT) return;
+  op->layout = mi355::kLayoutLines;
+  op->epb    = plan_default_epb(op, op->layout);
+  int layout, epb;
+  if (tuned_launch(op, &layout, &epb)) op->layout = layout, op->epb = epb;
 }
 
 // A launch the plan can take: segment plans have one (the line layout with an
@@ -522,20 +624,20 @@ int mi355::create_plan(int qf, int scalar_type, int32_t num_comp, int32_t num_el
   // than the column layout at every order measured on MI355X, equal at p <= 2)
   // with its default workgroup size; CEED_MI355_LAYOUT / CEED_MI355_EPB override
   op->layout = mi355::kLayoutLines;
-  op->epb    = mi355::default_epb(P_1d, Q_1d, qf, op->scalar_bytes, op->layout);
+  op->epb    = mi355::default_epb(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, op->layout);
   {
     int layout, epb;
     if (tuned_launch(op, &layout, &epb)) op->layout = layout, op->epb = epb;
   }
   if (const char *env = getenv("CEED_MI355_LAYOUT")) {
     const int l = atoi(env);
-    if (layout_exists(Q_1d, qf, l)) op->layout = l, op->epb = mi355::default_epb(P_1d, Q_1d, qf, op->scalar_bytes, l);
+    if (layout_exists(Q_1d, qf, l)) op->own_launch = true, op->layout = l, op->epb = mi355::default_epb(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, l);
   }
   if (qf == kQfJit && op->layout != mi355::kLayoutLines)  // run-time compiled kernels exist in the line layout only
-    op->layout = mi355::kLayoutLines, op->epb = mi355::default_epb(P_1d, Q_1d, qf, op->scalar_bytes, op->layout);
+    op->layout = mi355::kLayoutLines, op->epb = mi355::default_epb(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, op->layout);
   if (const char *env = getenv("CEED_MI355_EPB")) {
     const int v = atoi(env);
-    if (admissible(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, op->layout, v)) op->epb = v;
+    if (admissible(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, op->layout, v)) op->own_launch = true, op->epb = v;
   }
 
   const int            es = P_1d * P_1d * P_1d;
@@ -591,7 +693,7 @@ int mi355::create_plan(int qf, int scalar_type, int32_t num_comp, int32_t num_el
     // 256 threads hold (within the CU's LDS), no other launch
     int max_len = 256 / (Q_1d * Q_1d);
     if (const char *env = getenv("CEED_MI355_SEGMENT_MAX")) max_len = std::max(1, std::min(max_len, atoi(env)));
-    while (max_len > 1 && mi355::lds_bytes(P_1d, Q_1d, qf, max_len, op->scalar_bytes, mi355::kLayoutLines) > mi355::kMaxLdsBytes) max_len--;
+    while (max_len > 1 && mi355::lds_bytes(P_1d, Q_1d, qf, num_comp, max_len, op->scalar_bytes, mi355::kLayoutLines) > mi355::kMaxLdsBytes) max_len--;
     mi355::SegmentLayout L;
     ierr = mi355::segment_layout(offsets_host, num_elem, P_1d, max_len, L);
     if (ierr) {
@@ -731,13 +833,29 @@ extern "C" int CeedMi355OperatorBuildQData(CeedMi355Operator op, int build, int3
   MI355_HIP(hipMemcpyAsync(d_mats, mats.data(), sizeof(double) * mats.size(), hipMemcpyHostToDevice, s));
   int ierr;
   const int64_t blk = elem_block(op);
-  if (op->scalar_type == CEED_MI355_FP64)
+  bool                trilinear = false;
+  std::vector<double> pts(2 * Q);  // read by the copy below until the synchronisation
+  if (PM == 2 && linear_mesh_basis(Q, mesh_interp_1d_host, mesh_grad_1d_host)) {
+    for (int q = 0; q < Q; q++) pts[q] = mesh_interp_1d_host[2 * q + 1] - mesh_interp_1d_host[2 * q], pts[Q + q] = q_weight_1d_host[q];
+    if (!op->d_geo) MI355_HIP(hipMalloc(&op->d_geo, sizeof(double) * mi355::kGeoStride * ((size_t)op->num_elem + 1)));
+    if (!op->d_geo_pts) MI355_HIP(hipMalloc(&op->d_geo_pts, sizeof(double) * 2 * Q));
+    MI355_HIP(hipMemcpyAsync(op->d_geo_pts, pts.data(), sizeof(double) * 2 * Q, hipMemcpyHostToDevice, s));
+    const int64_t q3 = (int64_t)Q * Q * Q;
+    geo_coefficients<<<mi355_blocks(op->num_elem * 3, 256), 256, 0, s>>>(op->num_elem, d_mo, mesh_comp_stride, coords, op->d_geo);
+    if (op->scalar_type == CEED_MI355_FP64)
+      geo_qdata<double><<<mi355_blocks(op->num_elem * q3, 256), 256, 0, s>>>(op->num_elem, Q, build == 0, blk, op->d_geo, op->d_geo_pts, (double *)op->d_qdata);
+    else geo_qdata<float><<<mi355_blocks(op->num_elem * q3, 256), 256, 0, s>>>(op->num_elem, Q, build == 0, blk, op->d_geo, op->d_geo_pts, (float *)op->d_qdata);
+    ierr          = hipGetLastError() == hipSuccess ? CEED_MI355_SUCCESS : CEED_MI355_ERROR_BACKEND;
+    op->geo_lines = op->scalar_type == CEED_MI355_FP64 ? mi355::pick_geo_f64(op->P, Q, op->num_comp, op->qf) : mi355::pick_geo_f32(op->P, Q, op->num_comp, op->qf);
+    trilinear     = ierr == CEED_MI355_SUCCESS && op->geo_lines && mi355::geo_pays(Q, op->qf, op->num_comp, op->scalar_bytes);
+  } else if (op->scalar_type == CEED_MI355_FP64)
     ierr = dispatch_build<double>(Q, build, op->num_elem, PM, d_mo, mesh_comp_stride, coords, d_mats, blk, (double *)op->d_qdata, s);
   else ierr = dispatch_build<float>(Q, build, op->num_elem, PM, d_mo, mesh_comp_stride, coords, d_mats, blk, (float *)op->d_qdata, s);
   MI355_HIP(hipStreamSynchronize(s));
   (void)hipFree(d_mo);
   (void)hipFree(d_mats);
   if (ierr) return ierr;
+  set_geo_valid(op, trilinear);
   if (op->qf == kQfDiffusionKappa) {
     // kappa slot defaults to 1 until CeedMi355OperatorSetKappa
     const int64_t Q3 = (int64_t)Q * Q * Q, n = op->num_elem * Q3;
@@ -755,6 +873,7 @@ extern "C" int CeedMi355OperatorSetQData(CeedMi355Operator op, const void *q_dat
   const int64_t blk = elem_block(op);
   hipStream_t   s   = (hipStream_t)stream;
   MI355_CHECK(per == blk || op->qf == kQfDiffusionKappa, CEED_MI355_ERROR_BACKEND, "layout mismatch");
+  if (op->qf != kQfDiffusionKappa) set_geo_valid(op, false);  // the caller's factors from here on
   if (op->qf != kQfDiffusionKappa) {
     if (op->scalar_type == CEED_MI355_FP64)
       permute_elements<double, double><<<mi355_blocks(op->num_elem * per, 256), 256, 0, s>>>(op->num_elem, per, op->d_perm, 1,
@@ -830,7 +949,8 @@ extern "C" int CeedMi355OperatorSetLaunch(CeedMi355Operator op, int32_t elems_pe
   MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
   MI355_CHECK(plan_admissible(op, op->layout, elems_per_block), CEED_MI355_ERROR_BACKEND,
               "%d elements per workgroup do not fit (at most 256 threads and 160 KiB of LDS for P=%d Q=%d)", elems_per_block, op->P, op->Q);
-  op->epb = elems_per_block;
+  op->epb        = elems_per_block;
+  op->own_launch = true;
   return CEED_MI355_SUCCESS;
 }
 
@@ -843,11 +963,12 @@ extern "C" int CeedMi355OperatorSetLayout(CeedMi355Operator op, int32_t layout, 
   MI355_CHECK(layout_exists(op->Q, op->qf, layout), CEED_MI355_ERROR_UNSUPPORTED, "the point layout needs Q^3 <= 256 (Q = %d)", op->Q);
   const int epb = elems_per_block > 0                       ? elems_per_block
                   : op->scatter == CEED_MI355_PLAN_SEGMENT ? op->seg_max
-                                                           : mi355::default_epb(op->P, op->Q, op->qf, op->scalar_bytes, layout);
+                                                           : plan_default_epb(op, layout);
   MI355_CHECK(plan_admissible(op, layout, epb), CEED_MI355_ERROR_BACKEND,
               "%d elements per workgroup do not fit layout %d (at most 256 threads and 160 KiB of LDS for P=%d Q=%d)", epb, layout, op->P, op->Q);
-  op->layout = layout;
-  op->epb    = epb;
+  op->layout     = layout;
+  op->epb        = epb;
+  op->own_launch = true;
   return CEED_MI355_SUCCESS;
 }
 
@@ -978,6 +1099,8 @@ extern "C" int CeedMi355OperatorDestroy(CeedMi355Operator *op) {
   (void)hipFree((*op)->d_bslot);
   (void)hipFree((*op)->d_partials);
   (void)hipFree((*op)->d_seg_start);
+  (void)hipFree((*op)->d_geo);
+  (void)hipFree((*op)->d_geo_pts);
   delete *op;
   *op = nullptr;
   return CEED_MI355_SUCCESS;
