@@ -7,77 +7,228 @@
 //   diffusion:  sum_q g_i(q)^T S(q) g_i(q),  g_i = (G_a B_b B_c, B_a G_b B_c, B_a B_b G_c)
 //               (times kappa(q) for the kappa-weighted operator),
 // with G = D B, D the plan's collocated derivative; every component of a
-// vector operator has the same diagonal.  The element diagonals are summed
-// into the L-vector by the plan's E^T mode (transpose map, colours, atomics).
-// One workgroup per element; the element's geometric factors sit in LDS.
+// vector operator has the same diagonal.  Written out, each of the six entries
+// of S meets a tensor product of three of the matrices BB = B o B, BG = B o G,
+// GG = G o G (entrywise products), so the diagonal is six sum-factorised
+// transposes that share their last steps:
+//   z:  A0 = BB S00, A1 = BB S11, A2 = GG S22, A3 = 2 BG S12, A4 = 2 BG S02, A5 = 2 BB S01
+//   y:  R0 = BB A0,  R1 = GG A1 + BB A2 + BG A3,  R2 = BB A4 + BG A5
+//   x:  GG R0 + BB R1 + BG R2
+// 6 Q^3 P + 6 Q^2 P^2 + 3 Q P^3 multiply-adds per element instead of the
+// P^3 Q^3 terms of the sum itself (27 thousand against 74 thousand terms of 20
+// operations each at P = 6, Q = 7).
+//
+// One Q x Q slab of threads per element: the z step on the columns (factors
+// read, or recomputed where the plan's apply does), the y step on the lines
+// (qx, z) and the x step on the rows (y, z), in place in the slabs.  The
+// element diagonals are summed into the L-vector by the plan's E^T mode.
+// MI355X, FP64 diffusion, p=5, 1.1M DoFs: 592 us with the P^3 Q^3 loop, 40 us
+// now; its 0.5 GFLOP take 7 us at the FP64 rate, and what bounds it is latency
+// at the three or four waves per SIMD that 6 P accumulators leave.
 #include "hex_plan.hpp"
 
 namespace mi355 {
 namespace {
 
-template <int P, int Q, typename T>
-__global__ void __launch_bounds__(128) hex_diag_kernel(int64_t elem_begin, int64_t elem_end, int scatter, int qf, int num_comp,
+// The products' slabs: mass one, diffusion three, which take the six products
+// in two turns (with six slabs LDS held a CU to 9 wavefronts at P = 6; p=5,
+// 1.1M DoFs, us per assembly: 48.7 with six, 42.5 with three).
+__host__ __device__ constexpr int diag_slabs(int qf) { return qf == kQfMass ? 1 : 3; }
+
+// Four waves per SIMD where the accumulators fit 128 VGPRs without spills
+// (P <= 5; at P = 6 the bound spills 92 bytes: 47 us against 40).
+template <int P, int Q, int QF, bool kGeo, typename T>
+__global__ void __launch_bounds__(256, (P <= 5 ? 4 : 1)) hex_diag_kernel(int64_t elem_begin, int64_t elem_end, int scatter, int num_comp,
                                                        const int32_t *__restrict__ offsets, int32_t comp_stride, const T *__restrict__ q_data,
-                                                       int q_comp, const T *__restrict__ mats, T *__restrict__ v, T *__restrict__ evec,
+                                                       const T *__restrict__ mats, const double *__restrict__ geo,
+                                                       const double *__restrict__ geo_pts, T *__restrict__ v, T *__restrict__ evec,
                                                        const int32_t *__restrict__ tpos) {
-  constexpr int P3 = P * P * P, Q3 = Q * Q * Q;
+  constexpr int NT = Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QP = Q * P, QC = QfTraits<QF>::kComps, NS = diag_slabs(QF), NA = QF == kQfMass ? 1 : 6;
+  constexpr int SR = line_row_stride(Q, sizeof(T)), SP = line_plane_stride(Q, sizeof(T)), SLAB = P * SP;
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  T *sB  = reinterpret_cast<T *>(lds_raw);  // Q x P
-  T *sG  = sB + Q * P;                       // Q x P, G = D B
-  T *sQd = sG + Q * P;                       // q_comp x Q^3
-  const int64_t e = elem_begin + xcd_chunk(blockIdx.x, gridDim.x);
-  if (e >= elem_end) return;  // uniform per workgroup
-  const T *D = mats + Q * P;
-  for (int i = threadIdx.x; i < Q * P; i += blockDim.x) {
-    sB[i]            = mats[i];
-    const int qx = i / P, a = i % P;
-    T         g  = 0;
-    for (int c = 0; c < Q; c++) g += D[qx * Q + c] * mats[c * P + a];
-    sG[i] = g;
-  }
-  for (int i = threadIdx.x; i < q_comp * Q3; i += blockDim.x) sQd[i] = q_data[e * (int64_t)q_comp * Q3 + i];
-  __syncthreads();
-  for (int i = threadIdx.x; i < P3; i += blockDim.x) {
-    const int a = i % P, b = (i / P) % P, c = i / (P * P);
-    T         acc = 0;
+  const int     epb = blockDim.x / NT, le = threadIdx.x / NT, t = threadIdx.x - le * NT;
+  T            *A  = reinterpret_cast<T *>(lds_raw) + (size_t)le * NS * SLAB;
+  auto          at = [](int k, int z, int y, int x) { return k * SLAB + z * SP + y * SR + x; };
+  const int64_t e    = elem_begin + xcd_chunk(blockIdx.x, gridDim.x) * epb + le;
+  const bool    live = le < epb && e < elem_end;
+  const int64_t ec   = live ? e : elem_begin;  // lanes without an element work on the first one's factors and write nothing
+  const int     cx = t % Q, cy = t / Q;
+  const T      *sq = mats + QP + Q * Q;  // BB, BG, GG (Q x P each) behind B and D
+
+  // ---- z on the column (cx, cy): acc[k][b] = A_k at (b, cy, cx), b < P
+  T acc[NA][P];
+#pragma unroll
+  for (int k = 0; k < NA; k++)
+#pragma unroll
+    for (int b = 0; b < P; b++) acc[k][b] = 0;
+  {
+    const T  *qd = q_data + ec * (int64_t)QC * Q3 + cy * Q + cx;
+    GeoColumn col;
+    double    wxy = 0;
+    if constexpr (kGeo) {
+      col.load(geo + ec * kGeoStride, geo_pts[cx], geo_pts[cy]);
+      wxy = geo_pts[Q + cy] * geo_pts[Q + cx];
+    }
+#pragma unroll
     for (int qz = 0; qz < Q; qz++) {
-      const T bz = sB[qz * P + c], gz = sG[qz * P + c];
-      for (int qy = 0; qy < Q; qy++) {
-        const T by = sB[qy * P + b], gy = sG[qy * P + b];
-        for (int qx = 0; qx < Q; qx++) {
-          const T   bx = sB[qx * P + a], gx = sG[qx * P + a];
-          const int q  = (qz * Q + qy) * Q + qx;
-          if (qf == kQfMass) {
-            const T phi = bx * by * bz;
-            acc += phi * phi * sQd[q];
-          } else {
-            const T d0 = gx * by * bz, d1 = bx * gy * bz, d2 = bx * by * gz;
-            const T s00 = sQd[q], s11 = sQd[Q3 + q], s22 = sQd[2 * Q3 + q], s12 = sQd[3 * Q3 + q], s02 = sQd[4 * Q3 + q], s01 = sQd[5 * Q3 + q];
-            T       t   = d0 * (s00 * d0 + s01 * d1 + s02 * d2) + d1 * (s01 * d0 + s11 * d1 + s12 * d2) + d2 * (s02 * d0 + s12 * d1 + s22 * d2);
-            if (qf == kQfDiffusionKappa) t *= sQd[6 * Q3 + q];
-            acc += t;
-          }
+      T s[QC];
+      if constexpr (kGeo) {
+        const auto gp = phase_ptr(geo_pts);
+        double     g6[6];
+        __builtin_amdgcn_sched_barrier(0);  // one point's factors at a time in registers
+        geo_poisson(col, gp[qz], gp[Q + qz] * wxy, g6);
+#pragma unroll
+        for (int k = 0; k < 6; k++) s[k] = (T)g6[k];
+        if constexpr (QF == kQfDiffusionKappa) s[6] = __builtin_nontemporal_load(qd + 6 * Q3 + qz * Q * Q);
+      } else {
+#pragma unroll
+        for (int k = 0; k < QC; k++) s[k] = __builtin_nontemporal_load(qd + k * Q3 + qz * Q * Q);
+      }
+      const auto bb = phase_ptr(sq + qz * P), bg = phase_ptr(sq + QP + qz * P), gg = phase_ptr(sq + 2 * QP + qz * P);
+      if constexpr (QF == kQfMass) {
+#pragma unroll
+        for (int b = 0; b < P; b++) acc[0][b] += bb[b] * s[0];
+      } else {
+        if constexpr (QF == kQfDiffusionKappa) {
+#pragma unroll
+          for (int k = 0; k < 6; k++) s[k] *= s[6];
+        }
+        const T s3 = 2 * s[3], s4 = 2 * s[4], s5 = 2 * s[5];
+#pragma unroll
+        for (int b = 0; b < P; b++) {
+          acc[0][b] += bb[b] * s[0];
+          acc[1][b] += bb[b] * s[1];
+          acc[2][b] += gg[b] * s[2];
+          acc[3][b] += bg[b] * s3;
+          acc[4][b] += bg[b] * s4;
+          acc[5][b] += bb[b] * s5;
         }
       }
     }
-    const int32_t o = offsets[e * P3 + i];
-    for (int k = 0; k < num_comp; k++) {
-      if (scatter == kScatterElem) {  // element-major E-vector (brick plans)
-        evec[(e * num_comp + k) * (int64_t)P3 + i] = acc;
-        continue;
+  }
+  // the products are complete here: without this the compiler sinks half of
+  // their sums behind the first barrier and spills the matrices to carry them
+#pragma unroll
+  for (int k = 0; k < NA; k++)
+#pragma unroll
+    for (int b = 0; b < P; b++) asm volatile("" : "+v"(acc[k][b]));
+  const bool yline = t < QP, xline = t < P * P;
+  const int  ny = t % P, nz = t / P;
+  // ---- y on the lines (qx = cx, z = cy < P), then x on the rows (y, z)
+  if constexpr (QF == kQfMass) {
+#pragma unroll
+    for (int b = 0; b < P; b++) A[at(0, b, cy, cx)] = acc[0][b];
+    __syncthreads();
+    if (yline) {
+      T r[P] = {};
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+        const auto bb = phase_ptr(sq + q * P);
+        const T    a0 = A[at(0, cy, q, cx)];
+#pragma unroll
+        for (int b = 0; b < P; b++) r[b] += bb[b] * a0;
       }
-      if (scatter == kScatterEvec || (scatter == kScatterSplit && (o & 1))) {  // L-entry-sorted E-vector
-        evec[tpos[(e * num_comp + k) * (int64_t)P3 + i]] = acc;
-        continue;
+#pragma unroll
+      for (int b = 0; b < P; b++) A[at(0, cy, b, cx)] = r[b];
+    }
+    __syncthreads();
+    if (xline) {
+      T r[P] = {};
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+        const auto bb = phase_ptr(sq + q * P);
+        const T    a0 = A[at(0, nz, ny, q)];
+#pragma unroll
+        for (int x = 0; x < P; x++) r[x] += bb[x] * a0;
       }
-      T *dst = &v[(o >> 1) + (int64_t)k * comp_stride];
-      if (scatter == kScatterSplit) {  // at most two contributions: onto the zeroed target
-        unsafeAtomicAdd(dst, acc);
-        continue;
+#pragma unroll
+      for (int x = 0; x < P; x++) A[at(0, nz, ny, x)] = r[x];
+    }
+  } else {
+#pragma unroll
+    for (int b = 0; b < P; b++) A[at(0, b, cy, cx)] = acc[1][b], A[at(1, b, cy, cx)] = acc[2][b], A[at(2, b, cy, cx)] = acc[3][b];
+    __syncthreads();
+    T r1[P] = {};
+    if (yline) {
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+        if (q % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // two rows of each matrix in SGPRs at a time
+        const auto bb = phase_ptr(sq + q * P), bg = phase_ptr(sq + QP + q * P), gg = phase_ptr(sq + 2 * QP + q * P);
+        const T    a1 = A[at(0, cy, q, cx)], a2 = A[at(1, cy, q, cx)], a3 = A[at(2, cy, q, cx)];
+#pragma unroll
+        for (int b = 0; b < P; b++) {
+          r1[b] += gg[b] * a1;
+          r1[b] += bb[b] * a2;
+          r1[b] += bg[b] * a3;
+        }
       }
-      if (scatter == kScatterAtomic) unsafeAtomicAdd(dst, acc);
-      else if (scatter == kScatterOverwrite && (o & 1)) *dst = acc;
-      else *dst += acc;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < P; b++) A[at(0, b, cy, cx)] = acc[0][b], A[at(1, b, cy, cx)] = acc[4][b], A[at(2, b, cy, cx)] = acc[5][b];
+    __syncthreads();
+    if (yline) {
+      T r0[P] = {}, r2[P] = {};
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+        if (q % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // two rows of each matrix in SGPRs at a time
+        const auto bb = phase_ptr(sq + q * P), bg = phase_ptr(sq + QP + q * P);
+        const T    a0 = A[at(0, cy, q, cx)], a4 = A[at(1, cy, q, cx)], a5 = A[at(2, cy, q, cx)];
+#pragma unroll
+        for (int b = 0; b < P; b++) {
+          r0[b] += bb[b] * a0;
+          r2[b] += bb[b] * a4;
+          r2[b] += bg[b] * a5;
+        }
+      }
+#pragma unroll
+      for (int b = 0; b < P; b++) A[at(0, cy, b, cx)] = r0[b], A[at(1, cy, b, cx)] = r1[b], A[at(2, cy, b, cx)] = r2[b];
+    }
+    __syncthreads();
+    if (xline) {
+      T r[P] = {};
+#pragma unroll
+      for (int q = 0; q < Q; q++) {
+        if (q % 2 == 0) __builtin_amdgcn_sched_barrier(0);  // two rows of each matrix in SGPRs at a time
+        const auto bb = phase_ptr(sq + q * P), bg = phase_ptr(sq + QP + q * P), gg = phase_ptr(sq + 2 * QP + q * P);
+        const T    a0 = A[at(0, nz, ny, q)], a1 = A[at(1, nz, ny, q)], a2 = A[at(2, nz, ny, q)];
+#pragma unroll
+        for (int x = 0; x < P; x++) {
+          r[x] += gg[x] * a0;
+          r[x] += bb[x] * a1;
+          r[x] += bg[x] * a2;
+        }
+      }
+#pragma unroll
+      for (int x = 0; x < P; x++) A[at(0, nz, ny, x)] = r[x];
+    }
+  }
+  __syncthreads();
+  // ---- E^T from the node columns, as the fused apply
+  if (live && cx < P && cy < P) {
+#pragma unroll
+    for (int z = 0; z < P; z++) {
+      const int     i   = (z * P + cy) * P + cx;
+      const T       acc = A[at(0, z, cy, cx)];
+      const int32_t o   = offsets[e * P3 + i];
+      for (int k = 0; k < num_comp; k++) {
+        if (scatter == kScatterElem) {  // element-major E-vector (brick plans)
+          evec[(e * num_comp + k) * (int64_t)P3 + i] = acc;
+          continue;
+        }
+        if (scatter == kScatterEvec || (scatter == kScatterSplit && (o & 1))) {  // L-entry-sorted E-vector
+          evec[tpos[(e * num_comp + k) * (int64_t)P3 + i]] = acc;
+          continue;
+        }
+        T *dst = &v[(o >> 1) + (int64_t)k * comp_stride];
+        if (scatter == kScatterSplit) {  // at most two contributions: onto the zeroed target
+          unsafeAtomicAdd(dst, acc);
+          continue;
+        }
+        if (scatter == kScatterAtomic) unsafeAtomicAdd(dst, acc);
+        else if (scatter == kScatterOverwrite && (o & 1)) *dst = acc;
+        else *dst += acc;
+      }
     }
   }
 }
@@ -87,12 +238,34 @@ __global__ void __launch_bounds__(256) diag_zero(int64_t n, T *__restrict__ x) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) x[i] = T(0);
 }
 
+// Element diagonals of packed elements [b, e), added or stored by `scatter`
+template <int P, int Q, typename T>
+int launch_diag_elements(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, T *v, hipStream_t s) {
+  // as many elements as fit 256 threads and the default LDS budget (at least
+  // one: 44 kB at P = 9, Q = 10 in FP64)
+  const size_t per = sizeof(T) * (size_t)diag_slabs(op->qf) * P * line_plane_stride(Q, sizeof(T));
+  int          epb = 256 / (Q * Q);
+  while (epb > 1 && epb * per > (size_t)kDefaultLdsBytes) epb--;
+  const unsigned grid = (unsigned)((e - b + epb - 1) / epb), nt = (unsigned)(epb * Q * Q);
+#define MI355_DIAG_LAUNCH(QF, GEO)                                                                                                        \
+  hex_diag_kernel<P, Q, QF, GEO, T><<<grid, nt, epb * per, s>>>(b, e, scatter, op->num_comp, op->d_offsets, op->comp_stride,              \
+                                                                (const T *)op->d_qdata, (const T *)op->d_mats, op->d_geo, op->d_geo_pts, v, \
+                                                                (T *)op->d_evec, op->d_tpos)
+  if (op->qf == kQfMass) MI355_DIAG_LAUNCH(kQfMass, false);
+  else if (op->qf == kQfDiffusion && op->geo_valid) MI355_DIAG_LAUNCH(kQfDiffusion, true);
+  else if (op->qf == kQfDiffusion) MI355_DIAG_LAUNCH(kQfDiffusion, false);
+  else if (op->geo_valid) MI355_DIAG_LAUNCH(kQfDiffusionKappa, true);
+  else MI355_DIAG_LAUNCH(kQfDiffusionKappa, false);
+#undef MI355_DIAG_LAUNCH
+  MI355_LAUNCH_CHECK();
+  return CEED_MI355_SUCCESS;
+}
+
 template <int P, int Q, typename T>
 int launch_diag(const CeedMi355Operator_private *op, void *v, int add, hipStream_t s) {
-  const size_t lds  = sizeof(T) * (size_t)(2 * Q * P + op->q_comp * Q * Q * Q);
-  const bool   tmap = op->scatter == 0;
-  const bool   split = op->scatter == CEED_MI355_PLAN_SPLIT;
-  const bool   brick = op->scatter == CEED_MI355_PLAN_BRICK;
+  const bool tmap  = op->scatter == 0;
+  const bool split = op->scatter == CEED_MI355_PLAN_SPLIT;
+  const bool brick = op->scatter == CEED_MI355_PLAN_BRICK;
   MI355_CHECK(op->scatter != CEED_MI355_PLAN_SEGMENT, CEED_MI355_ERROR_UNSUPPORTED,
               "diagonal assembly does not take segment plans (elements of a colour share segment faces)");
   if (brick) {  // element diagonals into the element-major E-vector, then the brick E^T
@@ -100,11 +273,8 @@ int launch_diag(const CeedMi355Operator_private *op, void *v, int add, hipStream
       diag_zero<T><<<mi355_blocks(op->l_size, 256, 4096), 256, 0, s>>>(op->l_size, (T *)v);
       MI355_LAUNCH_CHECK();
     }
-    hex_diag_kernel<P, Q, T><<<(unsigned)op->num_elem, 128, lds, s>>>(0, op->num_elem, kScatterElem, op->qf, op->num_comp, op->d_offsets,
-                                                                     op->comp_stride, (const T *)op->d_qdata, op->q_comp,
-                                                                     (const T *)op->d_mats, (T *)v, (T *)op->d_evec, op->d_tpos);
-    MI355_LAUNCH_CHECK();
-    return brick_evec(op, op->d_evec, v, !add, s);
+    const int err = launch_diag_elements<P, Q, T>(op, 0, op->num_elem, kScatterElem, (T *)v, s);
+    return err ? err : brick_evec(op, op->d_evec, v, !add, s);
   }
   // the split mode's atomic adds land on a zeroed target: v, or with add the scratch vector
   T *target = split && add ? (T *)op->d_scratch : (T *)v;
@@ -118,16 +288,13 @@ int launch_diag(const CeedMi355Operator_private *op, void *v, int add, hipStream
     const int scatter = tmap ? kScatterEvec
                         : split ? kScatterSplit
                                 : (op->scatter == CEED_MI355_PLAN_ATOMIC ? kScatterAtomic : (add ? kScatterAdd : kScatterOverwrite));
-    hex_diag_kernel<P, Q, T><<<(unsigned)(e - b), 128, lds, s>>>(b, e, scatter, op->qf, op->num_comp, op->d_offsets, op->comp_stride,
-                                                               (const T *)op->d_qdata, op->q_comp, (const T *)op->d_mats, target,
-                                                               (T *)op->d_evec, op->d_tpos);
+    const int err = launch_diag_elements<P, Q, T>(op, b, e, scatter, target, s);
+    if (err) return err;
   }
-  MI355_LAUNCH_CHECK();
   if (tmap) return transpose_gather(op, v, !add, s);
   if (split) return split_finish(op, v, !add, s);
   return CEED_MI355_SUCCESS;
 }
-
 using DiagFn = int (*)(const CeedMi355Operator_private *, void *, int, hipStream_t);
 
 template <typename T>

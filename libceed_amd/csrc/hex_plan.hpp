@@ -167,7 +167,7 @@ struct CeedMi355Operator_private {
   std::vector<int32_t> perm;  // packed position -> caller's element index
   int32_t             *d_offsets = nullptr;  // [elem][P^3], packed order
   int32_t             *d_perm    = nullptr;
-  void                *d_mats    = nullptr;  // B (Q x P) then D (Q x Q), plan scalar type
+  void                *d_mats    = nullptr;  // B (Q x P), D (Q x Q), then B o B, B o G, G o G (Q x P each), plan scalar type
   void                *d_qdata   = nullptr;  // [elem][q_comp][Q^3], packed order
   mi355::ApplyFn       apply     = nullptr;
   // trilinear geometry: the map's coefficients [elem][kGeoStride] in packed

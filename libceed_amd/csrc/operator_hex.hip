@@ -787,10 +787,20 @@ int mi355::create_plan(int qf, int scalar_type, int32_t num_comp, int32_t num_el
     }
   }
 
-  // B and the collocated derivative D = G pinv(B), in the plan's scalar type
-  std::vector<double> mats(Q_1d * P_1d + Q_1d * Q_1d);
+  // B and the collocated derivative D = G pinv(B), then (for the diagonal) the
+  // entrywise products B B, B G, G G with G = D B, in the plan's scalar type
+  const int           QP = Q_1d * P_1d, QQ = Q_1d * Q_1d;
+  std::vector<double> mats(QP + QQ + 3 * QP);
   memcpy(mats.data(), interp_1d_host, sizeof(double) * Q_1d * P_1d);
   mi355::collocated_grad(P_1d, Q_1d, interp_1d_host, grad_1d_host, &mats[Q_1d * P_1d]);
+  for (int q = 0; q < Q_1d; q++)
+    for (int a = 0; a < P_1d; a++) {
+      double g = 0;
+      for (int c = 0; c < Q_1d; c++) g += mats[QP + q * Q_1d + c] * mats[c * P_1d + a];
+      const double b = mats[q * P_1d + a];
+      const int    i = QP + QQ + q * P_1d + a;
+      mats[i] = b * b, mats[i + QP] = b * g, mats[i + 2 * QP] = g * g;
+    }
 
   MI355_HIP(hipMalloc(&op->d_offsets, sizeof(int32_t) * (packed.size() + 1)));
   MI355_HIP(hipMemcpy(op->d_offsets, packed.data(), sizeof(int32_t) * packed.size(), hipMemcpyHostToDevice));
