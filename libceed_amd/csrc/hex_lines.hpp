@@ -175,6 +175,24 @@ struct LineQData {
   }
 };
 
+// acc[i] += sum_j M[j][i] in[j] for a row-major J x I matrix at m: the sums in
+// ascending j, as a line contraction with the transposed matrix forms them.
+// By rows (from Q = 7, where the matrix does not fit the SGPRs) a row of I
+// contiguous entries is loaded for each j; column by column it is I J scalar
+// loads of one entry each (705 against 255 scalar loads per wave at p=8; MI355X,
+// FP64 diffusion, us per apply, columns / rows: stored factors 8M DoFs p=6 252
+// / 246, p=8 299 / 278, three components 4M DoFs p=5 168 / 125, p=7 145 / 132;
+// recomputed 8M DoFs p=8 199 / 187).
+template <int I, int J, typename T>
+__device__ __forceinline__ void transposed_line(const T *m, const T (&in)[J], T (&acc)[I]) {
+#pragma unroll
+  for (int j = 0; j < J; j++) {
+    const auto r = phase_ptr(m + j * I);
+#pragma unroll
+    for (int i = 0; i < I; i++) acc[i] += r[i] * in[j];
+  }
+}
+
 // Synchronisation of one element's threads between the phases of the line
 // pipeline: the whole workgroup, or the wavefront alone when an element never
 // spans two wavefronts (a wavefront's LDS operations are performed in the
@@ -614,14 +632,22 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo
         qd.point(qz, cx, s);
         uq[qz] *= s[0];
       }
-      const auto gB = phase_ptr(mats);
+      if constexpr (kRowWise) {
+        T out[P];
 #pragma unroll
-      for (int b = 0; b < P; b++) {
-        const auto m = kRowWise ? phase_ptr(mats + b) : gB + b;
-        T          s = 0;
+        for (int i = 0; i < P; i++) out[i] = 0;
+        transposed_line(mats, uq, out);
 #pragma unroll
-        for (int qz = 0; qz < Q; qz++) s += m[qz * P] * uq[qz];
-        X[at(b, cy, cx)] = s;
+        for (int i = 0; i < P; i++) X[at(i, cy, cx)] = out[i];
+      } else {
+        const auto m = phase_ptr(mats);
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+          T s = 0;
+#pragma unroll
+          for (int j = 0; j < Q; j++) s += m[j * P + i] * uq[j];
+          X[at(i, cy, cx)] = s;
+        }
       }
     } else {
       // ---- collocated derivatives: z on the column; x by x-lines of X into Y,
@@ -710,83 +736,129 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo
       // ---- D_x^T by x-lines of Y, D_y^T by y-lines of X, both in place
       {
         T in[Q];
-        {
-          const auto gD = phase_ptr(mats + Q * P);
 #pragma unroll
-          for (int c = 0; c < Q; c++) in[c] = Y[at(cy, cx, c)];
+        for (int c = 0; c < Q; c++) in[c] = Y[at(cy, cx, c)];
+        if constexpr (kRowWise) {
+          T out[Q];
 #pragma unroll
-          for (int qx = 0; qx < Q; qx++) {
-            const auto m = kRowWise ? phase_ptr(mats + Q * P + qx) : gD + qx;
-            T          s = 0;
+          for (int i = 0; i < Q; i++) out[i] = 0;
+          transposed_line(mats + Q * P, in, out);
 #pragma unroll
-            for (int c = 0; c < Q; c++) s += m[c * Q] * in[c];
-            Y[at(cy, cx, qx)] = s;
+          for (int i = 0; i < Q; i++) Y[at(cy, cx, i)] = out[i];
+        } else {
+          const auto m = phase_ptr(mats + Q * P);
+#pragma unroll
+          for (int i = 0; i < Q; i++) {
+            T s = 0;
+#pragma unroll
+            for (int j = 0; j < Q; j++) s += m[j * Q + i] * in[j];
+            Y[at(cy, cx, i)] = s;
           }
         }
-        const auto gD = phase_ptr(mats + Q * P);
 #pragma unroll
         for (int c = 0; c < Q; c++) in[c] = X[at(cy, c, cx)];
+        if constexpr (kRowWise) {
+          T out[Q];
 #pragma unroll
-        for (int qy = 0; qy < Q; qy++) {
-          const auto m = kRowWise ? phase_ptr(mats + Q * P + qy) : gD + qy;
-          T          s = 0;
+          for (int i = 0; i < Q; i++) out[i] = 0;
+          transposed_line(mats + Q * P, in, out);
 #pragma unroll
-          for (int c = 0; c < Q; c++) s += m[c * Q] * in[c];
-          X[at(cy, qy, cx)] = s;
+          for (int i = 0; i < Q; i++) X[at(cy, i, cx)] = out[i];
+        } else {
+          const auto m = phase_ptr(mats + Q * P);
+#pragma unroll
+          for (int i = 0; i < Q; i++) {
+            T s = 0;
+#pragma unroll
+            for (int j = 0; j < Q; j++) s += m[j * Q + i] * in[j];
+            X[at(cy, i, cx)] = s;
+          }
         }
       }
       __syncthreads();
       // ---- sum of the three transposes on the column, then B_z^T into X
-      const auto gDz = phase_ptr(mats + Q * P);
-      T          w[Q];
+      T w[Q];
+      if constexpr (kRowWise) {
+        T out[Q];
 #pragma unroll
-      for (int qz = 0; qz < Q; qz++) {
-        const auto m = kRowWise ? phase_ptr(mats + Q * P + qz) : gDz + qz;
-        T          s = Y[at(qz, cy, cx)] + X[at(qz, cy, cx)];
+        for (int i = 0; i < Q; i++) out[i] = Y[at(i, cy, cx)] + X[at(i, cy, cx)];
+        transposed_line(mats + Q * P, vz, out);
 #pragma unroll
-        for (int c = 0; c < Q; c++) s += m[c * Q] * vz[c];
-        w[qz] = s;
+        for (int i = 0; i < Q; i++) w[i] = out[i];
+      } else {
+        const auto m = phase_ptr(mats + Q * P);
+#pragma unroll
+        for (int i = 0; i < Q; i++) {
+          T s = Y[at(i, cy, cx)] + X[at(i, cy, cx)];
+#pragma unroll
+          for (int j = 0; j < Q; j++) s += m[j * Q + i] * vz[j];
+          w[i] = s;
+        }
       }
-      const auto gBz = phase_ptr(mats);
+      if constexpr (kRowWise) {
+        T out[P];
 #pragma unroll
-      for (int b = 0; b < P; b++) {
-        const auto m = kRowWise ? phase_ptr(mats + b) : gBz + b;
-        T          s = 0;
+        for (int i = 0; i < P; i++) out[i] = 0;
+        transposed_line(mats, w, out);
 #pragma unroll
-        for (int qz = 0; qz < Q; qz++) s += m[qz * P] * w[qz];
-        X[at(b, cy, cx)] = s;
+        for (int i = 0; i < P; i++) X[at(i, cy, cx)] = out[i];
+      } else {
+        const auto m = phase_ptr(mats);
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+          T s = 0;
+#pragma unroll
+          for (int j = 0; j < Q; j++) s += m[j * P + i] * w[j];
+          X[at(i, cy, cx)] = s;
+        }
       }
     }
     __syncthreads();
     // ---- B_y^T on the y-line (qx = cx, z = cy < P), in place
     if (t < Q * P) {
-      const auto gB = phase_ptr(mats);
-      T          in[Q];
+      T in[Q];
 #pragma unroll
       for (int a = 0; a < Q; a++) in[a] = X[at(cy, a, cx)];
+      if constexpr (kRowWise) {
+        T out[P];
 #pragma unroll
-      for (int y = 0; y < P; y++) {
-        const auto m = kRowWise ? phase_ptr(mats + y) : gB + y;
-        T          s = 0;
+        for (int i = 0; i < P; i++) out[i] = 0;
+        transposed_line(mats, in, out);
 #pragma unroll
-        for (int a = 0; a < Q; a++) s += m[a * P] * in[a];
-        X[at(cy, y, cx)] = s;
+        for (int i = 0; i < P; i++) X[at(cy, i, cx)] = out[i];
+      } else {
+        const auto m = phase_ptr(mats);
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+          T s = 0;
+#pragma unroll
+          for (int j = 0; j < Q; j++) s += m[j * P + i] * in[j];
+          X[at(cy, i, cx)] = s;
+        }
       }
     }
     __syncthreads();
     // ---- B_x^T on the x-line (ny, nz) of nodes, in place
     if (xline) {
-      const auto gB = phase_ptr(mats);
-      T          in[Q];
+      T in[Q];
 #pragma unroll
       for (int a = 0; a < Q; a++) in[a] = X[at(nz, ny, a)];
+      if constexpr (kRowWise) {
+        T out[P];
 #pragma unroll
-      for (int x = 0; x < P; x++) {
-        const auto m   = kRowWise ? phase_ptr(mats + x) : gB + x;
-        T          acc = 0;
+        for (int i = 0; i < P; i++) out[i] = 0;
+        transposed_line(mats, in, out);
 #pragma unroll
-        for (int a = 0; a < Q; a++) acc += m[a * P] * in[a];
-        X[at(nz, ny, x)] = acc;
+        for (int i = 0; i < P; i++) X[at(nz, ny, i)] = out[i];
+      } else {
+        const auto m = phase_ptr(mats);
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+          T s = 0;
+#pragma unroll
+          for (int j = 0; j < Q; j++) s += m[j * P + i] * in[j];
+          X[at(nz, ny, i)] = s;
+        }
       }
     }
     __syncthreads();

@@ -43,11 +43,11 @@ int64_t brick_lds_bytes(int P, int Q, int qf, int scalar_bytes, const int *shape
 // measured on MI355X at 4M DoFs (ms per apply, stored / recomputed): mass
 // replaces one value (p=2 0.135 / 0.161, p=4 0.068 / 0.065, p=6 0.057 /
 // 0.058); FP32 reads half the bytes but computes the factors in FP64 all the
-// same, which costs as much as it saves at Q = 8 (0.071 / 0.073) and Q = 10
-// (0.088 / 0.092), not at Q = 7 (0.092 / 0.084) or Q = 9 (0.088 / 0.081),
-// whose stored layouts fill the wavefronts less well; three components share
-// one read of the factors (Q = 4: 0.210 / 0.214; Q = 3 0.654 / 0.620, Q = 5
-// 0.128 / 0.112, Q = 8 0.119 / 0.104).
+// same, which costs as much as it saves at Q = 8 (0.069 / 0.069) and Q = 10
+// (0.084 / 0.082), not at Q = 7 (0.093 / 0.082) or Q = 9 (0.087 / 0.077),
+// whose elements fill the wavefronts less well; three components share one
+// read of the factors (Q = 4: 0.210 / 0.214; Q = 3 0.654 / 0.620, Q = 5
+// 0.128 / 0.112, Q = 8 0.109 / 0.098).
 bool geo_pays(int Q, int qf, int num_comp, int scalar_bytes) {
   if (qf != kQfDiffusion && qf != kQfDiffusionKappa) return false;
   if (scalar_bytes == 4 && num_comp == 1) return Q != 8 && Q != 10;
@@ -350,6 +350,13 @@ bool admissible(int P, int Q, int qf, int num_comp, int scalar_bytes, int layout
 
 int plan_default_epb(const CeedMi355Operator op, int layout) {
   if (layout == mi355::kLayoutLines && op->geo_valid) return mi355::geo_default_epb(op->Q);
+  // three components work three times as long on an element's factors: with
+  // the transpose map, whose one launch fills the GPU, full wavefronts beat
+  // small workgroups (MI355X, 2-4M DoFs, us per apply: Q = 5 5 elements 74.9,
+  // 2 elements 79.7, with colours 138 and 126; Q = 7 5 elements 125, one 131)
+  if (layout == mi355::kLayoutLines && op->num_comp == 3 && op->scalar_bytes == 8 && op->qf == kQfDiffusion && op->scatter == 0 &&
+      (op->Q == 5 || op->Q == 7))
+    return 5;
   return mi355::default_epb(op->P, op->Q, op->qf, op->num_comp, op->scalar_bytes, layout);
 }
 
@@ -624,7 +631,7 @@ int mi355::create_plan(int qf, int scalar_type, int32_t num_comp, int32_t num_el
   // than the column layout at every order measured on MI355X, equal at p <= 2)
   // with its default workgroup size; CEED_MI355_LAYOUT / CEED_MI355_EPB override
   op->layout = mi355::kLayoutLines;
-  op->epb    = mi355::default_epb(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, op->layout);
+  op->epb    = plan_default_epb(op, op->layout);
   {
     int layout, epb;
     if (tuned_launch(op, &layout, &epb)) op->layout = layout, op->epb = epb;
