@@ -46,8 +46,9 @@ enum { CEED_MI355_FP64 = 0, CEED_MI355_FP32 = 1 };
 enum { CEED_MI355_QF_MASS = 0, CEED_MI355_QF_DIFFUSION = 1, CEED_MI355_QF_DIFFUSION_KAPPA = 2 };
 /* Field kinds of a run-time compiled fused operator (CeedMi355OperatorCreateHexJit):
  * an active field evaluated with CEED_EVAL_INTERP or CEED_EVAL_GRAD, or the
- * passive CEED_EVAL_NONE input (the plan's q_data). */
-enum { CEED_MI355_FIELD_INTERP = 0, CEED_MI355_FIELD_GRAD = 1, CEED_MI355_FIELD_PASSIVE = 2 };
+ * passive CEED_EVAL_NONE input (the plan's q_data); and the quadrature weights
+ * (CeedMi355PointOperatorCreate). */
+enum { CEED_MI355_FIELD_INTERP = 0, CEED_MI355_FIELD_GRAD = 1, CEED_MI355_FIELD_PASSIVE = 2, CEED_MI355_FIELD_WEIGHT = 3 };
 
 /* E^T mode flags of CeedMi355OperatorCreateHex (0: transpose map for P >= 6, colours below). */
 enum {
@@ -173,6 +174,17 @@ int CeedMi355OperatorCreateHexJit(const char *source_path, const char *function_
                                   int32_t num_out, const int32_t *out_kinds_host, int32_t q_comp, int32_t num_elem, int32_t P_1d, int32_t Q_1d,
                                   const double *interp_1d_host, const double *grad_1d_host, const int32_t *offsets_host, int64_t l_size, int flags,
                                   CeedMi355Operator *op);
+/* The same with several passive inputs: in_sizes_host[i] values per point of
+ * passive input i (other entries are not read), at most 32 together.  The
+ * plan's q_data holds them one after the other in field order; each is set
+ * with CeedMi355OperatorSetQDataComponents. */
+int CeedMi355OperatorCreateHexJitFields(const char *source_path, const char *function_name, int32_t num_in, const int32_t *in_kinds_host,
+                                        const int32_t *in_sizes_host, int32_t num_out, const int32_t *out_kinds_host, int32_t num_elem,
+                                        int32_t P_1d, int32_t Q_1d, const double *interp_1d_host, const double *grad_1d_host,
+                                        const int32_t *offsets_host, int64_t l_size, int flags, CeedMi355Operator *op);
+/* Load components [first, first + num) of such a plan's passive values from
+ * q_data in [elem][num][qpt]. */
+int CeedMi355OperatorSetQDataComponents(CeedMi355Operator op, int32_t first, int32_t num, const void *q_data, void *stream);
 /* Device pointer of the QFunction context for later applies of a plan made by
  * CeedMi355OperatorCreateHexJit (NULL: none). */
 int CeedMi355OperatorSetContext(CeedMi355Operator op, void *ctx_device);
@@ -239,6 +251,26 @@ int CeedMi355OperatorGetColors(CeedMi355Operator op, int32_t *num_colors, int32_
  * fixed E^T each). */
 int CeedMi355OperatorGetScatter(CeedMi355Operator op, int32_t *mode);
 int CeedMi355OperatorDestroy(CeedMi355Operator *op);
+
+typedef struct CeedMi355PointOperator_private *CeedMi355PointOperator;
+/* A QFunction whose output stays at the quadrature points, in one kernel
+ * compiled at run time: E and B of one active field of num_comp components
+ * (inputs CEED_MI355_FIELD_INTERP and/or _GRAD, sizes num_comp and
+ * 3 num_comp), quadrature weights (_WEIGHT) and passive EVAL_NONE inputs
+ * (_PASSIVE, in_sizes_host[i] values per point, at most 32 together), out_size
+ * values per point out.  FP64, P_1d <= Q_1d <= 10, num_comp <= 3.  The fused
+ * form of the set-up operators of the reference's examples
+ * (examples/ceed/ex1-volume.c:195-236), which its generated backend runs as
+ * one kernel (backends/hip-gen/ceed-hip-gen-operator-build.cpp). */
+int CeedMi355PointOperatorCreate(const char *source_path, const char *function_name, int32_t num_in, const int32_t *in_kinds_host,
+                                 const int32_t *in_sizes_host, int32_t out_size, int32_t num_comp, int32_t num_elem, int32_t P_1d, int32_t Q_1d,
+                                 const double *interp_1d_host, const double *grad_1d_host, const double *q_weight_1d_host,
+                                 const int32_t *offsets_host, int32_t comp_stride, int64_t l_size, CeedMi355PointOperator *op);
+/* v (= or, with add, +=) the values in [elem][out_size][qpt]; passive_host: the
+ * passive fields' device arrays in field order, each [elem][size][qpt]. */
+int CeedMi355PointOperatorApply(CeedMi355PointOperator op, void *ctx_device, const double *u, const double *const *passive_host, double *v, int add,
+                                void *stream);
+int CeedMi355PointOperatorDestroy(CeedMi355PointOperator *op);
 
 /* ------------------------------------------------------------------------ */
 /* L-vector arithmetic                                                       */

@@ -79,7 +79,7 @@ __device__ __forceinline__ double pair_swap(double x) {
 // diffusion two, and a third where the z-derivatives wait in LDS:
 // line_dz_in_lds); the shared pipeline below (line_element) goes back and forth.
 __host__ __device__ constexpr bool line_dz_in_lds(int Q, int ncomp, int qf, int sb, bool geo) {
-  return !geo && qf != kQfMass && ncomp == 1 && sb == 8 && Q >= 10;
+  return !geo && (qf == kQfDiffusion || qf == kQfDiffusionKappa) && ncomp == 1 && sb == 8 && Q >= 10;
 }
 __host__ __device__ constexpr int line_kernel_slabs(int Q, int ncomp, int qf, int sb, bool geo) {
   return qf == kQfMass ? 1 : line_dz_in_lds(Q, ncomp, qf, sb, geo) ? 3 : 2;

@@ -18,7 +18,6 @@ namespace mi355 {
 void collocated_grad(int P, int Q, const double *interp, const double *grad, double *collo);
 
 int lds_bytes(int P, int Q, int qf, int num_comp, int epb, int scalar_bytes, int layout) {
-  if (layout == kLayoutLines && qf == kQfJit) return scalar_bytes * epb * 3 * Q * Q * Q;
   if (layout == kLayoutLines) return (int)line_lds_bytes(Q, num_comp, qf, scalar_bytes, false, epb);
   if (layout == kLayoutPoints) return scalar_bytes * (Q * P + Q * Q + epb * (qf == kQfMass ? 3 : 4) * Q * Q * Q);
   const int slabs = qf == kQfMass ? 2 : 3;
@@ -902,6 +901,32 @@ extern "C" int CeedMi355OperatorSetQData(CeedMi355Operator op, const void *q_dat
     return CEED_MI355_SUCCESS;
   }
   MI355_CHECK(false, CEED_MI355_ERROR_UNSUPPORTED, "SetQData for the kappa operator: build the 6 Voigt entries with BuildQData");
+}
+
+namespace {
+// components [first, first + nc) of every element block of q_comp components, from src [elem][nc][q3] in the caller's order
+__global__ void __launch_bounds__(256) scatter_components(int64_t num_elem, int32_t q3, int32_t q_comp, int32_t first, int32_t nc,
+                                                          const int32_t *__restrict__ perm, const double *__restrict__ src,
+                                                          double *__restrict__ q_data) {
+  const int64_t per = (int64_t)nc * q3, n = num_elem * per;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t p = i / per, r = i - p * per;
+    q_data[(p * q_comp + first) * q3 + r] = src[perm[p] * per + r];
+  }
+}
+}  // namespace
+
+extern "C" int CeedMi355OperatorSetQDataComponents(CeedMi355Operator op, int32_t first, int32_t num, const void *q_data, void *stream) {
+  MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
+  MI355_CHECK(op->qf == kQfJit && op->scalar_type == CEED_MI355_FP64, CEED_MI355_ERROR_UNSUPPORTED,
+              "components of the passive fields belong to plans of run-time compiled QFunctions");
+  MI355_CHECK(first >= 0 && num >= 1 && first + num <= op->q_comp, CEED_MI355_ERROR_DIMENSION, "components %d..%d of %d", first, first + num, op->q_comp);
+  const int32_t q3 = op->Q * op->Q * op->Q;
+  if (op->num_elem > 0)
+    scatter_components<<<mi355_blocks((int64_t)op->num_elem * num * q3, 256), 256, 0, (hipStream_t)stream>>>(
+        op->num_elem, q3, op->q_comp, first, num, op->d_perm, (const double *)q_data, (double *)op->d_qdata);
+  MI355_LAUNCH_CHECK();
+  return CEED_MI355_SUCCESS;
 }
 
 extern "C" int CeedMi355OperatorGetQData(CeedMi355Operator op, void *q_data, void *stream) {

@@ -12,9 +12,13 @@
 #include <string.h>
 
 #include <fstream>
+#include <list>
+#include <memory>
+#include <mutex>
 #include <set>
 #include <sstream>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "mi355_common.h"
@@ -99,27 +103,58 @@ int mi355_jit_user_source(const char *source_path, std::string &out) {
   return CEED_MI355_SUCCESS;
 }
 
+namespace {
+// Code objects hipRTC has made in this process, by their whole source text: an
+// operator set up again around the same QFunction (a new mesh, the next time
+// step) loads the code instead of compiling it, 0.1-0.2 s each time.  Host
+// memory only, every user loads a module of its own from it; the oldest go
+// when there are more than kMostObjects.
+constexpr size_t                                                   kMostObjects = 64;
+std::mutex                                                         g_code_mutex;
+std::list<std::pair<std::string, std::shared_ptr<std::vector<char>>>> g_code;  // most recently used first
+
+std::shared_ptr<std::vector<char>> cached_code(const std::string &text) {
+  std::lock_guard<std::mutex> lock(g_code_mutex);
+  for (auto it = g_code.begin(); it != g_code.end(); ++it)
+    if (it->first == text) {
+      g_code.splice(g_code.begin(), g_code, it);
+      return it->second;
+    }
+  return nullptr;
+}
+
+void keep_code(const std::string &text, const std::shared_ptr<std::vector<char>> &code) {
+  std::lock_guard<std::mutex> lock(g_code_mutex);
+  g_code.emplace_front(text, code);
+  if (g_code.size() > kMostObjects) g_code.pop_back();
+}
+}  // namespace
+
 int mi355_jit_build(const std::string &code, const char *what, const char *kernel_name, hipModule_t *module, hipFunction_t *fn) {
-  hiprtcProgram prog;
-  MI355_CHECK(hiprtcCreateProgram(&prog, code.c_str(), "ceed-mi355-jit.hip", 0, nullptr, nullptr) == HIPRTC_SUCCESS, CEED_MI355_ERROR_BACKEND,
-              "hiprtcCreateProgram failed");
-  const char  *opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=fast", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
-  hiprtcResult rc     = hiprtcCompileProgram(prog, 8, opts);
-  if (rc != HIPRTC_SUCCESS) {
-    size_t log_size = 0;
-    hiprtcGetProgramLogSize(prog, &log_size);
-    std::string log(log_size + 1, '\0');
-    hiprtcGetProgramLog(prog, &log[0]);
+  *module                                   = nullptr;
+  std::shared_ptr<std::vector<char>> binary = cached_code(code);
+  if (!binary) {
+    hiprtcProgram prog;
+    MI355_CHECK(hiprtcCreateProgram(&prog, code.c_str(), "ceed-mi355-jit.hip", 0, nullptr, nullptr) == HIPRTC_SUCCESS, CEED_MI355_ERROR_BACKEND,
+                "hiprtcCreateProgram failed");
+    const char *opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=fast", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
+    hiprtcResult rc    = hiprtcCompileProgram(prog, 8, opts);
+    if (rc != HIPRTC_SUCCESS) {
+      size_t log_size = 0;
+      hiprtcGetProgramLogSize(prog, &log_size);
+      std::string log(log_size + 1, '\0');
+      hiprtcGetProgramLog(prog, &log[0]);
+      hiprtcDestroyProgram(&prog);
+      MI355_CHECK(false, CEED_MI355_ERROR_BACKEND, "hipRTC failed for %s: %s", what, log.c_str());
+    }
+    size_t code_size = 0;
+    hiprtcGetCodeSize(prog, &code_size);
+    binary = std::make_shared<std::vector<char>>(code_size);
+    hiprtcGetCode(prog, binary->data());
     hiprtcDestroyProgram(&prog);
-    MI355_CHECK(false, CEED_MI355_ERROR_BACKEND, "hipRTC failed for %s: %s", what, log.c_str());
+    keep_code(code, binary);
   }
-  size_t code_size = 0;
-  hiprtcGetCodeSize(prog, &code_size);
-  std::vector<char> binary(code_size);
-  hiprtcGetCode(prog, binary.data());
-  hiprtcDestroyProgram(&prog);
-  *module = nullptr;
-  if (hipModuleLoadData(module, binary.data()) != hipSuccess || hipModuleGetFunction(fn, *module, kernel_name) != hipSuccess) {
+  if (hipModuleLoadData(module, binary->data()) != hipSuccess || hipModuleGetFunction(fn, *module, kernel_name) != hipSuccess) {
     if (*module) (void)hipModuleUnload(*module);
     *module = nullptr;
     MI355_CHECK(false, CEED_MI355_ERROR_BACKEND, "loading the compiled kernel %s failed", what);
@@ -157,34 +192,13 @@ extern "C" int CeedMi355QFunctionCompile(const char *source_path, const char *fu
   for (int i = 0; i < num_out; i++)
     src << "    for (int k = 0; k < " << out_sizes[i] << "; k++) f.out[" << i << "][(e * " << out_sizes[i] << " + k) * Q + q] = out_" << i << "[k];\n";
   src << "  }\n}\n";
-  const std::string code = src.str();
-
-  hiprtcProgram prog;
-  MI355_CHECK(hiprtcCreateProgram(&prog, code.c_str(), "ceed-mi355-qfunction.hip", 0, nullptr, nullptr) == HIPRTC_SUCCESS,
-              CEED_MI355_ERROR_BACKEND, "hiprtcCreateProgram failed");
-  const char  *opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=fast", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
-  hiprtcResult rc     = hiprtcCompileProgram(prog, 8, opts);
-  if (rc != HIPRTC_SUCCESS) {
-    size_t log_size = 0;
-    hiprtcGetProgramLogSize(prog, &log_size);
-    std::string log(log_size + 1, '\0');
-    hiprtcGetProgramLog(prog, &log[0]);
-    hiprtcDestroyProgram(&prog);
-    MI355_CHECK(false, CEED_MI355_ERROR_BACKEND, "hipRTC failed for %s:%s: %s", source_path, function_name, log.c_str());
-  }
-  size_t code_size = 0;
-  hiprtcGetCodeSize(prog, &code_size);
-  std::vector<char> binary(code_size);
-  hiprtcGetCode(prog, binary.data());
-  hiprtcDestroyProgram(&prog);
-
   CeedMi355QFunction qf = new CeedMi355QFunction_private();
   qf->num_in            = num_in;
   qf->num_out           = num_out;
-  if (hipModuleLoadData(&qf->module, binary.data()) != hipSuccess ||
-      hipModuleGetFunction(&qf->kernel, qf->module, "CeedMi355QFKernel") != hipSuccess) {
+  ierr = mi355_jit_build(src.str(), (std::string(source_path) + ":" + function_name).c_str(), "CeedMi355QFKernel", &qf->module, &qf->kernel);
+  if (ierr) {
     delete qf;
-    MI355_CHECK(false, CEED_MI355_ERROR_BACKEND, "loading the compiled QFunction %s failed", function_name);
+    return ierr;
   }
   *qf_out = qf;
   return CEED_MI355_SUCCESS;

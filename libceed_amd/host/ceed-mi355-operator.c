@@ -14,10 +14,12 @@
  * Fused path, run-time compiled: an operator whose pointwise function is a
  * user (or any non-inlined) QFunction, with scalar active fields on one
  * standard restriction and one 3D tensor basis (inputs INTERP and/or GRAD,
- * outputs INTERP and/or GRAD) and at most one passive EVAL_NONE input, runs
- * as one fused kernel too: the QFunction source is compiled with hipRTC into
+ * outputs INTERP and/or GRAD) and passive EVAL_NONE inputs, runs as one fused
+ * kernel too: the QFunction source is compiled with hipRTC into
  * the line-layout kernel (CeedMi355OperatorCreateHexJit), the role of the
  * reference's hip-gen backend (backends/hip-gen/ceed-hip-gen-operator-build.cpp).
+ * So does one whose output stays at the quadrature points (geometric factors
+ * from coordinates: CeedMi355PointOperatorCreate).
  * CEED_MI355_FUSE_QFUNCTIONS=0 keeps such operators on the generic path.
  *
  * Generic path (any other operator): the staged apply of the reference
@@ -32,14 +34,24 @@
 
 #include "ceed-mi355-backend.h"
 
+/* A kernel library without these entry points leaves their operators on the
+ * generic path. */
+#pragma weak CeedMi355OperatorCreateHexJitFields
+#pragma weak CeedMi355OperatorSetQDataComponents
+#pragma weak CeedMi355PointOperatorCreate
+#pragma weak CeedMi355PointOperatorApply
+#pragma weak CeedMi355PointOperatorDestroy
+
 typedef struct {
   bool     is_set_up, fused, jit;
   /* fused path */
   CeedMi355Operator hex;
   CeedSize          l_size;
-  uint64_t          qdata_state;
-  bool              qdata_loaded;
-  CeedInt           qdata_field; /* input field of the geometric factors, -1: none */
+  CeedInt           num_passive; /* passive inputs held in the plan: their fields, in order, and sizes */
+  CeedInt           passive_field[CEED_FIELD_MAX], passive_size[CEED_FIELD_MAX];
+  /* values at the quadrature points (CeedMi355PointOperator) */
+  CeedMi355PointOperator points;
+  CeedSize               points_size; /* E-vector length of the output */
   /* generic path */
   CeedInt  num_in, num_out, num_elem, Q;
   double  *e_in[CEED_FIELD_MAX], *q_in[CEED_FIELD_MAX];
@@ -168,8 +180,9 @@ static int try_fused(CeedOperator op, OperatorData *d) {
     }
   }
 done:
-  d->fused       = ok;
-  d->qdata_field = 1;
+  d->fused            = ok;
+  d->num_passive      = 1;
+  d->passive_field[0] = 1;
   CeedCallBackend(CeedElemRestrictionDestroy(&ru));
   CeedCallBackend(CeedElemRestrictionDestroy(&rv));
   CeedCallBackend(CeedElemRestrictionDestroy(&rq));
@@ -189,13 +202,13 @@ done:
 static int try_fused_jit(CeedOperator op, OperatorData *d) {
   Ceed                 ceed;
   CeedQFunction        qf;
-  CeedInt              num_in, num_out, q_comp = 0, qdata_field = -1, P = 0, Q = 0;
+  CeedInt              num_in, num_out, q_comp = 0, num_passive = 0, P = 0, Q = 0;
   CeedOperatorField   *in, *out;
   CeedQFunctionField  *qf_in, *qf_out;
   const char          *path, *name;
   CeedElemRestriction  ru = NULL;
   CeedBasis            bu = NULL;
-  int32_t              in_kinds[3], out_kinds[2];
+  int32_t              in_kinds[CEED_FIELD_MAX], in_sizes[CEED_FIELD_MAX], out_kinds[2];
   int                  ok = 1;
   const char          *env = getenv("CEED_MI355_FUSE_QFUNCTIONS");
 
@@ -207,7 +220,7 @@ static int try_fused_jit(CeedOperator op, OperatorData *d) {
   CeedCallBackend(CeedQFunctionGetKernelName(qf, &name));
   CeedCallBackend(CeedOperatorGetFields(op, &num_in, &in, &num_out, &out));
   CeedCallBackend(CeedQFunctionGetFields(qf, NULL, &qf_in, NULL, &qf_out));
-  if (!path || !name || num_in < 1 || num_in > 3 || num_out < 1 || num_out > 2) ok = 0;
+  if (!path || !name || num_in < 1 || num_in > 10 || num_out < 1 || num_out > 2) ok = 0;
   for (CeedInt f = 0; ok && f < num_in + num_out; f++) {
     const bool          is_in = f < num_in;
     const CeedInt       i     = is_in ? f : f - num_in;
@@ -232,10 +245,12 @@ static int try_fused_jit(CeedOperator op, OperatorData *d) {
       const int32_t kind = mode == CEED_EVAL_GRAD ? CEED_MI355_FIELD_GRAD : CEED_MI355_FIELD_INTERP;
       if (is_in) in_kinds[i] = kind;
       else out_kinds[i] = kind;
-    } else if (is_in && vec != CEED_VECTOR_NONE && mode == CEED_EVAL_NONE && qdata_field < 0 && rstr != CEED_ELEMRESTRICTION_NONE) {
-      in_kinds[i] = CEED_MI355_FIELD_PASSIVE;
-      qdata_field = i;
-      q_comp      = size;
+    } else if (is_in && vec != CEED_VECTOR_NONE && mode == CEED_EVAL_NONE && rstr != CEED_ELEMRESTRICTION_NONE) {
+      in_kinds[i]                     = CEED_MI355_FIELD_PASSIVE;
+      in_sizes[i]                     = size;
+      d->passive_field[num_passive]   = i;
+      d->passive_size[num_passive++]  = size;
+      q_comp += size;
     } else {
       ok = 0;
     }
@@ -255,16 +270,17 @@ static int try_fused_jit(CeedOperator op, OperatorData *d) {
     CeedCallBackend(CeedElemRestrictionGetElementSize(ru, &elem_size));
     CeedCallBackend(CeedElemRestrictionGetNumElements(ru, &num_elem));
     ok = type == CEED_RESTRICTION_STANDARD && dim == 3 && nc == 1 && rc == 1 && elem_size == P * P * P && P >= 2 && P <= 9 && Q >= P && Q <= 10;
-    if (ok && qdata_field >= 0) {  /* the passive field: Q^3 points per element, its size per point */
+    for (CeedInt k = 0; ok && k < num_passive; k++) {  /* a passive field: Q^3 points per element, its size per point */
       CeedElemRestriction rq;
       CeedInt             q_elem, q_nc, q_ne;
-      CeedCallBackend(CeedOperatorFieldGetElemRestriction(in[qdata_field], &rq));
+      CeedCallBackend(CeedOperatorFieldGetElemRestriction(in[d->passive_field[k]], &rq));
       CeedCallBackend(CeedElemRestrictionGetElementSize(rq, &q_elem));
       CeedCallBackend(CeedElemRestrictionGetNumComponents(rq, &q_nc));
       CeedCallBackend(CeedElemRestrictionGetNumElements(rq, &q_ne));
-      ok = q_elem == Q * Q * Q && q_nc == q_comp && q_ne == num_elem;
+      ok = q_elem == Q * Q * Q && q_nc == d->passive_size[k] && q_ne == num_elem;
       CeedCallBackend(CeedElemRestrictionDestroy(&rq));
     }
+    if (num_passive > 1 && !(CeedMi355OperatorCreateHexJitFields && CeedMi355OperatorSetQDataComponents)) ok = 0;
     if (ok) {
       const CeedScalar *interp, *grad;
       const CeedInt    *offsets;
@@ -272,8 +288,10 @@ static int try_fused_jit(CeedOperator op, OperatorData *d) {
       CeedCallBackend(CeedBasisGetGrad1D(bu, &grad));
       CeedCallBackend(CeedElemRestrictionGetLVectorSize(ru, &d->l_size));
       CeedCallBackend(CeedElemRestrictionGetOffsets(ru, CEED_MEM_HOST, &offsets));
-      int ierr = CeedMi355OperatorCreateHexJit(path, name, num_in, in_kinds, num_out, out_kinds, q_comp, num_elem, P, Q, interp, grad, offsets,
-                                               d->l_size, 0, &d->hex);
+      int ierr = num_passive > 1 ? CeedMi355OperatorCreateHexJitFields(path, name, num_in, in_kinds, in_sizes, num_out, out_kinds, num_elem, P, Q,
+                                                                       interp, grad, offsets, d->l_size, 0, &d->hex)
+                                 : CeedMi355OperatorCreateHexJit(path, name, num_in, in_kinds, num_out, out_kinds, q_comp, num_elem, P, Q, interp,
+                                                                 grad, offsets, d->l_size, 0, &d->hex);
       CeedCallBackend(CeedElemRestrictionRestoreOffsets(ru, &offsets));
       if (ierr == CEED_MI355_ERROR_UNSUPPORTED) ok = 0;
       else CeedCallBackend(CeedMi355Check(ceed, ierr));
@@ -283,7 +301,7 @@ static int try_fused_jit(CeedOperator op, OperatorData *d) {
   }
   d->fused       = ok;
   d->jit         = ok;
-  d->qdata_field = qdata_field;
+  d->num_passive = num_passive;
   CeedCallBackend(CeedElemRestrictionDestroy(&ru));
   CeedCallBackend(CeedBasisDestroy(&bu));
   CeedCallBackend(CeedQFunctionDestroy(&qf));
@@ -291,14 +309,11 @@ static int try_fused_jit(CeedOperator op, OperatorData *d) {
   return CEED_ERROR_SUCCESS;
 }
 
-/* reload the geometric factors into the plan when their vector changed, and
- * (run-time compiled plans) hand over the current device context */
+/* reload the passive values into the plan whose vector changed, and (run-time
+ * compiled plans) hand over the current device context */
 static int fused_sync_qdata(CeedOperator op, OperatorData *d) {
-  Ceed                ceed;
-  CeedOperatorField  *in;
-  CeedElemRestriction rq;
-  CeedVector          vq;
-  uint64_t            state;
+  Ceed               ceed;
+  CeedOperatorField *in;
   CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
   if (d->jit) {
     CeedQFunction qf;
@@ -308,24 +323,177 @@ static int fused_sync_qdata(CeedOperator op, OperatorData *d) {
     CeedCallBackend(CeedMi355Check(ceed, CeedMi355OperatorSetContext(d->hex, ctx)));
     CeedCallBackend(CeedQFunctionDestroy(&qf));
   }
-  if (d->qdata_field < 0) return CeedDestroy(&ceed);
   CeedCallBackend(CeedOperatorGetFields(op, NULL, &in, NULL, NULL));
-  CeedCallBackend(CeedOperatorFieldGetElemRestriction(in[d->qdata_field], &rq));
-  CeedCallBackend(CeedOperatorFieldGetVector(in[d->qdata_field], &vq));
-  CeedCallBackend(CeedVectorGetState(vq, &state));
-  if (!d->qdata_loaded || state != d->qdata_state) {
-    const double *e;
-    double       *temp;
-    CeedCallBackend(qdata_evector(ceed, rq, vq, &e, &temp));
-    CeedCallBackend(CeedMi355Check(ceed, CeedMi355OperatorSetQData(d->hex, e, NULL)));
-    if (temp) CeedMi355Free(temp);
-    d->qdata_state  = state;
-    d->qdata_loaded = true;
+  for (CeedInt k = 0, first = 0; k < d->num_passive; first += d->passive_size[k++]) {
+    CeedElemRestriction rq;
+    CeedVector          vq;
+    uint64_t            state;
+    CeedCallBackend(CeedOperatorFieldGetVector(in[d->passive_field[k]], &vq));
+    CeedCallBackend(CeedVectorGetState(vq, &state));
+    if (!d->in_valid[k] || state != d->in_state[k]) {
+      const double *e;
+      double       *temp;
+      CeedCallBackend(CeedOperatorFieldGetElemRestriction(in[d->passive_field[k]], &rq));
+      CeedCallBackend(qdata_evector(ceed, rq, vq, &e, &temp));
+      if (d->num_passive > 1) CeedCallBackend(CeedMi355Check(ceed, CeedMi355OperatorSetQDataComponents(d->hex, first, d->passive_size[k], e, NULL)));
+      else CeedCallBackend(CeedMi355Check(ceed, CeedMi355OperatorSetQData(d->hex, e, NULL)));
+      if (temp) CeedMi355Free(temp);
+      CeedCallBackend(CeedElemRestrictionDestroy(&rq));
+      d->in_state[k] = state;
+      d->in_valid[k] = true;
+    }
+    CeedCallBackend(CeedVectorDestroy(&vq));
   }
-  CeedCallBackend(CeedVectorDestroy(&vq));
-  CeedCallBackend(CeedElemRestrictionDestroy(&rq));
+  return CeedDestroy(&ceed);
+}
+
+/* ------------------------------------------------------------------------ */
+/* values at the quadrature points                                           */
+/* ------------------------------------------------------------------------ */
+/* Set up CeedMi355PointOperator when the operator has its shape: one active
+ * field of up to three components on a standard restriction and a 3D tensor
+ * basis (INTERP and/or GRAD), any of quadrature weights and passive EVAL_NONE
+ * fields with backend strides, and one active EVAL_NONE output with backend
+ * strides; leaves d->points NULL otherwise. */
+static int try_points(CeedOperator op, OperatorData *d) {
+  Ceed                ceed;
+  CeedQFunction       qf;
+  CeedInt             num_in, num_out, num_elem, num_qpts, num_comp = 0, num_passive = 0, P = 0, Q = 0, out_size = 0;
+  CeedOperatorField  *in, *out;
+  CeedQFunctionField *qf_in, *qf_out;
+  const char         *path, *name, *env = getenv("CEED_MI355_FUSE_QFUNCTIONS");
+  CeedElemRestriction ru = NULL;
+  CeedBasis           bu = NULL, bw = NULL;
+  int32_t             in_kinds[CEED_FIELD_MAX], in_sizes[CEED_FIELD_MAX];
+  bool                ok;
+
+  if ((env && !strcmp(env, "0")) || !CeedMi355PointOperatorCreate || !CeedMi355PointOperatorApply || !CeedMi355PointOperatorDestroy)
+    return CEED_ERROR_SUCCESS;
+  CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
+  CeedCallBackend(CeedOperatorGetQFunction(op, &qf));
+  CeedCallBackend(CeedQFunctionGetSourcePath(qf, &path));
+  CeedCallBackend(CeedQFunctionGetKernelName(qf, &name));
+  CeedCallBackend(CeedOperatorGetFields(op, &num_in, &in, &num_out, &out));
+  CeedCallBackend(CeedQFunctionGetFields(qf, NULL, &qf_in, NULL, &qf_out));
+  CeedCallBackend(CeedOperatorGetNumElements(op, &num_elem));
+  CeedCallBackend(CeedOperatorGetNumQuadraturePoints(op, &num_qpts));
+  ok = path && name && num_in >= 1 && num_in <= 10 && num_out == 1;
+  for (CeedInt f = 0; ok && f < num_in + num_out; f++) {
+    const bool          is_in = f < num_in;
+    const CeedInt       i     = is_in ? f : f - num_in;
+    CeedElemRestriction rstr;
+    CeedBasis           basis;
+    CeedVector          vec;
+    CeedEvalMode        mode;
+    CeedInt             size, elem_size = 0, rstr_comp = 0;
+    bool                backend = false;
+    CeedCallBackend(CeedOperatorFieldGetElemRestriction(is_in ? in[i] : out[i], &rstr));
+    CeedCallBackend(CeedOperatorFieldGetBasis(is_in ? in[i] : out[i], &basis));
+    CeedCallBackend(CeedOperatorFieldGetVector(is_in ? in[i] : out[i], &vec));
+    CeedCallBackend(CeedQFunctionFieldGetEvalMode(is_in ? qf_in[i] : qf_out[i], &mode));
+    CeedCallBackend(CeedQFunctionFieldGetSize(is_in ? qf_in[i] : qf_out[i], &size));
+    if (rstr != CEED_ELEMRESTRICTION_NONE) {
+      CeedCallBackend(CeedElemRestrictionHasBackendStrides(rstr, &backend));
+      CeedCallBackend(CeedElemRestrictionGetElementSize(rstr, &elem_size));
+      CeedCallBackend(CeedElemRestrictionGetNumComponents(rstr, &rstr_comp));
+    }
+    const bool at_points = mode == CEED_EVAL_NONE && backend && elem_size == num_qpts && rstr_comp == size;
+    if (!is_in) {
+      ok       = vec == CEED_VECTOR_ACTIVE && at_points;
+      out_size = size;
+      if (ok) CeedCallBackend(CeedElemRestrictionGetEVectorSize(rstr, &d->points_size));
+    } else if (vec == CEED_VECTOR_ACTIVE) {
+      ok = (mode == CEED_EVAL_INTERP || mode == CEED_EVAL_GRAD) && (!ru || (rstr == ru && basis == bu));
+      if (ok && !ru) {
+        CeedCallBackend(CeedElemRestrictionReferenceCopy(rstr, &ru));
+        CeedCallBackend(CeedBasisReferenceCopy(basis, &bu));
+      }
+      in_kinds[i] = mode == CEED_EVAL_GRAD ? CEED_MI355_FIELD_GRAD : CEED_MI355_FIELD_INTERP;
+    } else if (mode == CEED_EVAL_WEIGHT && basis != CEED_BASIS_NONE) {
+      ok          = !bw || basis == bw;
+      in_kinds[i] = CEED_MI355_FIELD_WEIGHT;
+      if (ok && !bw) CeedCallBackend(CeedBasisReferenceCopy(basis, &bw));
+    } else {
+      ok                            = vec != CEED_VECTOR_NONE && at_points;
+      in_kinds[i]                   = CEED_MI355_FIELD_PASSIVE;
+      d->passive_field[num_passive] = i;
+      d->passive_size[num_passive++] = size;
+    }
+    if (is_in) in_sizes[i] = size;
+    CeedCallBackend(CeedVectorDestroy(&vec));
+    CeedCallBackend(CeedBasisDestroy(&basis));
+    CeedCallBackend(CeedElemRestrictionDestroy(&rstr));
+  }
+  if (ok && ru && bu != CEED_BASIS_NONE) {
+    CeedRestrictionType type;
+    CeedInt             dim, rc, elem_size, re, Qw = 0, dim_w = 3;
+    CeedCallBackend(CeedElemRestrictionGetType(ru, &type));
+    CeedCallBackend(CeedBasisGetDimension(bu, &dim));
+    CeedCallBackend(CeedBasisGetNumComponents(bu, &num_comp));
+    CeedCallBackend(CeedElemRestrictionGetNumComponents(ru, &rc));
+    CeedCallBackend(CeedBasisGetNumNodes1D(bu, &P));
+    CeedCallBackend(CeedBasisGetNumQuadraturePoints1D(bu, &Q));
+    CeedCallBackend(CeedElemRestrictionGetElementSize(ru, &elem_size));
+    CeedCallBackend(CeedElemRestrictionGetNumElements(ru, &re));
+    if (bw) {
+      CeedCallBackend(CeedBasisGetDimension(bw, &dim_w));
+      CeedCallBackend(CeedBasisGetNumQuadraturePoints1D(bw, &Qw));
+    }
+    ok = type == CEED_RESTRICTION_STANDARD && dim == 3 && dim_w == 3 && rc == num_comp && elem_size == P * P * P && re == num_elem &&
+         num_qpts == Q * Q * Q && (!bw || Qw == Q) && P >= 2 && P <= Q && Q <= 10;
+    if (ok) {
+      const CeedScalar *interp, *grad, *weights = NULL;
+      const CeedInt    *offsets;
+      CeedInt           comp_stride;
+      CeedSize          l_size;
+      CeedCallBackend(CeedBasisGetInterp1D(bu, &interp));
+      CeedCallBackend(CeedBasisGetGrad1D(bu, &grad));
+      if (bw) CeedCallBackend(CeedBasisGetQWeights(bw, &weights));
+      CeedCallBackend(CeedElemRestrictionGetCompStride(ru, &comp_stride));
+      CeedCallBackend(CeedElemRestrictionGetLVectorSize(ru, &l_size));
+      CeedCallBackend(CeedElemRestrictionGetOffsets(ru, CEED_MEM_HOST, &offsets));
+      const int ierr = CeedMi355PointOperatorCreate(path, name, num_in, in_kinds, in_sizes, out_size, num_comp, num_elem, P, Q, interp, grad, weights,
+                                                    offsets, comp_stride, l_size, &d->points);
+      CeedCallBackend(CeedElemRestrictionRestoreOffsets(ru, &offsets));
+      if (ierr != CEED_MI355_ERROR_UNSUPPORTED) CeedCallBackend(CeedMi355Check(ceed, ierr));
+    }
+  }
+  d->num_passive = num_passive;
+  CeedCallBackend(CeedElemRestrictionDestroy(&ru));
+  CeedCallBackend(CeedBasisDestroy(&bu));
+  CeedCallBackend(CeedBasisDestroy(&bw));
+  CeedCallBackend(CeedQFunctionDestroy(&qf));
   CeedCallBackend(CeedDestroy(&ceed));
   return CEED_ERROR_SUCCESS;
+}
+
+/* out (= or +=) the values at the quadrature points */
+static int points_apply(CeedOperator op, OperatorData *d, CeedVector in_vec, CeedVector out_vec, bool add) {
+  Ceed               ceed;
+  CeedQFunction      qf;
+  CeedOperatorField *in;
+  CeedScalar        *du, *dv;
+  const double      *passive[CEED_FIELD_MAX];
+  void              *ctx;
+  CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
+  CeedCallBackend(CeedOperatorGetQFunction(op, &qf));
+  CeedCallBackend(CeedMi355QFunctionContextDevice(qf, &ctx));
+  CeedCallBackend(CeedOperatorGetFields(op, NULL, &in, NULL, NULL));
+  for (CeedInt k = 0; k < d->num_passive; k++) {
+    CeedVector  vec;
+    CeedScalar *dp;
+    CeedCallBackend(CeedOperatorFieldGetVector(in[d->passive_field[k]], &vec));
+    CeedCallBackend(CeedMi355VectorDevice(vec, false, &dp));
+    passive[k] = dp;
+    CeedCallBackend(CeedVectorDestroy(&vec));
+  }
+  CeedCallBackend(CeedMi355VectorDevice(in_vec, false, &du));
+  if (add) CeedCallBackend(CeedVectorGetArray(out_vec, CEED_MEM_DEVICE, &dv));
+  else CeedCallBackend(CeedVectorGetArrayWrite(out_vec, CEED_MEM_DEVICE, &dv));
+  CeedCallBackend(CeedMi355Check(ceed, CeedMi355PointOperatorApply(d->points, ctx, du, passive, dv, add, NULL)));
+  CeedCallBackend(CeedVectorRestoreArray(out_vec, &dv));
+  CeedCallBackend(CeedQFunctionDestroy(&qf));
+  return CeedDestroy(&ceed);
 }
 
 /* ------------------------------------------------------------------------ */
@@ -491,7 +659,8 @@ static int setup(CeedOperator op, OperatorData *d) {
   if (d->is_set_up) return CEED_ERROR_SUCCESS;
   CeedCallBackend(try_fused(op, d));
   if (!d->fused) CeedCallBackend(try_fused_jit(op, d));
-  if (!d->fused) CeedCallBackend(generic_setup(op, d));
+  if (!d->fused) CeedCallBackend(try_points(op, d));
+  if (!d->fused && !d->points) CeedCallBackend(generic_setup(op, d));
   d->is_set_up = true;
   return CEED_ERROR_SUCCESS;
 }
@@ -502,6 +671,7 @@ static int OperatorApplyAdd(CeedOperator op, CeedVector in, CeedVector out, Ceed
   (void)request;
   CeedCallBackend(CeedOperatorGetData(op, &d));
   CeedCallBackend(setup(op, d));
+  if (d->points && out != CEED_VECTOR_NONE) return points_apply(op, d, in, out, true);
   if (!d->fused) return generic_apply_add(op, d, in, out);
   CeedScalar *du, *dv;
   CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
@@ -521,6 +691,7 @@ static int OperatorApply(CeedOperator op, CeedVector in, CeedVector out, CeedReq
   CeedCallBackend(CeedOperatorGetData(op, &d));
   CeedCallBackend(setup(op, d));
   if (out != CEED_VECTOR_NONE) CeedCallBackend(CeedVectorGetLength(out, &out_len));
+  if (d->points && out != CEED_VECTOR_NONE && out_len == d->points_size) return points_apply(op, d, in, out, false);
   /* the fused plan overwrites its whole L-vector; a longer output (or the
    * generic path) is zeroed first and accumulated into */
   if (!d->fused || out == CEED_VECTOR_NONE || out_len != d->l_size) {
@@ -569,6 +740,7 @@ static int OperatorDestroy(CeedOperator op) {
   OperatorData *d;
   CeedCallBackend(CeedOperatorGetData(op, &d));
   if (d->hex) CeedMi355OperatorDestroy(&d->hex);
+  if (d->points) CeedMi355PointOperatorDestroy(&d->points);
   for (CeedInt i = 0; i < CEED_FIELD_MAX; i++) {
     if (d->q_in[i] && !d->q_in_is_e[i]) CeedMi355Free(d->q_in[i]);
     if (d->e_in[i]) CeedMi355Free(d->e_in[i]);
