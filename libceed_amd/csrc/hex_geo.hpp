@@ -21,6 +21,8 @@ namespace mi355 {
 
 // doubles per element: the vectors c_100, c_010, c_001, c_110, c_101, c_011, c_111, and 3 unused (192 bytes)
 constexpr int kGeoStride = 24;
+// and in LDS, where a multiple of 8 would put the elements of a wavefront on the same banks
+constexpr int kGeoLds = 26;
 
 // Jacobian columns on one column of quadrature points: d/dxi = p0 + zeta q0,
 // d/deta = p1 + zeta q1, d/dzeta = c

@@ -100,16 +100,31 @@ struct LineSlabs {
 // FP64 p=6 0.648-0.650 vs 0.689-0.691, scalar FP64 p=6 unchanged within run
 // to run noise.  At Q = 7 (FP64) planes of 58 model 10% fewer conflict
 // cycles: 3-component p=5 0.783-0.784 vs 0.794-0.796 ms, scalar p=5
-// unchanged; the same search gave no measurable gain at Q = 4 or 10.
+// unchanged.  With the factors recomputed LDS weighs more (conflicts 38% of
+// the cycles at p=1, 14% at p=4), and planes of 18 at Q = 4 and 5 entries
+// between elements at Q = 3, which model 44% and 19% fewer passes, measure
+// 0.245 vs 0.256 (p=2) and 0.770 vs 0.790 ms (p=1, 4M DoFs, two interleaved
+// runs); the same search changed nothing at Q = 2, 5 and 10 and cost 2% at
+// Q = 6 (planes of 37 and 39).
 __host__ __device__ constexpr int line_row_stride(int Q, int sb) { return sb == 8 && Q == 8 ? 9 : Q; }
-__host__ __device__ constexpr int line_plane_stride(int Q, int sb) { return Q == 8 ? (sb == 8 ? 72 : 73) : Q == 7 && sb == 8 ? 58 : Q * Q; }
+__host__ __device__ constexpr int line_plane_stride(int Q, int sb) {
+  if (sb == 8) return Q == 4 ? 18 : Q == 7 ? 58 : Q == 8 ? 72 : Q * Q;
+  return Q == 8 ? 73 : Q * Q;
+}
+// entries between the slabs of one element and the next
+__host__ __device__ constexpr int line_elem_pad(int Q, int sb) { return sb == 8 && Q == 3 ? 5 : 0; }
 __host__ __device__ constexpr int line_slab_entries(int Q, int sb) { return Q * line_plane_stride(Q, sb); }
+
+// Entries from one element's slabs to the next one's in the line kernel
+__host__ __device__ constexpr int line_elem_entries(int Q, int ncomp, int qf, int sb, bool geo) {
+  return line_kernel_slabs(Q, ncomp, qf, sb, geo) * line_slab_entries(Q, sb) + line_elem_pad(Q, sb);
+}
 
 // LDS bytes of a workgroup of epb elements: the slabs and, where the factors
 // are recomputed, the elements' trilinear maps behind them
 __host__ __device__ constexpr size_t line_lds_bytes(int Q, int ncomp, int qf, int sb, bool geo, int epb) {
-  const size_t slabs = (size_t)sb * epb * line_kernel_slabs(Q, ncomp, qf, sb, geo) * line_slab_entries(Q, sb);
-  return geo ? ((slabs + 15) & ~(size_t)15) + sizeof(double) * kGeoStride * (size_t)epb : slabs;
+  const size_t slabs = (size_t)sb * epb * line_elem_entries(Q, ncomp, qf, sb, geo);
+  return geo ? ((slabs + 15) & ~(size_t)15) + sizeof(double) * kGeoLds * (size_t)epb : slabs;
 }
 
 // Where the factors are recomputed (kGeo): once per element into the registers
@@ -494,7 +509,7 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo
   constexpr int NT = Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QC = QfTraits<QF>::kComps;
   constexpr int SR = line_row_stride(Q, sizeof(T)), SP = line_plane_stride(Q, sizeof(T)), SLAB = Q * SP;
   static_assert(SR >= Q && SP >= Q * SR, "slab rows and planes must not overlap");
-  constexpr int NS = line_kernel_slabs(Q, NCOMP, QF, sizeof(T), kGeo);
+  constexpr int ES = line_elem_entries(Q, NCOMP, QF, sizeof(T), kGeo);
   constexpr bool kDzLds = line_dz_in_lds(Q, NCOMP, QF, sizeof(T), kGeo);
   constexpr bool kOnce = line_geo_once(Q, NCOMP, sizeof(T));
   // from Q = 7 one phase's matrix entries no longer fit the SGPRs: load them
@@ -505,12 +520,12 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo
 
   const int epb = blockDim.x / NT;
   const int le = threadIdx.x / NT, t = threadIdx.x - le * NT;
-  T        *X = reinterpret_cast<T *>(lds_raw) + (size_t)le * NS * SLAB;
+  T        *X = reinterpret_cast<T *>(lds_raw) + le * ES;
   T        *Y = X + SLAB;  // diffusion only
   T        *Z = Y + SLAB;  // kDzLds only
   auto      at = [](int z, int y, int x) { return z * SP + y * SR + x; };
   // kGeo: the element's trilinear map behind the slabs
-  double *sgeo = reinterpret_cast<double *>(lds_raw + (((size_t)epb * NS * SLAB * sizeof(T) + 15) & ~(size_t)15)) + le * kGeoStride;
+  double *sgeo = reinterpret_cast<double *>(lds_raw + (((size_t)epb * ES * sizeof(T) + 15) & ~(size_t)15)) + le * kGeoLds;
 
   // the workgroup's elements: epb consecutive packed elements, or (kSeg)
   // segment elem_begin + chunk, whose consecutive elements share x-faces
@@ -889,7 +904,7 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo
         bool write = true;
         if constexpr (kSeg) {
           if (cx == P - 1 && le + 1 < slen) {
-            const T *Sn = X + NS * SLAB;
+            const T *Sn = X + ES;
 #pragma unroll
             for (int z = 0; z < P; z++) s[z] += Sn[at(z, cy, 0)];
           }
