@@ -25,10 +25,18 @@
 //   k_dot:       p . Ap                                        (reads 2n)
 //   k_update_r:  r -= alpha Ap [z = D^-1 r], partial r.r [r.z]  (reads 2n [3n], writes n [2n])
 //   k_update_px: x += alpha p, p = z + beta p  (z = r unpreconditioned)  (reads 3n, writes 2n)
-// plus single-block reductions that finish the dot products and form
-// alpha and beta.
+// Where the plan's apply ends in the transpose map's gather, the gather forms
+// p . Ap as it writes Ap and k_dot is not run.  alpha and beta are formed by
+// the blocks of the kernels that use them, each from all partial sums in the
+// same order (8-16 KB out of L2), rather than by a one-block kernel in between
+// whose 4.5 us, twice an iteration, were as long as a vector update at a
+// million DoFs.  MI355X, FP64, p=3, 1.2M DoFs: 50 iterations in 3.54 ms before
+// and 3.40 after (apply 2.0, gather 0.63, updates 0.82); preconditioned at 30k DoFs 24 and 21 us
+// an iteration.
 #include <math.h>
 #include <string.h>
+
+#include <algorithm>
 
 #include "hex_plan.hpp"
 #include "mi355_common.h"
@@ -39,7 +47,9 @@ constexpr int kThreads = 256;
 constexpr int kBlocks  = 1024;  // fixed reduction grid: bitwise-deterministic sums
 
 // device scalar slots: kRho = r . z (= r . r unpreconditioned) drives alpha and beta, kRR = r . r the stopping test
-enum { kRR = 0, kPAP, kAlpha, kBeta, kRRTrue, kBB, kRho, kNumScal = 8 };
+// (k_update_px, whose blocks all read kRho, leaves the next one in kRhoNext; the
+// kernel that forms p . Ap takes it over)
+enum { kRR = 0, kPAP, kAlpha, kBeta, kRRTrue, kBB, kRho, kRhoNext, kNumScal = 8 };
 
 __device__ double block_sum(double v) {
   __shared__ double s[kThreads];
@@ -52,44 +62,79 @@ __device__ double block_sum(double v) {
   return s[0];
 }
 
+// the sum of nb partial sums, in one order whatever block forms it, for every
+// thread; a thread's loads are all in flight together
+__device__ double all_partials(int nb, const double *__restrict__ partial) {
+  constexpr int kMost = mi355::kDotBlocks / kThreads;
+  static_assert(kBlocks <= mi355::kDotBlocks, "partial sums of a dot product");
+  double v[kMost], acc = 0;
+#pragma unroll
+  for (int j = 0; j < kMost; j++) v[j] = j * kThreads < nb && j * kThreads + (int)threadIdx.x < nb ? partial[j * kThreads + threadIdx.x] : 0.0;
+#pragma unroll
+  for (int j = 0; j < kMost; j++) acc += v[j];
+  const double s = block_sum(acc);
+  __syncthreads();  // block_sum's shared buffer is used again
+  return s;
+}
+
 template <typename A, typename B>
-__global__ void __launch_bounds__(kThreads) k_dot(int64_t n, const A *__restrict__ a, const B *__restrict__ b, double *__restrict__ partial) {
+__global__ void __launch_bounds__(kThreads) k_dot(int64_t n, const A *__restrict__ a, const B *__restrict__ b, double *__restrict__ partial,
+                                                  double *__restrict__ scal) {
+  if (scal && blockIdx.x == 0 && threadIdx.x == 0) scal[kRho] = scal[kRhoNext];
   double acc = 0;
   for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) acc += (double)a[i] * (double)b[i];
   const double s = block_sum(acc);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
-// Finish a dot product into scal[slot]; mode 1: alpha = Rho / PAP; mode 2: beta = new / Rho, Rho = new
-// (and scal[slot] = new, slot kRR when unpreconditioned, kRho otherwise).
-__global__ void __launch_bounds__(kThreads) k_finish(int nb, const double *__restrict__ partial, double *__restrict__ scal, int slot, int mode) {
-  double acc = 0;
-  for (int i = threadIdx.x; i < nb; i += kThreads) acc += partial[i];
-  const double s = block_sum(acc);
+// Finish a dot product into scal[slot] (kRho: and kRhoNext)
+__global__ void __launch_bounds__(kThreads) k_finish(int nb, const double *__restrict__ partial, double *__restrict__ scal, int slot) {
+  const double s = all_partials(nb, partial);
   if (threadIdx.x == 0) {
-    if (mode == 1) {
-      scal[kPAP]   = s;
-      scal[kAlpha] = s != 0.0 ? scal[kRho] / s : 0.0;
-    } else if (mode == 2) {
-      scal[kBeta] = scal[kRho] != 0.0 ? s / scal[kRho] : 0.0;
-      scal[kRho]  = s;
-      scal[slot]  = s;
-    } else {
-      scal[slot] = s;
-    }
+    scal[slot] = s;
+    if (slot == kRho) scal[kRhoNext] = s;
   }
+}
+
+// alpha = rho / p . Ap from the partial sums of p . Ap
+__device__ double form_alpha(int nb, const double *__restrict__ pap_partial, double *__restrict__ scal) {
+  const double pap = all_partials(nb, pap_partial), alpha = pap != 0.0 ? scal[kRho] / pap : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x == 0) scal[kPAP] = pap, scal[kAlpha] = alpha;
+  return alpha;
+}
+
+// The vector updates take kBatch entries of a thread's stride at a time, and
+// load the first of them before alpha or beta is formed: the partial sums and
+// the vectors come in together.
+constexpr int kBatch = 4;
+template <typename T>
+__device__ __forceinline__ void load_batch(int64_t i, int64_t step, int64_t n, const T *__restrict__ x, T (&v)[kBatch]) {
+#pragma unroll
+  for (int j = 0; j < kBatch; j++) v[j] = i + j * step < n ? x[i + j * step] : T(0);
 }
 
 // r -= alpha Ap, and the partial sums of r . r
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_update_r(int64_t n, const double *__restrict__ scal, T *__restrict__ r, const T *__restrict__ Ap,
-                                                       double *__restrict__ partial) {
-  const T alpha = (T)scal[kAlpha];
+__global__ void __launch_bounds__(kThreads) k_update_r(int64_t n, int pap_nb, const double *__restrict__ pap_partial, double *__restrict__ scal,
+                                                       T *__restrict__ r, const T *__restrict__ Ap, double *__restrict__ partial) {
+  const int64_t step = (int64_t)gridDim.x * kThreads;
+  int64_t       i    = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  T             rv[kBatch], av[kBatch];
+  load_batch(i, step, n, r, rv);
+  load_batch(i, step, n, Ap, av);
+  const T alpha = (T)form_alpha(pap_nb, pap_partial, scal);
   double  acc   = 0;
-  for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
-    const T ri = r[i] - alpha * Ap[i];
-    r[i]       = ri;
-    acc += (double)ri * (double)ri;
+  while (i < n) {
+#pragma unroll
+    for (int j = 0; j < kBatch; j++) {
+      if (i + j * step >= n) break;
+      const T ri      = rv[j] - alpha * av[j];
+      r[i + j * step] = ri;
+      acc += (double)ri * (double)ri;
+    }
+    i += kBatch * step;
+    load_batch(i, step, n, r, rv);
+    load_batch(i, step, n, Ap, av);
   }
   const double s = block_sum(acc);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
@@ -97,10 +142,11 @@ __global__ void __launch_bounds__(kThreads) k_update_r(int64_t n, const double *
 
 // r -= alpha Ap, z = invd r, and the partial sums of r . r and r . z
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_update_r_jacobi(int64_t n, const double *__restrict__ scal, T *__restrict__ r, const T *__restrict__ Ap,
+__global__ void __launch_bounds__(kThreads) k_update_r_jacobi(int64_t n, int pap_nb, const double *__restrict__ pap_partial,
+                                                              double *__restrict__ scal, T *__restrict__ r, const T *__restrict__ Ap,
                                                               const T *__restrict__ invd, T *__restrict__ z, double *__restrict__ partial_rr,
                                                               double *__restrict__ partial_rz) {
-  const T alpha = (T)scal[kAlpha];
+  const T alpha = (T)form_alpha(pap_nb, pap_partial, scal);
   double  rr = 0, rz = 0;
   for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
     const T ri = r[i] - alpha * Ap[i];
@@ -129,15 +175,36 @@ __global__ void __launch_bounds__(kThreads) k_invert(int64_t n, const double *__
   for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) invd[i] = (T)(1.0 / diag[i]);
 }
 
-// x += alpha p;  p = z + beta p  (z = r unpreconditioned)
+// x += alpha p;  p = z + beta p  (z = r unpreconditioned), beta = rho_next / rho
+// from the partial sums of rho_next = r . z; rr_partial: those of r . r where
+// they are others (preconditioned)
 template <typename T>
-__global__ void __launch_bounds__(kThreads) k_update_px(int64_t n, const double *__restrict__ scal, T *__restrict__ x, T *__restrict__ p,
-                                                        const T *__restrict__ r) {
-  const T alpha = (T)scal[kAlpha], beta = (T)scal[kBeta];
-  for (int64_t i = blockIdx.x * (int64_t)kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
-    const T pi = p[i];
-    x[i] += alpha * pi;
-    p[i] = r[i] + beta * pi;
+__global__ void __launch_bounds__(kThreads) k_update_px(int64_t n, int nb, const double *__restrict__ rho_partial,
+                                                        const double *__restrict__ rr_partial, double *__restrict__ scal, T *__restrict__ x,
+                                                        T *__restrict__ p, const T *__restrict__ r) {
+  const int64_t step = (int64_t)gridDim.x * kThreads;
+  int64_t       i    = blockIdx.x * (int64_t)kThreads + threadIdx.x;
+  T             xv[kBatch], pv[kBatch], rv[kBatch];
+  load_batch(i, step, n, x, xv);
+  load_batch(i, step, n, p, pv);
+  load_batch(i, step, n, r, rv);
+  const double rho_next = all_partials(nb, rho_partial), rho = scal[kRho], b = rho != 0.0 ? rho_next / rho : 0.0;
+  if (blockIdx.x == 0) {
+    const double rr = rr_partial ? all_partials(nb, rr_partial) : rho_next;
+    if (threadIdx.x == 0) scal[kBeta] = b, scal[kRhoNext] = rho_next, scal[kRR] = rr;
+  }
+  const T alpha = (T)scal[kAlpha], beta = (T)b;
+  while (i < n) {
+#pragma unroll
+    for (int j = 0; j < kBatch; j++) {
+      if (i + j * step >= n) break;
+      x[i + j * step] = xv[j] + alpha * pv[j];
+      p[i + j * step] = rv[j] + beta * pv[j];
+    }
+    i += kBatch * step;
+    load_batch(i, step, n, x, xv);
+    load_batch(i, step, n, p, pv);
+    load_batch(i, step, n, r, rv);
   }
 }
 
@@ -185,7 +252,7 @@ struct CeedMi355CG_private {
   int64_t           n     = 0;
   hipStream_t       stream = nullptr;
   hipEvent_t        ev     = nullptr;
-  double           *scal = nullptr, *h_scal = nullptr, *partial = nullptr, *partial2 = nullptr;
+  double           *scal = nullptr, *h_scal = nullptr, *partial = nullptr, *partial2 = nullptr, *pap_partial = nullptr;
   void             *r = nullptr, *p = nullptr, *Ap = nullptr, *dx = nullptr;  // inner scalar type
   bool              jacobi = false;
   void             *invd = nullptr, *z = nullptr;  // Jacobi: 1 / diag and z = invd r, inner scalar type
@@ -206,19 +273,20 @@ int iteration(CeedMi355CG cg, T *x) {
   hipStream_t s  = cg->stream;
   const int   nb = nblocks(cg->n);
   T *r = (T *)cg->r, *p = (T *)cg->p, *Ap = (T *)cg->Ap, *z = cg->jacobi ? (T *)cg->z : r;
-  int ierr = CeedMi355OperatorApply(cg->op, p, Ap, s);
+  int pap_nb = 0;  // partial sums of p . Ap the apply has left, if its last kernel forms them
+  int ierr   = mi355::apply_dot(cg->op, p, Ap, cg->pap_partial, cg->scal + kRho, cg->scal + kRhoNext, &pap_nb, s);
   if (ierr) return ierr;
-  k_dot<T, T><<<nb, kThreads, 0, s>>>(cg->n, p, Ap, cg->partial);
-  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kPAP, 1);
-  if (cg->jacobi) {
-    k_update_r_jacobi<T><<<nb, kThreads, 0, s>>>(cg->n, cg->scal, r, Ap, (const T *)cg->invd, z, cg->partial, cg->partial2);
-    k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial2, cg->scal, kRho, 2);
-    k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kRR, 0);
-  } else {
-    k_update_r<T><<<nb, kThreads, 0, s>>>(cg->n, cg->scal, r, Ap, cg->partial);
-    k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kRR, 2);
+  if (!pap_nb) {
+    k_dot<T, T><<<nb, kThreads, 0, s>>>(cg->n, p, Ap, cg->pap_partial, cg->scal);
+    pap_nb = nb;
   }
-  k_update_px<T><<<nb, kThreads, 0, s>>>(cg->n, cg->scal, x, p, z);
+  if (cg->jacobi) {
+    k_update_r_jacobi<T><<<nb, kThreads, 0, s>>>(cg->n, pap_nb, cg->pap_partial, cg->scal, r, Ap, (const T *)cg->invd, z, cg->partial, cg->partial2);
+    k_update_px<T><<<nb, kThreads, 0, s>>>(cg->n, nb, cg->partial2, cg->partial, cg->scal, x, p, z);
+  } else {
+    k_update_r<T><<<nb, kThreads, 0, s>>>(cg->n, pap_nb, cg->pap_partial, cg->scal, r, Ap, cg->partial);
+    k_update_px<T><<<nb, kThreads, 0, s>>>(cg->n, nb, cg->partial, nullptr, cg->scal, x, p, z);
+  }
   MI355_LAUNCH_CHECK();
   return CEED_MI355_SUCCESS;
 }
@@ -230,7 +298,7 @@ int true_residual(CeedMi355CG cg, const double *b, const double *x, double *r64,
   int         err = CeedMi355OperatorApply(cg->mixed ? cg->op64 : cg->op, x, Ap64, s);
   if (err) return err;
   k_residual<<<nb, kThreads, 0, s>>>(cg->n, b, Ap64, r64, cg->partial);
-  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kRRTrue, 0);
+  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kRRTrue);
   MI355_LAUNCH_CHECK();
   return CEED_MI355_SUCCESS;
 }
@@ -247,10 +315,10 @@ int start_search(CeedMi355CG cg, bool set_p) {
     z = (const T *)cg->z;
   }
   if (set_p) k_copy2<T, T><<<nb, kThreads, 0, s>>>(cg->n, z, (T *)cg->p, nullptr);
-  k_dot<T, T><<<nb, kThreads, 0, s>>>(cg->n, r, r, cg->partial);
-  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kRR, 0);
-  if (cg->jacobi) k_dot<T, T><<<nb, kThreads, 0, s>>>(cg->n, r, z, cg->partial);
-  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kRho, 0);
+  k_dot<T, T><<<nb, kThreads, 0, s>>>(cg->n, r, r, cg->partial, nullptr);
+  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kRR);
+  if (cg->jacobi) k_dot<T, T><<<nb, kThreads, 0, s>>>(cg->n, r, z, cg->partial, nullptr);
+  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kRho);
   MI355_LAUNCH_CHECK();
   return CEED_MI355_SUCCESS;
 }
@@ -324,7 +392,8 @@ extern "C" int CeedMi355CGCreate(CeedMi355Operator op, CeedMi355Operator op64, C
   bool         ok = hipStreamCreateWithFlags(&cg->stream, hipStreamNonBlocking) == hipSuccess && hipEventCreateWithFlags(&cg->ev, hipEventDisableTiming) == hipSuccess &&
             hipMalloc(&cg->scal, sizeof(double) * kNumScal) == hipSuccess &&
             hipHostMalloc(&cg->h_scal, sizeof(double) * kNumScal, hipHostMallocDefault) == hipSuccess &&
-            hipMalloc(&cg->partial, sizeof(double) * kBlocks) == hipSuccess && hipMalloc(&cg->partial2, sizeof(double) * kBlocks) == hipSuccess &&
+            hipMalloc(&cg->partial, sizeof(double) * kBlocks) == hipSuccess &&
+            hipMalloc(&cg->pap_partial, sizeof(double) * std::max<int>(kBlocks, mi355::kDotBlocks)) == hipSuccess && hipMalloc(&cg->partial2, sizeof(double) * kBlocks) == hipSuccess &&
             hipMalloc(&cg->r, s * n) == hipSuccess &&
             hipMalloc(&cg->p, s * n) == hipSuccess && hipMalloc(&cg->Ap, s * n) == hipSuccess;
   if (ok && mixed)
@@ -375,8 +444,8 @@ extern "C" int CeedMi355CGSolve(CeedMi355CG cg, const double *b, double *x, int3
   MI355_HIP(hipStreamWaitEvent(s, cg->ev, 0));
 
   k_fill<double><<<1, kThreads, 0, s>>>(kNumScal, 0.0, cg->scal);
-  k_dot<double, double><<<nb, kThreads, 0, s>>>(cg->n, b, b, cg->partial);
-  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kBB, 0);
+  k_dot<double, double><<<nb, kThreads, 0, s>>>(cg->n, b, b, cg->partial, nullptr);
+  k_finish<<<1, kThreads, 0, s>>>(nb, cg->partial, cg->scal, kBB);
   MI355_LAUNCH_CHECK();
   int err;
   if (cg->mixed) {  // r64 = b - A x, r = (float) r64, p = [D^-1] r, dx = 0
@@ -428,6 +497,7 @@ extern "C" int CeedMi355CGDestroy(CeedMi355CG *cg) {
   (void)hipHostFree(c->h_scal);
   (void)hipFree(c->partial);
   (void)hipFree(c->partial2);
+  (void)hipFree(c->pap_partial);
   (void)hipFree(c->invd);
   (void)hipFree(c->z);
   (void)hipFree(c->r);

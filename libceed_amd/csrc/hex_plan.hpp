@@ -21,6 +21,11 @@ using GeoLinesFn = void (*)(const CeedMi355Operator_private *op, int64_t b, int6
 using ApplyFn = int (*)(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s);
 // v (=|+=) E^T evec by the plan's transpose map (operator_hex.hip)
 int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, hipStream_t s);
+// v = A u and, where the apply ends in transpose_gather, the partial sums of
+// u . v into partial (*nb of them, at most kDotBlocks), with *to = *from done
+// on the way; *nb = 0 where it does not (nothing but the apply is done then).
+constexpr int kDotBlocks = 2048;
+int           apply_dot(CeedMi355Operator_private *op, const void *u, void *v, double *partial, double *to, const double *from, int *nb, hipStream_t s);
 // The split mode's second step: Apply (overwrite) writes the shared entries of
 // v; ApplyAdd adds the scratch target and the shared sums into v.
 int split_finish(const CeedMi355Operator_private *op, void *v, int overwrite, hipStream_t s);

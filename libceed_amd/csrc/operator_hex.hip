@@ -484,6 +484,40 @@ __global__ void __launch_bounds__(256) transpose_gather_kernel(int64_t l_size, c
   }
 }
 
+// The gather with the partial sums of u . v, in a fixed order: the blocks'
+// strides, then a tree over the block (CeedMi355CG: p . Ap while Ap is in
+// registers, instead of a kernel that reads both vectors again)
+template <typename T>
+__global__ void __launch_bounds__(256) transpose_gather_dot_kernel(int64_t l_size, const int32_t *__restrict__ row, const T *__restrict__ evec,
+                                                                   const T *__restrict__ u, T *__restrict__ v, double *__restrict__ partial,
+                                                                   double *__restrict__ to, const double *__restrict__ from) {
+  __shared__ double sum[256];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *to = *from;
+  double dot = 0;
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < l_size; t += (int64_t)gridDim.x * blockDim.x) {
+    T acc = 0;
+    for (int32_t m = row[t]; m < row[t + 1]; m++) acc += evec[m];
+    v[t] = acc;
+    dot += (double)u[t] * (double)acc;
+  }
+  sum[threadIdx.x] = dot;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (threadIdx.x < w) sum[threadIdx.x] += sum[threadIdx.x + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) partial[blockIdx.x] = sum[0];
+}
+
+// What apply_dot asks of the transpose_gather its apply ends in, on its own thread
+struct GatherDot {
+  const void   *u = nullptr;
+  double       *partial = nullptr, *to = nullptr;
+  const double *from = nullptr;
+  int           nb   = 0;
+};
+thread_local GatherDot *t_gather_dot = nullptr;
+
 // The same over chunks of L entries, one block per chunk; chunks of inactive
 // systems (batched solvers) are left out
 template <typename T>
@@ -536,6 +570,18 @@ int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite
     else
       transpose_gather_chunks_kernel<float><<<nb, 256, 0, s>>>(op->d_gather_chunk_begin, op->d_gather_chunk_sys, op->d_sys_active, op->d_trow,
                                                                (const float *)op->d_evec, (float *)v, overwrite);
+    MI355_LAUNCH_CHECK();
+    return CEED_MI355_SUCCESS;
+  }
+  if (t_gather_dot && overwrite) {
+    GatherDot &d = *t_gather_dot;
+    d.nb         = mi355_blocks(op->l_size, 256, kDotBlocks);
+    if (op->scalar_type == CEED_MI355_FP64)
+      transpose_gather_dot_kernel<double><<<d.nb, 256, 0, s>>>(op->l_size, op->d_trow, (const double *)op->d_evec, (const double *)d.u, (double *)v,
+                                                               d.partial, d.to, d.from);
+    else
+      transpose_gather_dot_kernel<float><<<d.nb, 256, 0, s>>>(op->l_size, op->d_trow, (const float *)op->d_evec, (const float *)d.u, (float *)v,
+                                                              d.partial, d.to, d.from);
     MI355_LAUNCH_CHECK();
     return CEED_MI355_SUCCESS;
   }
@@ -985,6 +1031,16 @@ extern "C" int CeedMi355OperatorApply(CeedMi355Operator op, const void *u, void 
   }
   if (op->num_elem == 0) return CEED_MI355_SUCCESS;
   return op->apply(op, u, v, 1, s);
+}
+
+int mi355::apply_dot(CeedMi355Operator op, const void *u, void *v, double *partial, double *to, const double *from, int *nb, hipStream_t s) {
+  GatherDot d;
+  d.u = u, d.partial = partial, d.to = to, d.from = from;
+  t_gather_dot   = &d;
+  const int ierr = CeedMi355OperatorApply(op, u, v, s);
+  t_gather_dot   = nullptr;
+  *nb            = d.nb;
+  return ierr;
 }
 
 extern "C" int CeedMi355OperatorSetLaunch(CeedMi355Operator op, int32_t elems_per_block) {
