@@ -213,6 +213,12 @@ int CeedMi355OperatorSetKappa(CeedMi355Operator op, const double *kappa, void *s
  * The transpose apply is the reference's CeedOperatorApply of the same
  * operator (A symmetric; ceed-ref-operator.c:381-470). */
 int CeedMi355OperatorApplyAdjoint(CeedMi355Operator op, const double *u, const double *lambda, double *v, double *dkappa, void *stream);
+/* CeedMi355OperatorSetKappa and then Apply / ApplyAdjoint, in one pass over
+ * kappa where the plan's kernel can take it as it comes (NULL in the adjoint:
+ * the plan's kappa). */
+int CeedMi355OperatorApplyKappa(CeedMi355Operator op, const double *kappa, const void *u, void *v, void *stream);
+int CeedMi355OperatorApplyAdjointKappa(CeedMi355Operator op, const double *kappa, const double *u, const double *lambda, double *v, double *dkappa,
+                                       void *stream);
 /* Diagonal of the plan's operator into the L-vector diag (plan scalar type);
  * add != 0 sums into diag.  Replaces CeedOperatorLinearAssembleDiagonal /
  * AddDiagonal (interface/ceed-preconditioning.c:2395-2480) for this operator. */

@@ -46,6 +46,8 @@ SIGNATURES = {
     "CeedMi355OperatorGetQData": (c_int, [vp, vp, vp]),
     "CeedMi355OperatorSetKappa": (c_int, [vp, vp, vp]),
     "CeedMi355OperatorApplyAdd": (c_int, [vp, vp, vp, vp]),
+    "CeedMi355OperatorApplyKappa": (c_int, [vp, vp, vp, vp, vp]),
+    "CeedMi355OperatorApplyAdjointKappa": (c_int, [vp, vp, vp, vp, vp, vp, vp]),
     "CeedMi355OperatorApplyAdjoint": (c_int, [vp, vp, vp, vp, vp, vp]),
     "CeedMi355OperatorAssembleDiagonal": (c_int, [vp, vp, c_int, vp]),
     "CeedMi355OperatorApply": (c_int, [vp, vp, vp, vp]),

@@ -21,9 +21,8 @@ class KappaDiffusion(torch.autograd.Function):
         if op.qf != ops.QF_DIFFUSION_KAPPA or op.dtype != torch.float64:
             raise ValueError("KappaDiffusion needs an FP64 QF_DIFFUSION_KAPPA operator")
         u, kappa = u.contiguous(), kappa.contiguous()
-        op.set_kappa(kappa)
         v = torch.empty_like(u)
-        op.apply(u, v)
+        op.apply_kappa(kappa, u, v)
         ctx.op = op
         ctx.save_for_backward(u, kappa)
         return v
@@ -32,10 +31,9 @@ class KappaDiffusion(torch.autograd.Function):
     def backward(ctx, lam: torch.Tensor):
         u, kappa = ctx.saved_tensors
         op = ctx.op
-        op.set_kappa(kappa)  # the plan may have been re-used with another kappa since forward
         gu = torch.empty_like(u)
         gk = torch.empty_like(kappa)
-        op.apply_adjoint(u, lam.contiguous(), gu, gk)
+        op.apply_adjoint(u, lam.contiguous(), gu, gk, kappa=kappa)  # the plan may have been re-used with another kappa since forward
         return gu, gk, None
 
 

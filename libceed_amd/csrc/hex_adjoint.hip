@@ -16,6 +16,9 @@
 namespace mi355 {
 namespace {
 
+// Entries from one element's slabs to the next one's in the line kernel
+__host__ __device__ constexpr int adjoint_elem_entries(int Q) { return 4 * line_slab_entries(Q, 8) + line_elem_pad(Q, 8); }
+
 template <int P, int Q>
 __global__ void __launch_bounds__(256) hex_adjoint_kernel(int64_t elem_begin, int64_t elem_end, int scatter, const int32_t *__restrict__ offsets,
                                                           const int32_t *__restrict__ perm, const double *__restrict__ q_data,
@@ -193,24 +196,34 @@ __global__ void __launch_bounds__(256) hex_adjoint_kernel(int64_t elem_begin, in
 }
 
 // The same adjoint in the line thread layout (hex_lines.hpp): x and y
-// contractions by whole 1D lines per thread, z contractions and the pointwise
-// work on the (x, y) columns.  Five slabs per element: grad u's x and y parts
-// stay in two of them while lambda is interpolated and differentiated through
-// the other three.
-template <int P, int Q>
+// contractions by whole 1D lines per thread and in place, z contractions and
+// the pointwise work on the (x, y) columns.  Four slabs per element: grad u's
+// x and y parts stay in two of them while lambda is interpolated and
+// differentiated in the other two.  kGeo: the geometric factors are recomputed
+// from the element's trilinear map.  kappa_src (kGeo only): kappa comes from the
+// caller's array (its element order) and is kept in the plan on the way.
+// MI355X, FP64, us per adjoint with the E^T pass, five slabs and stored factors
+// / four slabs and stored / four and recomputed: p=1 Q=3 512k elements 241 / 247
+// / 188; p=4 Q=5 59k (3.9M DoFs) 167 / 163 / 131; p=6 Q=8 5.8k 85 / 80 / 70;
+// p=8 Q=9 1.7k 79 / 58 / 54.  Bound by the chip at Q <= 6 (123 registers, four
+// waves a SIMD, twice the apply's LDS traffic), by too few workgroups above.
+template <int P, int Q, bool kGeo>
 __global__ void __launch_bounds__(256) hex_adjoint_lines_kernel(int64_t elem_begin, int64_t elem_end, int scatter, const int32_t *__restrict__ offsets,
-                                                                const int32_t *__restrict__ perm, const double *__restrict__ q_data,
+                                                                const int32_t *__restrict__ perm, double *__restrict__ q_data,
                                                                 const double *__restrict__ mats, const double *__restrict__ u,
                                                                 const double *__restrict__ lam, double *__restrict__ v, double *__restrict__ evec,
-                                                                const int32_t *__restrict__ tpos, double *__restrict__ g) {
-  constexpr int  NT = Q * Q, SLAB = Q * Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QC = 7, NS = 5;
+                                                                const int32_t *__restrict__ tpos, double *__restrict__ g,
+                                                                const double *__restrict__ geo, const double *__restrict__ geo_pts,
+                                                                const double *__restrict__ kappa_src) {
+  constexpr int  NT = Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QC = 7;
+  constexpr int  SR = line_row_stride(Q, 8), SP = line_plane_stride(Q, 8), SLAB = Q * SP, ES = adjoint_elem_entries(Q);
   constexpr bool kRowWise = Q >= 7;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   const int epb = blockDim.x / NT;
   const int le = threadIdx.x / NT, t = threadIdx.x - le * NT;
-  double   *S0 = reinterpret_cast<double *>(lds_raw) + (size_t)le * NS * SLAB;
-  double   *S1 = S0 + SLAB, *S2 = S1 + SLAB, *S3 = S2 + SLAB, *S4 = S3 + SLAB;
-  auto      at = [](int z, int y, int x) { return (z * Q + y) * Q + x; };
+  double   *X = reinterpret_cast<double *>(lds_raw) + le * ES, *Y = X + SLAB, *UX = Y + SLAB, *UY = UX + SLAB;
+  double   *sgeo = reinterpret_cast<double *>(lds_raw) + epb * ES + le * kGeoLds;
+  auto      at = [](int z, int y, int x) { return z * SP + y * SR + x; };
 
   const int64_t e    = elem_begin + xcd_chunk(blockIdx.x, gridDim.x) * epb + le;
   const bool    live = le < epb && e < elem_end;
@@ -222,58 +235,72 @@ __global__ void __launch_bounds__(256) hex_adjoint_lines_kernel(int64_t elem_beg
 #pragma unroll
     for (int z = 0; z < P; z++) off[z] = offsets[e * P3 + (z * P + cy) * P + cx];
   }
-  const double *qd = q_data + (live ? e : 0) * (int64_t)QC * Q3 + (cy * Q + cx);
-  double        sq[Q][QC];
+  double       *qd = q_data + (live ? e : 0) * (int64_t)QC * Q3 + (cy * Q + cx);
+  const int64_t ge = live ? (int64_t)perm[e] * Q3 + cy * Q + cx : 0;  // the column in the caller's arrays
+  double        sq[Q][kGeo ? 1 : QC];
+  double        wxy = 0;
+  if constexpr (kGeo) {
+    for (int i = t; i < kGeoStride; i += NT) sgeo[i] = geo[(live ? e : 0) * kGeoStride + i];
+    wxy = geo_pts[Q + cy] * geo_pts[Q + cx];
+    if (kappa_src) {
+      if (live) {
 #pragma unroll
-  for (int qz = 0; qz < Q; qz++)
+        for (int qz = 0; qz < Q; qz++) sq[qz][0] = __builtin_nontemporal_load(kappa_src + ge + qz * Q * Q);
+      }
+    } else {
 #pragma unroll
-    for (int k = 0; k < QC; k++) sq[qz][k] = __builtin_nontemporal_load(&qd[k * Q3 + qz * Q * Q]);
+      for (int qz = 0; qz < Q; qz++) sq[qz][0] = __builtin_nontemporal_load(qd + 6 * Q3 + qz * Q * Q);
+    }
+  } else {
+#pragma unroll
+    for (int qz = 0; qz < Q; qz++)
+#pragma unroll
+      for (int k = 0; k < QC; k++) sq[qz][k] = __builtin_nontemporal_load(&qd[k * Q3 + qz * Q * Q]);
+  }
 
   // reference-space gradient of src at the quadrature points: x part into SX,
-  // y part into SY, z part in dz (this thread's column); Sa and Sb are
-  // scratch (SY may be Sa: the last phase reads only Sb)
-  auto gradient = [&](const double *__restrict__ src, double *SX, double *SY, double *Sa, double *Sb, double(&dz)[Q]) {
+  // y part into SY (through which the values pass), z part in dz
+  auto gradient = [&](const double *__restrict__ src, double *SY, double *SX, double(&dz)[Q]) {
     if (node) {
 #pragma unroll
-      for (int z = 0; z < P; z++) Sa[at(z, cy, cx)] = src[off[z] >> 1];
+      for (int z = 0; z < P; z++) SY[at(z, cy, cx)] = src[off[z] >> 1];
     }
     __syncthreads();
     if (xline) {  // B_x on the x-lines of nodes
       const auto gB = phase_ptr(mats);
       double     in[P];
 #pragma unroll
-      for (int x = 0; x < P; x++) in[x] = Sa[at(nz, ny, x)];
+      for (int x = 0; x < P; x++) in[x] = SY[at(nz, ny, x)];
 #pragma unroll
       for (int qx = 0; qx < Q; qx++) {
         const auto m = kRowWise ? phase_ptr(mats + qx * P) : gB + qx * P;
         double     s = 0;
 #pragma unroll
         for (int b = 0; b < P; b++) s += m[b] * in[b];
-        Sb[at(nz, ny, qx)] = s;
+        SY[at(nz, ny, qx)] = s;
       }
     }
     __syncthreads();
     if (t < Q * P) {  // B_y on the y-lines (qx, z), z < P
       const auto gB = phase_ptr(mats);
-      const int  qx = t % Q, z = t / Q;
       double     in[P];
 #pragma unroll
-      for (int b = 0; b < P; b++) in[b] = Sb[at(z, b, qx)];
+      for (int b = 0; b < P; b++) in[b] = SY[at(cy, b, cx)];
 #pragma unroll
       for (int qy = 0; qy < Q; qy++) {
         const auto m = kRowWise ? phase_ptr(mats + qy * P) : gB + qy * P;
         double     s = 0;
 #pragma unroll
         for (int b = 0; b < P; b++) s += m[b] * in[b];
-        Sa[at(z, qy, qx)] = s;
+        SY[at(cy, qy, cx)] = s;
       }
     }
     __syncthreads();
-    {  // B_z and D_z on the column; the values go to Sb for the x/y derivatives
+    {  // B_z and D_z on the column; the values go back for the x/y derivatives
       const auto gB = phase_ptr(mats);
       double     col[P], xq[Q];
 #pragma unroll
-      for (int b = 0; b < P; b++) col[b] = Sa[at(b, cy, cx)];
+      for (int b = 0; b < P; b++) col[b] = SY[at(b, cy, cx)];
 #pragma unroll
       for (int qz = 0; qz < Q; qz++) {
         const auto m = kRowWise ? phase_ptr(mats + qz * P) : gB + qz * P;
@@ -289,138 +316,143 @@ __global__ void __launch_bounds__(256) hex_adjoint_lines_kernel(int64_t elem_beg
         double     s = 0;
 #pragma unroll
         for (int c = 0; c < Q; c++) s += m[c] * xq[c];
-        dz[qz]              = s;
-        Sb[at(qz, cy, cx)] = xq[qz];
+        dz[qz]             = s;
+        SY[at(qz, cy, cx)] = xq[qz];
       }
     }
     __syncthreads();
-    {  // D_x by x-lines (qy = a, qz) into SX, D_y by y-lines (qx = a, qz) into SY
-      const auto gD = phase_ptr(mats + Q * P);
-      const int  a = t % Q, qz = t / Q;
-      double     in[Q];
+    {  // D_x by x-lines (qy = cx, qz = cy) into SX, D_y by y-lines (qx = cx, qz = cy) in place
+      double in[Q];
 #pragma unroll
-      for (int c = 0; c < Q; c++) in[c] = Sb[at(qz, a, c)];
+      for (int c = 0; c < Q; c++) in[c] = SY[at(cy, cx, c)];
+      {
+        const auto gD = phase_ptr(mats + Q * P);
 #pragma unroll
-      for (int qx = 0; qx < Q; qx++) {
-        const auto m = kRowWise ? phase_ptr(mats + Q * P + qx * Q) : gD + qx * Q;
-        double     s = 0;
+        for (int qx = 0; qx < Q; qx++) {
+          const auto m = kRowWise ? phase_ptr(mats + Q * P + qx * Q) : gD + qx * Q;
+          double     s = 0;
 #pragma unroll
-        for (int c = 0; c < Q; c++) s += m[c] * in[c];
-        SX[at(qz, a, qx)] = s;
+          for (int c = 0; c < Q; c++) s += m[c] * in[c];
+          SX[at(cy, cx, qx)] = s;
+        }
       }
 #pragma unroll
-      for (int c = 0; c < Q; c++) in[c] = Sb[at(qz, c, a)];
+      for (int c = 0; c < Q; c++) in[c] = SY[at(cy, c, cx)];
+      __syncthreads();
+      const auto gD = phase_ptr(mats + Q * P);
 #pragma unroll
       for (int qy = 0; qy < Q; qy++) {
         const auto m = kRowWise ? phase_ptr(mats + Q * P + qy * Q) : gD + qy * Q;
         double     s = 0;
 #pragma unroll
         for (int c = 0; c < Q; c++) s += m[c] * in[c];
-        SY[at(qz, qy, a)] = s;
+        SY[at(cy, qy, cx)] = s;
       }
     }
     __syncthreads();
   };
 
   double dzu[Q], dzl[Q];
-  gradient(u, S2, S3, S0, S1, dzu);    // grad u: S2 (x), S3 (y), dzu (z)
-  gradient(lam, S4, S0, S0, S1, dzl);  // grad lambda: S4 (x), S0 (y), dzl (z)
+  gradient(u, UY, UX, dzu);
+  gradient(lam, X, Y, dzl);
   // ---- pointwise: w = S grad lambda, g = w . grad u, then kappa w (in place on the column)
+  GeoColumn  k;
+  const auto gp = phase_ptr(geo_pts);
+  if constexpr (kGeo) {
+    if (kappa_src && live) {  // the plan's kappa from here on
+#pragma unroll
+      for (int qz = 0; qz < Q; qz++) qd[6 * Q3 + qz * Q * Q] = sq[qz][0];
+    }
+    k.load(sgeo, geo_pts[cx], geo_pts[cy]);
+  }
   double vz[Q];
 #pragma unroll
   for (int qz = 0; qz < Q; qz++) {
-    double wx, wy, wz;
-    poisson_regs<double>(sq[qz], S4[at(qz, cy, cx)], S0[at(qz, cy, cx)], dzl[qz], wx, wy, wz);
-    if (live) g[(int64_t)perm[e] * Q3 + qz * Q * Q + cy * Q + cx] = wx * S2[at(qz, cy, cx)] + wy * S3[at(qz, cy, cx)] + wz * dzu[qz];
-    const double k = live ? sq[qz][6] : 0.0;
-    S4[at(qz, cy, cx)] = wx * k;
-    S0[at(qz, cy, cx)] = wy * k;
-    vz[qz]             = wz * k;
+    double s[6], wx, wy, wz;
+    if constexpr (kGeo) {
+      __builtin_amdgcn_sched_barrier(0);  // one point's factors at a time in registers
+      geo_poisson(k, gp[qz], gp[Q + qz] * wxy, s);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 6; i++) s[i] = sq[qz][i];
+    }
+    poisson_regs<double>(s, Y[at(qz, cy, cx)], X[at(qz, cy, cx)], dzl[qz], wx, wy, wz);
+    if (live) g[ge + qz * Q * Q] = wx * UX[at(qz, cy, cx)] + wy * UY[at(qz, cy, cx)] + wz * dzu[qz];
+    const double kq    = sq[qz][kGeo ? 0 : 6];
+    Y[at(qz, cy, cx)] = wx * kq;
+    X[at(qz, cy, cx)] = wy * kq;
+    vz[qz]            = wz * kq;
   }
   __syncthreads();
-  {  // D_x^T by x-lines into S2, D_y^T by y-lines into S3
-    const auto gD = phase_ptr(mats + Q * P);
-    const int  a = t % Q, qz = t / Q;
-    double     in[Q];
+  // ---- the transposes of the line kernel, in place
+  auto transposed = [&](const double *M, const double(&in)[Q], double(&acc)[Q]) {
+    if constexpr (kRowWise) {
+      transposed_line(M, in, acc);
+    } else {
+      const auto m = phase_ptr(M);
 #pragma unroll
-    for (int c = 0; c < Q; c++) in[c] = S4[at(qz, a, c)];
+      for (int i = 0; i < Q; i++)
 #pragma unroll
-    for (int qx = 0; qx < Q; qx++) {
-      const auto m = kRowWise ? phase_ptr(mats + Q * P + qx) : gD + qx;
-      double     s = 0;
-#pragma unroll
-      for (int c = 0; c < Q; c++) s += m[c * Q] * in[c];
-      S2[at(qz, a, qx)] = s;
+        for (int j = 0; j < Q; j++) acc[i] += m[j * Q + i] * in[j];
     }
+  };
+  auto transposed_b = [&](const double(&in)[Q], double(&acc)[P]) {
+    if constexpr (kRowWise) {
+      transposed_line(mats, in, acc);
+    } else {
+      const auto m = phase_ptr(mats);
 #pragma unroll
-    for (int c = 0; c < Q; c++) in[c] = S0[at(qz, c, a)];
+      for (int i = 0; i < P; i++)
 #pragma unroll
-    for (int qy = 0; qy < Q; qy++) {
-      const auto m = kRowWise ? phase_ptr(mats + Q * P + qy) : gD + qy;
-      double     s = 0;
-#pragma unroll
-      for (int c = 0; c < Q; c++) s += m[c * Q] * in[c];
-      S3[at(qz, qy, a)] = s;
+        for (int j = 0; j < Q; j++) acc[i] += m[j * P + i] * in[j];
     }
+  };
+  {
+    double in[Q], out[Q];
+#pragma unroll
+    for (int c = 0; c < Q; c++) in[c] = Y[at(cy, cx, c)], out[c] = 0;
+    transposed(mats + Q * P, in, out);
+#pragma unroll
+    for (int c = 0; c < Q; c++) Y[at(cy, cx, c)] = out[c];
+#pragma unroll
+    for (int c = 0; c < Q; c++) in[c] = X[at(cy, c, cx)], out[c] = 0;
+    transposed(mats + Q * P, in, out);
+#pragma unroll
+    for (int c = 0; c < Q; c++) X[at(cy, c, cx)] = out[c];
   }
   __syncthreads();
-  {  // sum of the three transposes on the column, then B_z^T into S1
-    const auto gDz = phase_ptr(mats + Q * P);
-    double     w[Q];
+  {
+    double w[Q], out[P] = {};
 #pragma unroll
-    for (int qz = 0; qz < Q; qz++) {
-      const auto m = kRowWise ? phase_ptr(mats + Q * P + qz) : gDz + qz;
-      double     s = S2[at(qz, cy, cx)] + S3[at(qz, cy, cx)];
+    for (int qz = 0; qz < Q; qz++) w[qz] = Y[at(qz, cy, cx)] + X[at(qz, cy, cx)];
+    transposed(mats + Q * P, vz, w);
+    transposed_b(w, out);
 #pragma unroll
-      for (int c = 0; c < Q; c++) s += m[c * Q] * vz[c];
-      w[qz] = s;
-    }
-    const auto gBz = phase_ptr(mats);
-#pragma unroll
-    for (int b = 0; b < P; b++) {
-      const auto m = kRowWise ? phase_ptr(mats + b) : gBz + b;
-      double     s = 0;
-#pragma unroll
-      for (int qz = 0; qz < Q; qz++) s += m[qz * P] * w[qz];
-      S1[at(b, cy, cx)] = s;
-    }
+    for (int b = 0; b < P; b++) X[at(b, cy, cx)] = out[b];
   }
   __syncthreads();
-  if (t < Q * P) {  // B_y^T on the y-lines (qx, z), z < P, into S0
-    const auto gB = phase_ptr(mats);
-    const int  qx = t % Q, z = t / Q;
-    double     in[Q];
+  if (t < Q * P) {
+    double in[Q], out[P] = {};
 #pragma unroll
-    for (int a = 0; a < Q; a++) in[a] = S1[at(z, a, qx)];
+    for (int a = 0; a < Q; a++) in[a] = X[at(cy, a, cx)];
+    transposed_b(in, out);
 #pragma unroll
-    for (int y = 0; y < P; y++) {
-      const auto m = kRowWise ? phase_ptr(mats + y) : gB + y;
-      double     s = 0;
-#pragma unroll
-      for (int a = 0; a < Q; a++) s += m[a * P] * in[a];
-      S0[at(z, y, qx)] = s;
-    }
+    for (int y = 0; y < P; y++) X[at(cy, y, cx)] = out[y];
   }
   __syncthreads();
-  if (xline) {  // B_x^T on the x-lines of nodes, into S1
-    const auto gB = phase_ptr(mats);
-    double     in[Q];
+  if (xline) {
+    double in[Q], out[P] = {};
 #pragma unroll
-    for (int a = 0; a < Q; a++) in[a] = S0[at(nz, ny, a)];
+    for (int a = 0; a < Q; a++) in[a] = X[at(nz, ny, a)];
+    transposed_b(in, out);
 #pragma unroll
-    for (int x = 0; x < P; x++) {
-      const auto m = kRowWise ? phase_ptr(mats + x) : gB + x;
-      double     s = 0;
-#pragma unroll
-      for (int a = 0; a < Q; a++) s += m[a * P] * in[a];
-      S1[at(nz, ny, x)] = s;
-    }
+    for (int x = 0; x < P; x++) X[at(nz, ny, x)] = out[x];
   }
   __syncthreads();
   if (node) {  // E^T from the node columns
     double s[P];
 #pragma unroll
-    for (int z = 0; z < P; z++) s[z] = S1[at(z, cy, cx)];
+    for (int z = 0; z < P; z++) s[z] = X[at(z, cy, cx)];
     if (scatter == kScatterEvec) {
 #pragma unroll
       for (int z = 0; z < P; z++) evec[tpos[e * (int64_t)P3 + (z * P + cy) * P + cx]] = s[z];
@@ -448,11 +480,13 @@ __global__ void __launch_bounds__(256) zero_fill(int64_t n, double *__restrict__
 }
 
 template <int P, int Q>
-int launch_adjoint(const CeedMi355Operator_private *op, const double *u, const double *lam, double *v, double *g, hipStream_t s) {
+int launch_adjoint(const CeedMi355Operator_private *op, const double *u, const double *lam, double *v, double *g, const double *kappa_src,
+                   hipStream_t s) {
   const int    nt    = Q * Q;
   const int    epb   = op->epb;
   const bool   lines = op->layout == kLayoutLines;  // (plans in the point layout take the column kernel here)
-  const size_t lds   = sizeof(double) * (size_t)(lines ? epb * 5 * Q * Q * Q : Q * P + Q * Q + epb * 3 * Q * Q * Q);
+  const bool   geo   = lines && op->geo_valid;  // as in CeedMi355OperatorApplyAdjointKappa
+  const size_t lds   = sizeof(double) * (size_t)(lines ? epb * (adjoint_elem_entries(Q) + (geo ? kGeoLds : 0)) : Q * P + Q * Q + epb * 3 * Q * Q * Q);
   const bool   tmap  = op->scatter == 0;
   MI355_CHECK(op->scatter != CEED_MI355_PLAN_SEGMENT, CEED_MI355_ERROR_UNSUPPORTED,
               "the adjoint does not take segment plans (elements of a colour share segment faces)");
@@ -464,9 +498,14 @@ int launch_adjoint(const CeedMi355Operator_private *op, const double *u, const d
     const int     scatter = tmap ? kScatterEvec
                                  : op->scatter == CEED_MI355_PLAN_SPLIT ? kScatterSplit
                                                                         : (op->scatter == CEED_MI355_PLAN_ATOMIC ? kScatterAtomic : kScatterOverwrite);
-    if (lines)
-      hex_adjoint_lines_kernel<P, Q><<<(unsigned)grid, epb * nt, lds, s>>>(b, e, scatter, op->d_offsets, op->d_perm, (const double *)op->d_qdata,
-                                                                          (const double *)op->d_mats, u, lam, v, (double *)op->d_evec, op->d_tpos, g);
+    if (geo)
+      hex_adjoint_lines_kernel<P, Q, true><<<(unsigned)grid, epb * nt, lds, s>>>(b, e, scatter, op->d_offsets, op->d_perm, (double *)op->d_qdata,
+                                                                                (const double *)op->d_mats, u, lam, v, (double *)op->d_evec,
+                                                                                op->d_tpos, g, op->d_geo, op->d_geo_pts, kappa_src);
+    else if (lines)
+      hex_adjoint_lines_kernel<P, Q, false><<<(unsigned)grid, epb * nt, lds, s>>>(b, e, scatter, op->d_offsets, op->d_perm, (double *)op->d_qdata,
+                                                                                 (const double *)op->d_mats, u, lam, v, (double *)op->d_evec,
+                                                                                 op->d_tpos, g, nullptr, nullptr, nullptr);
     else
       hex_adjoint_kernel<P, Q><<<(unsigned)grid, epb * nt, lds, s>>>(b, e, scatter, op->d_offsets, op->d_perm, (const double *)op->d_qdata,
                                                                     (const double *)op->d_mats, u, lam, v, (double *)op->d_evec, op->d_tpos, g);
@@ -477,7 +516,7 @@ int launch_adjoint(const CeedMi355Operator_private *op, const double *u, const d
   return CEED_MI355_SUCCESS;
 }
 
-using AdjointFn = int (*)(const CeedMi355Operator_private *, const double *, const double *, double *, double *, hipStream_t);
+using AdjointFn = int (*)(const CeedMi355Operator_private *, const double *, const double *, double *, double *, const double *, hipStream_t);
 
 AdjointFn pick_adjoint(int P, int Q) {
 #define MI355_ADJ_CASE(PP, QQ) \
@@ -494,6 +533,11 @@ AdjointFn pick_adjoint(int P, int Q) {
 
 extern "C" int CeedMi355OperatorApplyAdjoint(CeedMi355Operator op, const double *u, const double *lambda, double *v, double *dkappa,
                                              void *stream) {
+  return CeedMi355OperatorApplyAdjointKappa(op, nullptr, u, lambda, v, dkappa, stream);
+}
+
+extern "C" int CeedMi355OperatorApplyAdjointKappa(CeedMi355Operator op, const double *kappa, const double *u, const double *lambda, double *v,
+                                                  double *dkappa, void *stream) {
   MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
   MI355_CHECK(op->qf == mi355::kQfDiffusionKappa && op->scalar_type == CEED_MI355_FP64 && op->num_comp == 1, CEED_MI355_ERROR_BACKEND,
               "the adjoint needs an FP64 scalar kappa-diffusion plan");
@@ -501,9 +545,14 @@ extern "C" int CeedMi355OperatorApplyAdjoint(CeedMi355Operator op, const double 
   if (op->num_elem == 0) return CEED_MI355_SUCCESS;
   auto fn = mi355::pick_adjoint(op->P, op->Q);
   MI355_CHECK(fn, CEED_MI355_ERROR_UNSUPPORTED, "no adjoint kernel for P=%d Q=%d", op->P, op->Q);
+  if (kappa && !(op->layout == mi355::kLayoutLines && op->geo_valid)) {  // only that kernel takes kappa from the caller
+    const int err = CeedMi355OperatorSetKappa(op, kappa, stream);
+    if (err) return err;
+    kappa = nullptr;
+  }
   if (!op->covers_all) {  // a fill kernel, not a memset node: safe under graph capture
     mi355::zero_fill<<<mi355_blocks(op->l_size, 256, 4096), 256, 0, s>>>(op->l_size, v);
     MI355_LAUNCH_CHECK();
   }
-  return fn(op, u, lambda, v, dkappa, s);
+  return fn(op, u, lambda, v, dkappa, kappa, s);
 }

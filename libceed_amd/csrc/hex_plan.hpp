@@ -17,7 +17,11 @@ struct CeedMi355Operator_private;
 namespace mi355 {
 
 // the line kernel with recomputed geometric factors over elements [b, e) of a plan (hex_geo_*.hip)
-using GeoLinesFn = void (*)(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, hipStream_t s);
+// (kappa_src: kappa-weighted plans, the caller's kappa, nullptr for the plan's)
+using GeoLinesFn = void (*)(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, const double *kappa_src,
+                            hipStream_t s);
+// Kappa of the apply running on this thread (CeedMi355OperatorApplyKappa), nullptr for the plan's own.
+const double *kappa_of_apply();
 using ApplyFn = int (*)(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s);
 // v (=|+=) E^T evec by the plan's transpose map (operator_hex.hip)
 int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, hipStream_t s);
@@ -186,6 +190,13 @@ struct CeedMi355Operator_private {
 
 namespace mi355 {
 
+// The plan's applies run the line kernel that recomputes the geometric factors
+inline bool plan_recomputes(const CeedMi355Operator_private *op) {
+  return op->layout == kLayoutLines && op->geo_valid && op->geo_lines && op->scatter != CEED_MI355_PLAN_BRICK &&
+         op->scatter != CEED_MI355_PLAN_SEGMENT &&
+         line_lds_bytes(op->Q, op->num_comp, op->qf, op->scalar_bytes, true, op->epb) <= (size_t)kMaxLdsBytes;
+}
+
 template <int P, int Q, int NC, int QF, typename T>
 int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s) {
   const int    nt     = Q * Q;
@@ -210,7 +221,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
         if (e <= b) continue;
         hex_apply_lines_kernel<P, Q, NC, QF, T, true><<<(unsigned)(e - b), epb * nt, lds, s>>>(
             b, e, overwrite ? kScatterOverwrite : kScatterAdd, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats,
-            (const T *)u, (T *)v, nullptr, nullptr, op->d_elem_sys, op->d_sys_active, op->d_seg_start, nullptr, nullptr);
+            (const T *)u, (T *)v, nullptr, nullptr, op->d_elem_sys, op->d_sys_active, op->d_seg_start, nullptr, nullptr, nullptr, nullptr, nullptr);
       }
       MI355_LAUNCH_CHECK();
       return CEED_MI355_SUCCESS;
@@ -225,7 +236,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
     const int err = fill_zero(op, target, s);
     if (err) return err;
   }
-  const bool geo = lines && op->geo_valid && op->geo_lines && line_lds_bytes(Q, NC, QF, sizeof(T), true, epb) <= (size_t)kMaxLdsBytes;
+  const bool geo = plan_recomputes(op);
   for (size_t c = 0; c + 1 < op->color_start.size(); c++) {
     const int64_t b = op->color_start[c], e = op->color_start[c + 1];
     if (e <= b) continue;
@@ -233,11 +244,11 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
     const int     scatter = tmap ? kScatterEvec
                                  : split ? kScatterSplit
                                          : (op->scatter == CEED_MI355_PLAN_ATOMIC ? kScatterAtomic : (overwrite ? kScatterOverwrite : kScatterAdd));
-    if (geo) op->geo_lines(op, b, e, scatter, u, target, s);
+    if (geo) op->geo_lines(op, b, e, scatter, u, target, kappa_of_apply(), s);
     else if (lines)
       hex_apply_lines_kernel<P, Q, NC, QF, T><<<(unsigned)grid, epb * nt, lds, s>>>(
           b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, target, (T *)op->d_evec,
-          op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, nullptr, nullptr);
+          op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
     else if (points) {
       if constexpr (Q * Q * Q <= 256)
         hex_apply_points_kernel<P, Q, NC, QF, T><<<(unsigned)grid, epb * Q * Q * Q, lds, s>>>(
@@ -257,11 +268,12 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
 }
 
 template <int P, int Q, int NC, int QF, typename T>
-void launch_geo_lines(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, hipStream_t s) {
+void launch_geo_lines(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, const double *kappa_src,
+                      hipStream_t s) {
   const int64_t epb = op->epb, grid = (e - b + epb - 1) / epb;
   hex_apply_lines_kernel<P, Q, NC, QF, T, false, true><<<(unsigned)grid, (unsigned)(epb * Q * Q), line_lds_bytes(Q, NC, QF, sizeof(T), true, (int)epb), s>>>(
       b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec,
-      op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, op->d_geo, op->d_geo_pts);
+      op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, op->d_geo, op->d_geo_pts, op->d_perm, kappa_src, (T *)op->d_qdata);
 }
 
 // Dispatch over the instantiated (P, Q) pairs: P = 2..9, Q in {P, P+1}.

@@ -1013,6 +1013,27 @@ extern "C" int CeedMi355OperatorSetKappa(CeedMi355Operator op, const double *kap
   return CEED_MI355_SUCCESS;
 }
 
+namespace {
+thread_local const double *t_kappa = nullptr;  // set for the time of one ApplyKappa
+}  // namespace
+
+const double *mi355::kappa_of_apply() { return t_kappa; }
+
+extern "C" int CeedMi355OperatorApplyKappa(CeedMi355Operator op, const double *kappa, const void *u, void *v, void *stream) {
+  MI355_CHECK(op && op->qf == kQfDiffusionKappa && (kappa || op->num_elem == 0), CEED_MI355_ERROR_BACKEND,
+              "ApplyKappa needs a kappa-diffusion operator and kappa");
+  // the line kernel that recomputes the factors takes kappa from the caller
+  // and keeps it on the way, unless it may skip elements (stopped systems)
+  if (!mi355::plan_recomputes(op) || op->d_elem_sys) {
+    const int err = CeedMi355OperatorSetKappa(op, kappa, stream);
+    return err ? err : CeedMi355OperatorApply(op, u, v, stream);
+  }
+  t_kappa        = kappa;
+  const int ierr = CeedMi355OperatorApply(op, u, v, stream);
+  t_kappa        = nullptr;
+  return ierr;
+}
+
 extern "C" int CeedMi355OperatorApplyAdd(CeedMi355Operator op, const void *u, void *v, void *stream) {
   MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
   if (op->num_elem == 0) return CEED_MI355_SUCCESS;

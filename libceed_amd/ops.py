@@ -204,14 +204,25 @@ class HexOperator:
         self._check(u, v)
         call("CeedMi355OperatorApplyAdd", self._h, _ptr(u), _ptr(v), _stream())
 
-    def apply_adjoint(self, u: torch.Tensor, lam: torch.Tensor, v: torch.Tensor, dkappa: torch.Tensor) -> None:
-        """v = A(kappa)^T lam and dkappa[e, q] = grad(lam) . S grad(u) (QF_DIFFUSION_KAPPA, FP64)."""
+    def apply_kappa(self, kappa: torch.Tensor, u: torch.Tensor, v: torch.Tensor) -> None:
+        """set_kappa(kappa) and v = A(kappa) u, reading kappa once."""
+        self._check(u, v)
+        call("CeedMi355OperatorApplyKappa", self._h, _ptr(self._check_kappa(kappa)), _ptr(u), _ptr(v), _stream())
+
+    def _check_kappa(self, kappa: torch.Tensor) -> torch.Tensor:
+        if kappa.numel() < self.num_elem * self.Q ** 3:
+            raise ValueError("kappa needs num_elem * Q^3 entries")
+        return _device_tensor(kappa, torch.float64)
+
+    def apply_adjoint(self, u: torch.Tensor, lam: torch.Tensor, v: torch.Tensor, dkappa: torch.Tensor, kappa: torch.Tensor | None = None) -> None:
+        """v = A(kappa)^T lam and dkappa[e, q] = grad(lam) . S grad(u) (QF_DIFFUSION_KAPPA, FP64); kappa: set_kappa(kappa) first."""
         self._check(u, v)
         self._check(lam, v)
         _device_tensor(dkappa, torch.float64)
         if dkappa.numel() < self.num_elem * self.Q ** 3:
             raise ValueError("dkappa needs num_elem * Q^3 entries")
-        call("CeedMi355OperatorApplyAdjoint", self._h, _ptr(u), _ptr(lam), _ptr(v), _ptr(dkappa), _stream())
+        kappa = self._check_kappa(kappa) if kappa is not None else None
+        call("CeedMi355OperatorApplyAdjointKappa", self._h, _ptr(kappa), _ptr(u), _ptr(lam), _ptr(v), _ptr(dkappa), _stream())
 
     def assemble_diagonal(self, diag: torch.Tensor, add: bool = False) -> None:
         """diag (=|+=) the diagonal of the operator."""
