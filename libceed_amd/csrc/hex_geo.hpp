@@ -70,13 +70,11 @@ __device__ __forceinline__ double geo_mass(const GeoColumn &k, double zeta, doub
   return w * geo_dot(n, k.c);
 }
 
-// (w / det J) adj(J) adj(J)^T in Voigt order {xx, yy, zz, yz, xz, xy}  (Poisson3DBuild)
-__device__ __forceinline__ void geo_poisson(const GeoColumn &k, double zeta, double w, double (&s)[6]) {
-  double a[3], b[3], A0[3], A1[3], A2[3];
-#pragma unroll
-  for (int d = 0; d < 3; d++) a[d] = __builtin_fma(zeta, k.q0[d], k.p0[d]), b[d] = __builtin_fma(zeta, k.q1[d], k.p1[d]);
-  geo_cross(b, k.c, A0);
-  geo_cross(k.c, a, A1);
+// (w / det J) adj(J) adj(J)^T in Voigt order {xx, yy, zz, yz, xz, xy}  (Poisson3DBuild), J = (a b c)
+__device__ __forceinline__ void geo_poisson(const double (&a)[3], const double (&b)[3], const double (&c)[3], double w, double (&s)[6]) {
+  double A0[3], A1[3], A2[3];
+  geo_cross(b, c, A0);
+  geo_cross(c, a, A1);
   geo_cross(a, b, A2);
   const double qw = w * geo_rcp(geo_dot(a, A0));
   s[0] = qw * geo_dot(A0, A0);
@@ -85,6 +83,12 @@ __device__ __forceinline__ void geo_poisson(const GeoColumn &k, double zeta, dou
   s[3] = qw * geo_dot(A1, A2);
   s[4] = qw * geo_dot(A0, A2);
   s[5] = qw * geo_dot(A0, A1);
+}
+__device__ __forceinline__ void geo_poisson(const GeoColumn &k, double zeta, double w, double (&s)[6]) {
+  double a[3], b[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) a[d] = __builtin_fma(zeta, k.q0[d], k.p0[d]), b[d] = __builtin_fma(zeta, k.q1[d], k.p1[d]);
+  geo_poisson(a, b, k.c, w, s);
 }
 
 }  // namespace mi355

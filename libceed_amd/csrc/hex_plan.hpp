@@ -8,6 +8,7 @@
 
 #include "hex_brick.hpp"
 #include "hex_fused.hpp"
+#include "hex_elements.hpp"
 #include "hex_lines.hpp"
 #include "hex_points.hpp"
 #include "mi355_common.h"
@@ -270,6 +271,14 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
 template <int P, int Q, int NC, int QF, typename T>
 void launch_geo_lines(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, const double *kappa_src,
                       hipStream_t s) {
+  if constexpr (P == 2 && NC == 1 && QF == kQfDiffusion) {
+    if (e - b >= elements_min<Q, T>()) {
+      hex_apply_elements_kernel<P, Q, T><<<(unsigned)((e - b + kElemThreads - 1) / kElemThreads), kElemThreads, 0, s>>>(
+          b, e, scatter, op->d_offsets, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec, op->d_tpos, op->d_elem_sys, op->d_sys_active,
+          op->d_geo, op->d_geo_pts);
+      return;
+    }
+  }
   const int64_t epb = op->epb, grid = (e - b + epb - 1) / epb;
   hex_apply_lines_kernel<P, Q, NC, QF, T, false, true><<<(unsigned)grid, (unsigned)(epb * Q * Q), line_lds_bytes(Q, NC, QF, sizeof(T), true, (int)epb), s>>>(
       b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec,
