@@ -478,6 +478,53 @@ __device__ __forceinline__ void line_element(T *S0, T *S1, T *S2, int t, bool ac
   sync();
 }
 
+// E^T in the apply's own launch, for the node column of one thread: each
+// contribution goes to its slot in the E-vector sorted by L entry, and the
+// last of an entry's contributions to arrive (tcount) forms the entry's sum in
+// the slots' order: the bits of the gather that otherwise follows.  The slots
+// are written and read at agent scope, the release before the count and the
+// acquire after it order them across the XCDs' caches; nobody waits.  The last
+// contribution takes the count back by the number of contributions.
+// Only for launches of at most one workgroup per CU: every wavefront's release
+// writes its XCD's L2 back, and these serialise (MI355X, FP64 diffusion, us per
+// apply, gather launch / this: 54 workgroups, p=2 11.2 / 8.9; 183, p=2 11.0 /
+// 9.7; 247, p=1 11.4 / 9.5; 1229, p=2 12.6 / 26.5); only below P = 5: the
+// nodes of a column follow one another (p=4 11.6 / 11.3, p=7 13.9 / 16.9); only
+// one component: a release each (three, p=2 12.2 / 21.6).
+__host__ __device__ constexpr bool line_takes_last(int P, int ncomp) { return P <= 4 && ncomp == 1; }
+constexpr int64_t kLastWorkgroups = 256;
+template <int P, typename T>
+__device__ __forceinline__ void line_last(bool overwrite, const int (&off)[P], const int32_t *__restrict__ tpos, int tstride, const T (&s)[P],
+                                          T *__restrict__ v, T *__restrict__ evec, const int32_t *__restrict__ trow, int32_t *__restrict__ tcount) {
+  int32_t beg[P], num[P], old[P];
+#pragma unroll
+  for (int z = 0; z < P; z++) {
+    const int32_t n = off[z] >> 1;
+    beg[z]          = trow[n];
+    num[z]          = trow[n + 1] - beg[z];
+    __hip_atomic_store(&evec[tpos[z * tstride]], s[z], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+#pragma unroll
+  for (int z = 0; z < P; z++) old[z] = __hip_atomic_fetch_add(&tcount[off[z] >> 1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+  for (int z = 0; z < P; z++) {
+    if ((old[z] + 1) % num[z]) continue;
+    const int32_t n = off[z] >> 1;
+    T             c[8], acc = overwrite ? T(0) : v[n];
+    (void)__hip_atomic_fetch_sub(&tcount[n], num[z], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int m = 0; m < 8; m++) c[m] = __hip_atomic_load(&evec[beg[z] + (m < num[z] ? m : 0)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+      if (m < num[z]) acc += c[m];
+    }
+    for (int m = 8; m < num[z]; m++) acc += __hip_atomic_load(&evec[beg[z] + m], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v[n] = acc;
+  }
+}
+
 // The line kernel keeps the pipeline written out in its own body rather than
 // calling line_element: the same code through the shared function compiles
 // to a different register allocation here (P=7, Q=8 diffusion: 186 against
@@ -507,7 +554,8 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo
                                                                const int32_t *__restrict__ seg_start, const double *__restrict__ geo,
                                                                const double *__restrict__ geo_pts,
                                                                const int32_t *__restrict__ perm, const double *__restrict__ kappa_src,
-                                                               T *__restrict__ kappa_keep) {
+                                                               T *__restrict__ kappa_keep, const int32_t *__restrict__ trow,
+                                                               int32_t *__restrict__ tcount) {
   constexpr int NT = Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QC = QfTraits<QF>::kComps;
   constexpr int SR = line_row_stride(Q, sizeof(T)), SP = line_plane_stride(Q, sizeof(T)), SLAB = Q * SP;
   static_assert(SR >= Q && SP >= Q * SR, "slab rows and planes must not overlap");
@@ -898,7 +946,9 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo
       T s[P];
 #pragma unroll
       for (int z = 0; z < P; z++) s[z] = X[at(z, cy, cx)];
-      if (!kSeg && scatter == kScatterEvec) {  // tpos gives each contribution's slot in the E-vector sorted by L entry
+      if (line_takes_last(P, NCOMP) && !kSeg && scatter >= kScatterLast) {
+        if constexpr (line_takes_last(P, NCOMP)) line_last<P>(scatter == kScatterLast, off, &tpos[e * P3 + cy * P + cx], P * P, s, v, evec, trow, tcount);
+      } else if (!kSeg && scatter == kScatterEvec) {  // tpos gives each contribution's slot in the E-vector sorted by L entry
         int32_t pos[P];
 #pragma unroll
         for (int z = 0; z < P; z++) pos[z] = tpos[(e * NCOMP + comp) * (int64_t)P3 + (z * P + cy) * P + cx];

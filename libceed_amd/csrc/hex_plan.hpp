@@ -23,6 +23,8 @@ using GeoLinesFn = void (*)(const CeedMi355Operator_private *op, int64_t b, int6
                             hipStream_t s);
 // Kappa of the apply running on this thread (CeedMi355OperatorApplyKappa), nullptr for the plan's own.
 const double *kappa_of_apply();
+// The apply running on this thread wants its transpose_gather to form a dot product (apply_dot).
+bool gather_dot_wanted();
 using ApplyFn = int (*)(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s);
 // v (=|+=) E^T evec by the plan's transpose map (operator_hex.hip)
 int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, hipStream_t s);
@@ -130,6 +132,7 @@ struct CeedMi355Operator_private {
   // L entry t owns the contiguous run d_evec[d_trow[t] .. d_trow[t+1]), in
   // ascending (elem, comp, node) order
   int32_t *d_trow = nullptr, *d_tpos = nullptr;
+  int32_t *d_tcount = nullptr;  // contributions that have arrived at each L entry (plans whose E^T may run in the apply's own launch: line_last)
   void    *d_evec = nullptr;  // E-vector sorted by L entry, plan scalar type
   // multiplicity split (scatter == CEED_MI355_PLAN_SPLIT): L entries reached by
   // at most two contributions are summed by atomic adds onto a zeroed target
@@ -222,7 +225,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
         if (e <= b) continue;
         hex_apply_lines_kernel<P, Q, NC, QF, T, true><<<(unsigned)(e - b), epb * nt, lds, s>>>(
             b, e, overwrite ? kScatterOverwrite : kScatterAdd, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats,
-            (const T *)u, (T *)v, nullptr, nullptr, op->d_elem_sys, op->d_sys_active, op->d_seg_start, nullptr, nullptr, nullptr, nullptr, nullptr);
+            (const T *)u, (T *)v, nullptr, nullptr, op->d_elem_sys, op->d_sys_active, op->d_seg_start, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
       }
       MI355_LAUNCH_CHECK();
       return CEED_MI355_SUCCESS;
@@ -238,18 +241,24 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
     if (err) return err;
   }
   const bool geo = plan_recomputes(op);
+  // kScatterLast: frozen systems' contributions never arrive, a dot product
+  // wants the gather, and where u and v overlap all of u is read first
+  const size_t l_bytes = sizeof(T) * (size_t)op->l_size;
+  const bool   last    = tmap && lines && op->d_tcount && (op->num_elem + epb - 1) / epb <= kLastWorkgroups && !op->d_elem_sys && !gather_dot_wanted() &&
+                    ((const char *)u + l_bytes <= (const char *)v || (const char *)v + l_bytes <= (const char *)u);
   for (size_t c = 0; c + 1 < op->color_start.size(); c++) {
     const int64_t b = op->color_start[c], e = op->color_start[c + 1];
     if (e <= b) continue;
     const int64_t grid    = (e - b + epb - 1) / epb;
-    const int     scatter = tmap ? kScatterEvec
+    const int     scatter = last ? (overwrite ? kScatterLast : kScatterLastAdd)
+                            : tmap ? kScatterEvec
                                  : split ? kScatterSplit
                                          : (op->scatter == CEED_MI355_PLAN_ATOMIC ? kScatterAtomic : (overwrite ? kScatterOverwrite : kScatterAdd));
     if (geo) op->geo_lines(op, b, e, scatter, u, target, kappa_of_apply(), s);
     else if (lines)
       hex_apply_lines_kernel<P, Q, NC, QF, T><<<(unsigned)grid, epb * nt, lds, s>>>(
           b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, target, (T *)op->d_evec,
-          op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr);
+          op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, op->d_trow, op->d_tcount);
     else if (points) {
       if constexpr (Q * Q * Q <= 256)
         hex_apply_points_kernel<P, Q, NC, QF, T><<<(unsigned)grid, epb * Q * Q * Q, lds, s>>>(
@@ -263,7 +272,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
                                                                             op->d_tpos, op->d_elem_sys, op->d_sys_active);
   }
   MI355_LAUNCH_CHECK();
-  if (tmap) return transpose_gather(op, v, overwrite, s);
+  if (tmap && !last) return transpose_gather(op, v, overwrite, s);
   if (split) return split_finish(op, v, overwrite, s);
   return CEED_MI355_SUCCESS;
 }
@@ -272,7 +281,7 @@ template <int P, int Q, int NC, int QF, typename T>
 void launch_geo_lines(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, const double *kappa_src,
                       hipStream_t s) {
   if constexpr (P == 2 && NC == 1 && QF == kQfDiffusion) {
-    if (e - b >= elements_min<Q, T>()) {
+    if (scatter < kScatterLast && e - b >= elements_min<Q, T>()) {
       hex_apply_elements_kernel<P, Q, T><<<(unsigned)((e - b + kElemThreads - 1) / kElemThreads), kElemThreads, 0, s>>>(
           b, e, scatter, op->d_offsets, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec, op->d_tpos, op->d_elem_sys, op->d_sys_active,
           op->d_geo, op->d_geo_pts);
@@ -282,7 +291,7 @@ void launch_geo_lines(const CeedMi355Operator_private *op, int64_t b, int64_t e,
   const int64_t epb = op->epb, grid = (e - b + epb - 1) / epb;
   hex_apply_lines_kernel<P, Q, NC, QF, T, false, true><<<(unsigned)grid, (unsigned)(epb * Q * Q), line_lds_bytes(Q, NC, QF, sizeof(T), true, (int)epb), s>>>(
       b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec,
-      op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, op->d_geo, op->d_geo_pts, op->d_perm, kappa_src, (T *)op->d_qdata);
+      op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, op->d_geo, op->d_geo_pts, op->d_perm, kappa_src, (T *)op->d_qdata, op->d_trow, op->d_tcount);
 }
 
 // Dispatch over the instantiated (P, Q) pairs: P = 2..9, Q in {P, P+1}.

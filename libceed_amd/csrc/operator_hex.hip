@@ -406,6 +406,14 @@ int build_transpose_map(CeedMi355Operator op, const int32_t *offsets) {
   MI355_HIP(hipMalloc(&op->d_evec, (size_t)op->scalar_bytes * (nnz + 1)));
   MI355_HIP(hipMemcpy(op->d_trow, row.data(), sizeof(int32_t) * row.size(), hipMemcpyHostToDevice));
   MI355_HIP(hipMemcpy(op->d_tpos, pos.data(), sizeof(int32_t) * pos.size(), hipMemcpyHostToDevice));
+  // line_last: every L entry has a contribution (the gather also zeroes the
+  // others), and the elements fit its workgroups at the most there can be in one
+  bool last = mi355::line_takes_last(op->P, op->num_comp) && op->num_elem <= mi355::kLastWorkgroups * (256 / (op->Q * op->Q));
+  for (int64_t t = 0; t < op->l_size && last; t++) last = row[t] < row[t + 1];
+  if (last) {
+    MI355_HIP(hipMalloc(&op->d_tcount, sizeof(int32_t) * (size_t)op->l_size));
+    MI355_HIP(hipMemset(op->d_tcount, 0, sizeof(int32_t) * (size_t)op->l_size));
+  }
   return CEED_MI355_SUCCESS;
 }
 
@@ -560,6 +568,8 @@ int split_finish(const CeedMi355Operator_private *op, void *v, int overwrite, hi
   MI355_LAUNCH_CHECK();
   return CEED_MI355_SUCCESS;
 }
+
+bool gather_dot_wanted() { return t_gather_dot != nullptr; }
 
 int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, hipStream_t s) {
   if (op->d_gather_chunk_begin && op->d_sys_active && op->gather_num_chunks > 0) {
@@ -1206,6 +1216,7 @@ extern "C" int CeedMi355OperatorDestroy(CeedMi355Operator *op) {
   (void)hipFree((*op)->d_mats);
   (void)hipFree((*op)->d_qdata);
   (void)hipFree((*op)->d_trow);
+  (void)hipFree((*op)->d_tcount);
   (void)hipFree((*op)->d_tpos);
   (void)hipFree((*op)->d_evec);
   (void)hipFree((*op)->d_srows);
