@@ -37,9 +37,10 @@ HBM_PEAK_GBS = 8000.0      # MI355X HBM3E, vendor datasheet
 FP64_PEAK_TFLOPS = 78.6    # MI355X FP64 vector/matrix, vendor datasheet
 
 
-def alg_bytes(N: int, E: int, P: int, Q: int, ncomp: int = 1, qcomp: int = 6, s: int = 8) -> int:
-    """Read u + write v + read q_data + read int32 offsets (each stream counted once)."""
-    return s * ncomp * N * 2 + s * qcomp * E * Q ** 3 + 4 * E * P ** 3
+def alg_bytes(N: int, E: int, P: int, Q: int, ncomp: int = 1, qcomp: int = 6, s: int = 8, recomputed: bool = False) -> int:
+    """Read u + write v + read q_data + read int32 offsets (each stream counted once); with the factors recomputed
+    the 21 doubles of the element's map in place of q_data."""
+    return s * ncomp * N * 2 + (8 * 21 * E if recomputed else s * qcomp * E * Q ** 3) + 4 * E * P ** 3
 
 
 def alg_flops(E: int, P: int, Q: int, ncomp: int = 1) -> int:
@@ -66,6 +67,7 @@ def time_gpu(fn, steps: int, warmup: int):
 
 
 LAYOUT_NAMES = ["columns", "lines", "points"]  # the fused kernel's thread layouts, by their index in the library
+# (order 1 on many elements: hex_apply_elements_kernel in the lines' place)
 KERNEL_OF_LAYOUT = ["hex_apply_kernel", "hex_apply_lines_kernel", "hex_apply_points_kernel"]
 
 
@@ -91,7 +93,8 @@ def run_case(p: int, dofs: float, dtype, steps: int, warmup: int, seed: int = 0,
     ms_apply, wall = time_gpu(lambda: op.apply(u, v), steps, warmup)
     ms_kernel, _ = time_gpu(lambda: op.apply_add(u, v), steps, warmup)
     s = 8 if dtype == torch.float64 else 4
-    B = alg_bytes(m.num_nodes, m.num_elem, P, Q, ncomp=num_comp, s=s)
+    recomputed = op.recomputes_factors()
+    B = alg_bytes(m.num_nodes, m.num_elem, P, Q, ncomp=num_comp, s=s, recomputed=recomputed)
     mode = {"tmap": "transpose map", "color": "element colours", "split": "multiplicity split", "atomic": "atomics",
             "brick": "element bricks", "segment": "element segments"}[op.scatter_mode()]
     F = alg_flops(m.num_elem, P, Q, ncomp=num_comp)
@@ -111,6 +114,7 @@ def run_case(p: int, dofs: float, dtype, steps: int, warmup: int, seed: int = 0,
         "ms_per_apply": ms_apply, "wall_ms_per_apply": wall, "gdofs": num_comp * m.num_nodes / (ms_apply * 1e-3) / 1e9,
         # the roofline figures use Apply's kernel time (the operator's kernels of one apply, HIP events on
         # their stream); ApplyAdd's is reported beside it (the split E^T adds a scratch pass there)
+        "factors": "recomputed from the elements' trilinear maps" if recomputed else "read",
         "kernel_ms": ms_apply, "apply_add_ms": ms_kernel, "alg_bytes": B, "alg_flops": F,
         "kernel_GBs": B / (ms_apply * 1e-3) / 1e9, "kernel_TFLOPs": F / (ms_apply * 1e-3) / 1e12,
     }
@@ -508,9 +512,9 @@ def cpu_baseline(p: int = 4, n: int = 50, seconds: float = 10.0) -> dict | None:
 
 def measured_traffic(head: dict, dtype: str, num_comp: int):
     """HBM bytes per apply from the committed rocprofv3 counter summary of this workload (same order, size,
-    arithmetic, components and E^T mode), and where it comes from.  A summary of another launch of the same
-    plan (layout, elements per workgroup) is used when none of this launch exists, and says so: the launch
-    changes the order of the memory accesses, not the bytes the plan reads and writes."""
+    arithmetic, components, E^T mode and layout), and where it comes from.  A summary of another number of
+    elements per workgroup is used when none of this launch exists, and says so: it changes the order of the
+    memory accesses, not the bytes the plan reads and writes."""
     best = None
     for f in sorted((ROOT / "profiles").glob("*_traffic.json")):
         try:
@@ -518,7 +522,8 @@ def measured_traffic(head: dict, dtype: str, num_comp: int):
         except (OSError, ValueError):
             continue
         w = d.get("workload", {})
-        if (w.get("p"), w.get("dofs"), w.get("dtype"), w.get("scatter"), w.get("num_comp", 1)) != (head["p"], head["dofs"], dtype, head["scatter"], num_comp):
+        if (w.get("p"), w.get("dofs"), w.get("dtype"), w.get("scatter"), w.get("num_comp", 1), w.get("layout")) != (
+                head["p"], head["dofs"], dtype, head["scatter"], num_comp, head["layout"]):
             continue
         same = (w.get("layout"), w.get("elems_per_block")) == (head["layout"], head["elems_per_block"])
         src = d.get("source", f.name) + ("" if same else f" (launch {w.get('layout')} x {w.get('elems_per_block')}; this run's launch "
@@ -642,7 +647,7 @@ def main() -> None:
                    "layout": head["layout"], "elems_per_block": head["elems_per_block"], "num_comp": args.ncomp},
         "roofline": {"bound": "hbm", "achieved": round(head["kernel_GBs"], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(head["hbm_frac"], 4), "traffic": traffic[0], "traffic_source": traffic[1],
-                     "kernel": head["kernels"],
+                     "kernel": head["kernels"], "factors": head["factors"],
                      "alg_bytes_per_apply": head["alg_bytes"], "kernel_ms_per_apply": round(head["kernel_ms"], 5),
                      "apply_add_ms": round(head["apply_add_ms"], 5),
                      "fp64_tflops": round(head["kernel_TFLOPs"], 2), "fp64_peak_tflops": FP64_PEAK_TFLOPS},

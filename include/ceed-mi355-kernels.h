@@ -241,6 +241,10 @@ int CeedMi355OperatorSetLaunch(CeedMi355Operator op, int32_t elems_per_block);
 int CeedMi355OperatorSetLayout(CeedMi355Operator op, int32_t layout, int32_t elems_per_block);
 /* Current thread layout and elements per workgroup (either pointer may be NULL). */
 int CeedMi355OperatorGetLaunch(CeedMi355Operator op, int32_t *layout, int32_t *elems_per_block);
+/* 1 if Apply recomputes the geometric factors from the elements' trilinear
+ * maps with the current launch (it then reads 168 bytes per element of them),
+ * 0 if it reads the stored ones. */
+int CeedMi355OperatorRecomputesFactors(CeedMi355Operator op, int32_t *yes);
 /* Autotuner (the reference has none: its hip-shared/hip-gen backends fix the
  * launch shape per P, Q): time Apply (reps times) for every admissible
  * (thread layout, elements per workgroup) on scratch vectors, time the three

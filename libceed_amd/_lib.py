@@ -77,6 +77,7 @@ SIGNATURES = {
     "CeedMi355OperatorSetLaunch": (c_int, [vp, c_i32]),
     "CeedMi355OperatorAutotune": (c_int, [vp, c_i32, vp, vp, vp]),
     "CeedMi355OperatorSetLayout": (c_int, [vp, c_i32, c_i32]),
+    "CeedMi355OperatorRecomputesFactors": (c_int, [vp, vp]),
     "CeedMi355OperatorGetLaunch": (c_int, [vp, vp, vp]),
     "CeedRegister_Mi355": (c_int, []),
     "CeedInit_Mi355": (c_int, [C.c_char_p, vp]),

@@ -412,7 +412,9 @@ int build_transpose_map(CeedMi355Operator op, const int32_t *offsets) {
   for (int64_t t = 0; t < op->l_size && last; t++) last = row[t] < row[t + 1];
   if (last) {
     MI355_HIP(hipMalloc(&op->d_tcount, sizeof(int32_t) * (size_t)op->l_size));
-    MI355_HIP(hipMemset(op->d_tcount, 0, sizeof(int32_t) * (size_t)op->l_size));
+    // (a copy: done when it returns, also for a stream that does not wait for the null stream)
+    const std::vector<int32_t> zero((size_t)op->l_size, 0);
+    MI355_HIP(hipMemcpy(op->d_tcount, zero.data(), sizeof(int32_t) * zero.size(), hipMemcpyHostToDevice));
   }
   return CEED_MI355_SUCCESS;
 }
@@ -1098,6 +1100,12 @@ extern "C" int CeedMi355OperatorSetLayout(CeedMi355Operator op, int32_t layout, 
   op->layout     = layout;
   op->epb        = epb;
   op->own_launch = true;
+  return CEED_MI355_SUCCESS;
+}
+
+extern "C" int CeedMi355OperatorRecomputesFactors(CeedMi355Operator op, int32_t *yes) {
+  MI355_CHECK(op && yes, CEED_MI355_ERROR_MAJOR, "null argument");
+  *yes = mi355::plan_recomputes(op);
   return CEED_MI355_SUCCESS;
 }
 

@@ -250,6 +250,12 @@ class HexOperator:
         call("CeedMi355OperatorAutotune", self._h, int(reps), C.byref(best), C.byref(ms), _stream())
         return best.value, ms.value
 
+    def recomputes_factors(self) -> bool:
+        """Whether apply recomputes the geometric factors (trilinear geometry) instead of reading them, with the current launch."""
+        yes = C.c_int32()
+        call("CeedMi355OperatorRecomputesFactors", self._h, C.byref(yes))
+        return bool(yes.value)
+
     def scatter_mode(self) -> str:
         """The plan's E^T mode: "tmap", "color", "split", "atomic", "brick" or "segment"."""
         mode = C.c_int32()
