@@ -358,7 +358,8 @@ int CeedMi355CGCreate(CeedMi355Operator op, CeedMi355Operator op64, CeedMi355CG 
  * ||r|| <= rtol ||b|| (tested every check_every iterations; the recursive
  * residual for plain CG, the replaced FP64 residual for mixed precision) or
  * after max_iter iterations.  use_graph != 0 captures check_every iterations
- * in a hipGraph once and replays it.  Ordered after the caller's stream;
+ * in a hipGraph once and replays it (captured again when a plan's factors
+ * become recomputed ones or stored ones).  Ordered after the caller's stream;
  * returns when the solve is done. */
 int CeedMi355CGSolve(CeedMi355CG cg, const double *b, double *x, int32_t max_iter, double rtol, int32_t check_every, int use_graph, void *stream,
                      CeedMi355CGStats *stats_host);

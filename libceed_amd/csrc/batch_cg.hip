@@ -168,6 +168,7 @@ struct CeedMi355BatchCG_private {
   int                            graph_len = 0;
   const void                    *graph_b = nullptr;
   void                          *graph_x = nullptr;
+  std::vector<bool>              graph_geo;  // geo_valid of the plans at the capture
 };
 
 namespace {
@@ -224,12 +225,17 @@ int segment(CeedMi355BatchCG cg, double *x, int len) {
 
 int run_segment(CeedMi355BatchCG cg, const double *b, double *x, int len, bool use_graph) {
   if (!use_graph) return segment(cg, x, len);
-  if (!cg->graph || cg->graph_len != len || cg->graph_b != b || cg->graph_x != x) {
+  // the captured kernels are those of the plans' factors then: recomputed or read
+  std::vector<bool> geo;
+  for (CeedMi355Operator op : cg->ops) geo.push_back(op->geo_valid);
+  if (!cg->graph || cg->graph_len != len || cg->graph_b != b || cg->graph_x != x || cg->graph_geo != geo) {
     if (cg->graph) (void)hipGraphExecDestroy(cg->graph);
     cg->graph = nullptr;
     hipGraph_t g;
     MI355_HIP(hipStreamBeginCapture(cg->stream, hipStreamCaptureModeThreadLocal));
-    const int  err = segment(cg, x, len);
+    for (CeedMi355Operator op : cg->ops) op->solver_graph = true;
+    const int err = segment(cg, x, len);
+    for (CeedMi355Operator op : cg->ops) op->solver_graph = false;
     hipError_t e   = hipStreamEndCapture(cg->stream, &g);
     if (err) return err;
     MI355_HIP(e);
@@ -239,6 +245,7 @@ int run_segment(CeedMi355BatchCG cg, const double *b, double *x, int len, bool u
     cg->graph_len = len;
     cg->graph_b   = b;
     cg->graph_x   = x;
+    cg->graph_geo = geo;
   }
   MI355_HIP(hipGraphLaunch(cg->graph, cg->stream));
   return CEED_MI355_SUCCESS;

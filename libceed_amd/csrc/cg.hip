@@ -261,6 +261,7 @@ struct CeedMi355CG_private {
   int               graph_len = 0;
   const void       *graph_b = nullptr;
   void             *graph_x = nullptr;
+  bool              graph_geo = false, graph_geo64 = false;  // geo_valid of op and op64 at the capture
 };
 
 namespace {
@@ -347,12 +348,18 @@ int segment(CeedMi355CG cg, const double *b, double *x, int len, bool update) {
 
 int run_segment(CeedMi355CG cg, const double *b, double *x, int len, bool update, bool use_graph) {
   if (!use_graph) return segment(cg, b, x, len, update);
-  if (!cg->graph || cg->graph_len != len || cg->graph_b != b || cg->graph_x != x) {
+  // the captured kernels are those of the plans' factors then: recomputed or read
+  const bool geo = cg->op->geo_valid, geo64 = cg->mixed && cg->op64->geo_valid;
+  if (!cg->graph || cg->graph_len != len || cg->graph_b != b || cg->graph_x != x || cg->graph_geo != geo || cg->graph_geo64 != geo64) {
     if (cg->graph) (void)hipGraphExecDestroy(cg->graph);
     cg->graph = nullptr;
     hipGraph_t g;
     MI355_HIP(hipStreamBeginCapture(cg->stream, hipStreamCaptureModeThreadLocal));
+    cg->op->solver_graph = true;
+    if (cg->mixed) cg->op64->solver_graph = true;
     const int err = segment(cg, b, x, len, update);
+    cg->op->solver_graph = false;
+    if (cg->mixed) cg->op64->solver_graph = false;
     hipError_t e  = hipStreamEndCapture(cg->stream, &g);
     if (err) return err;
     MI355_HIP(e);
@@ -362,6 +369,7 @@ int run_segment(CeedMi355CG cg, const double *b, double *x, int len, bool update
     cg->graph_len = len;
     cg->graph_b   = b;
     cg->graph_x   = x;
+    cg->graph_geo = geo, cg->graph_geo64 = geo64;
   }
   MI355_HIP(hipGraphLaunch(cg->graph, cg->stream));
   return CEED_MI355_SUCCESS;

@@ -214,11 +214,12 @@ __global__ void __launch_bounds__(256) hex_adjoint_lines_kernel(int64_t elem_beg
                                                                 const double *__restrict__ lam, double *__restrict__ v, double *__restrict__ evec,
                                                                 const int32_t *__restrict__ tpos, double *__restrict__ g,
                                                                 const double *__restrict__ geo, const double *__restrict__ geo_pts,
-                                                                const double *__restrict__ kappa_src) {
+                                                                const double *__restrict__ kappa_src, const int32_t *__restrict__ turn) {
   constexpr int  NT = Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QC = 7;
   constexpr int  SR = line_row_stride(Q, 8), SP = line_plane_stride(Q, 8), SLAB = Q * SP, ES = adjoint_elem_entries(Q);
   constexpr bool kRowWise = Q >= 7;
   extern __shared__ __align__(16) unsigned char lds_raw[];
+  if (turn && !*turn) return;  // in a caller's graph, where the other of the two kernels runs
   const int epb = blockDim.x / NT;
   const int le = threadIdx.x / NT, t = threadIdx.x - le * NT;
   double   *X = reinterpret_cast<double *>(lds_raw) + le * ES, *Y = X + SLAB, *UX = Y + SLAB, *UY = UX + SLAB;
@@ -488,6 +489,7 @@ int launch_adjoint(const CeedMi355Operator_private *op, const double *u, const d
   const bool   geo   = lines && op->geo_valid;  // as in CeedMi355OperatorApplyAdjointKappa
   const size_t lds   = sizeof(double) * (size_t)(lines ? epb * (adjoint_elem_entries(Q) + (geo ? kGeoLds : 0)) : Q * P + Q * Q + epb * 3 * Q * Q * Q);
   const bool   tmap  = op->scatter == 0;
+  const int32_t *turn = geo && into_callers_graph(op, s) ? op->d_geo_turn : nullptr;
   MI355_CHECK(op->scatter != CEED_MI355_PLAN_SEGMENT, CEED_MI355_ERROR_UNSUPPORTED,
               "the adjoint does not take segment plans (elements of a colour share segment faces)");
   MI355_CHECK(lds <= (size_t)kMaxLdsBytes, CEED_MI355_ERROR_BACKEND, "adjoint needs %zu bytes of LDS at %d elements per workgroup", lds, epb);
@@ -501,12 +503,12 @@ int launch_adjoint(const CeedMi355Operator_private *op, const double *u, const d
     if (geo)
       hex_adjoint_lines_kernel<P, Q, true><<<(unsigned)grid, epb * nt, lds, s>>>(b, e, scatter, op->d_offsets, op->d_perm, (double *)op->d_qdata,
                                                                                 (const double *)op->d_mats, u, lam, v, (double *)op->d_evec,
-                                                                                op->d_tpos, g, op->d_geo, op->d_geo_pts, kappa_src);
-    else if (lines)
+                                                                                op->d_tpos, g, op->d_geo, op->d_geo_pts, kappa_src, turn);
+    if (lines && (!geo || turn))
       hex_adjoint_lines_kernel<P, Q, false><<<(unsigned)grid, epb * nt, lds, s>>>(b, e, scatter, op->d_offsets, op->d_perm, (double *)op->d_qdata,
                                                                                  (const double *)op->d_mats, u, lam, v, (double *)op->d_evec,
-                                                                                 op->d_tpos, g, nullptr, nullptr, nullptr);
-    else
+                                                                                 op->d_tpos, g, nullptr, nullptr, nullptr, turn ? turn + 1 : nullptr);
+    if (!lines)
       hex_adjoint_kernel<P, Q><<<(unsigned)grid, epb * nt, lds, s>>>(b, e, scatter, op->d_offsets, op->d_perm, (const double *)op->d_qdata,
                                                                     (const double *)op->d_mats, u, lam, v, (double *)op->d_evec, op->d_tpos, g);
   }
@@ -545,7 +547,8 @@ extern "C" int CeedMi355OperatorApplyAdjointKappa(CeedMi355Operator op, const do
   if (op->num_elem == 0) return CEED_MI355_SUCCESS;
   auto fn = mi355::pick_adjoint(op->P, op->Q);
   MI355_CHECK(fn, CEED_MI355_ERROR_UNSUPPORTED, "no adjoint kernel for P=%d Q=%d", op->P, op->Q);
-  if (kappa && !(op->layout == mi355::kLayoutLines && op->geo_valid)) {  // only that kernel takes kappa from the caller
+  // only that kernel takes kappa from the caller, and in a caller's graph it may be the other one that runs
+  if (kappa && (!(op->layout == mi355::kLayoutLines && op->geo_valid) || mi355::into_callers_graph(op, s))) {
     const int err = CeedMi355OperatorSetKappa(op, kappa, stream);
     if (err) return err;
     kappa = nullptr;

@@ -42,10 +42,11 @@ __global__ void __launch_bounds__(256, (P <= 5 ? 4 : 1)) hex_diag_kernel(int64_t
                                                        const int32_t *__restrict__ offsets, int32_t comp_stride, const T *__restrict__ q_data,
                                                        const T *__restrict__ mats, const double *__restrict__ geo,
                                                        const double *__restrict__ geo_pts, T *__restrict__ v, T *__restrict__ evec,
-                                                       const int32_t *__restrict__ tpos) {
+                                                       const int32_t *__restrict__ tpos, const int32_t *__restrict__ turn) {
   constexpr int NT = Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QP = Q * P, QC = QfTraits<QF>::kComps, NS = diag_slabs(QF), NA = QF == kQfMass ? 1 : 6;
   constexpr int SR = line_row_stride(Q, sizeof(T)), SP = line_plane_stride(Q, sizeof(T)), SLAB = P * SP;
   extern __shared__ __align__(16) unsigned char lds_raw[];
+  if (turn && !*turn) return;  // in a caller's graph, where the other of the two kernels runs
   const int     epb = blockDim.x / NT, le = threadIdx.x / NT, t = threadIdx.x - le * NT;
   T            *A  = reinterpret_cast<T *>(lds_raw) + (size_t)le * NS * SLAB;
   auto          at = [](int k, int z, int y, int x) { return k * SLAB + z * SP + y * SR + x; };
@@ -250,12 +251,17 @@ int launch_diag_elements(const CeedMi355Operator_private *op, int64_t b, int64_t
 #define MI355_DIAG_LAUNCH(QF, GEO)                                                                                                        \
   hex_diag_kernel<P, Q, QF, GEO, T><<<grid, nt, epb * per, s>>>(b, e, scatter, op->num_comp, op->d_offsets, op->comp_stride,              \
                                                                 (const T *)op->d_qdata, (const T *)op->d_mats, op->d_geo, op->d_geo_pts, v, \
-                                                                (T *)op->d_evec, op->d_tpos)
-  if (op->qf == kQfMass) MI355_DIAG_LAUNCH(kQfMass, false);
-  else if (op->qf == kQfDiffusion && op->geo_valid) MI355_DIAG_LAUNCH(kQfDiffusion, true);
-  else if (op->qf == kQfDiffusion) MI355_DIAG_LAUNCH(kQfDiffusion, false);
-  else if (op->geo_valid) MI355_DIAG_LAUNCH(kQfDiffusionKappa, true);
-  else MI355_DIAG_LAUNCH(kQfDiffusionKappa, false);
+                                                                (T *)op->d_evec, op->d_tpos, two ? op->d_geo_turn + !GEO : nullptr)
+  const bool two = op->geo_valid && into_callers_graph(op, s), stored = !op->geo_valid || two;
+  if (op->qf == kQfMass) {
+    MI355_DIAG_LAUNCH(kQfMass, false);
+  } else if (op->qf == kQfDiffusion) {
+    if (op->geo_valid) MI355_DIAG_LAUNCH(kQfDiffusion, true);
+    if (stored) MI355_DIAG_LAUNCH(kQfDiffusion, false);
+  } else {
+    if (op->geo_valid) MI355_DIAG_LAUNCH(kQfDiffusionKappa, true);
+    if (stored) MI355_DIAG_LAUNCH(kQfDiffusionKappa, false);
+  }
 #undef MI355_DIAG_LAUNCH
   MI355_LAUNCH_CHECK();
   return CEED_MI355_SUCCESS;

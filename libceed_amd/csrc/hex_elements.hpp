@@ -46,7 +46,14 @@ __global__ void __launch_bounds__(kElemThreads, 2) hex_apply_elements_kernel(int
   const int64_t first = elem_begin + xcd_chunk(blockIdx.x, gridDim.x) * kElemThreads;
   const int     lane = threadIdx.x, n = (int)(elem_end - first < kElemThreads ? elem_end - first : kElemThreads);
   const int64_t e    = first + lane;
-  const bool    live = lane < n && (!elem_sys || sys_active[elem_sys[e]]);
+  bool          live = lane < n;
+  if (elem_sys) {
+    if (elem_sys == sys_active) {
+      if (!*sys_active) return;
+    } else {
+      live = live && sys_active[elem_sys[e]];
+    }
+  }
 
   // (lanes past the end read the last element and store nothing)
   const int64_t er = lane < n ? e : elem_end - 1;

@@ -583,8 +583,17 @@ __global__ void __launch_bounds__(256, (lines_min_waves<P, Q, NCOMP, QF, T, kGeo
   const int32_t sbeg  = kSeg ? seg_start[elem_begin + chunk] : 0;
   const int32_t slen  = kSeg ? seg_start[elem_begin + chunk + 1] - sbeg : 0;
   const int64_t e     = kSeg ? (int64_t)sbeg + le : elem_begin + chunk * epb + le;
-  const bool    live  = le < epb && (kSeg ? le < slen : e < elem_end) && (!elem_sys || sys_active[elem_sys[e]]);
-  if (elem_sys && !__syncthreads_or(live)) return;  // every element of the workgroup is frozen (uniform exit)
+  bool          live  = le < epb && (kSeg ? le < slen : e < elem_end);
+  // elem_sys: the system of each element, where some are frozen; the same
+  // pointer as sys_active: one entry for all, in a caller's graph (into_callers_graph)
+  if (elem_sys) {
+    if (elem_sys == sys_active) {
+      if (!*sys_active) return;
+    } else {
+      live = live && sys_active[elem_sys[e]];
+      if (!__syncthreads_or(live)) return;  // every element of the workgroup is frozen (uniform exit)
+    }
+  }
 
   const int  cx = t % Q, cy = t / Q;  // column; also the x-line (qy = cx, qz = cy) and the y-line (qx = cx, qz = cy)
   const int  ny = t % P, nz = t / P;  // x-line of nodes

@@ -19,8 +19,20 @@ namespace mi355 {
 
 // the line kernel with recomputed geometric factors over elements [b, e) of a plan (hex_geo_*.hip)
 // (kappa_src: kappa-weighted plans, the caller's kappa, nullptr for the plan's)
+// (two: the kernel that reads the factors is launched beside it, see into_callers_graph)
 using GeoLinesFn = void (*)(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, const double *kappa_src,
-                            hipStream_t s);
+                            bool two, hipStream_t s);
+// The launch on s goes into a graph of the caller's, which may be replayed
+// after the plan's factors have changed kind.  It takes both kernels, the one
+// that recomputes the factors and the one that reads them, and at a replay one
+// of them returns at once by the plan's d_geo_turn (in the line kernels on the
+// arguments for the batched solver's stopped systems: an early return behind
+// one more argument cost the applies outside graphs 1% at p=4, and a branch
+// around the factors inside the recomputing kernels costs them 14-40 VGPRs
+// from Q = 4, one or two waves per SIMD).  MI355X, us per replayed apply, the
+// one kernel / both: p=2 2k DoFs 7.6 / 9.1, p=3 0.9M 37.2 / 39.9, p=1 0.5M 77 /
+// 86, p=4 8M in eight colours 214 / 235.
+bool into_callers_graph(const CeedMi355Operator_private *op, hipStream_t s);
 // Kappa of the apply running on this thread (CeedMi355OperatorApplyKappa), nullptr for the plan's own.
 const double *kappa_of_apply();
 // The apply running on this thread wants its transpose_gather to form a dot product (apply_dot).
@@ -185,9 +197,15 @@ struct CeedMi355Operator_private {
   mi355::ApplyFn       apply     = nullptr;
   // trilinear geometry: the map's coefficients [elem][kGeoStride] in packed
   // order and the 1D points and weights (2 Q doubles); geo_valid: d_qdata
-  // holds the factors of this geometry, which geo_lines may recompute
+  // holds the factors of this geometry, which geo_lines may recompute.  A
+  // SetQData that went into a graph happens when that is replayed: the plan
+  // reads its factors from then on (qdata_in_graph).  solver_graph: the launches
+  // being captured are a solver's of this library, which captures again when
+  // geo_valid changes.  For the graphs of a caller: d_geo_turn, 1 and 0 while
+  // the factors are the geometry's and 0 and 1 once they are others.
   double              *d_geo = nullptr, *d_geo_pts = nullptr;
-  bool                 geo_valid = false;
+  int32_t             *d_geo_turn = nullptr;
+  bool                 geo_valid = false, qdata_in_graph = false, solver_graph = false;
   mi355::GeoLinesFn    geo_lines = nullptr;
   CeedMi355JitKernel  *jit       = nullptr;  // kQfJit plans: the compiled kernel and the QFunction context
 };
@@ -241,6 +259,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
     if (err) return err;
   }
   const bool geo = plan_recomputes(op);
+  const bool two = geo && into_callers_graph(op, s);  // both kernels, by turns (d_geo_turn)
   // kScatterLast: frozen systems' contributions never arrive, a dot product
   // wants the gather, and where u and v overlap all of u is read first
   const size_t l_bytes = sizeof(T) * (size_t)op->l_size;
@@ -254,12 +273,17 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
                             : tmap ? kScatterEvec
                                  : split ? kScatterSplit
                                          : (op->scatter == CEED_MI355_PLAN_ATOMIC ? kScatterAtomic : (overwrite ? kScatterOverwrite : kScatterAdd));
-    if (geo) op->geo_lines(op, b, e, scatter, u, target, kappa_of_apply(), s);
-    else if (lines)
-      hex_apply_lines_kernel<P, Q, NC, QF, T><<<(unsigned)grid, epb * nt, lds, s>>>(
-          b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, target, (T *)op->d_evec,
-          op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, op->d_trow, op->d_tcount);
-    else if (points) {
+    if (lines) {
+      if (geo) op->geo_lines(op, b, e, scatter, u, target, kappa_of_apply(), two, s);
+      if (!geo || two) {
+        // (beside the recomputing kernel it mostly returns at once, the faster the fewer its workgroups)
+        const int n = two && line_lds_bytes(Q, NC, QF, sizeof(T), false, 256 / nt) <= (size_t)kMaxLdsBytes ? 256 / nt : epb;
+        hex_apply_lines_kernel<P, Q, NC, QF, T><<<(unsigned)((e - b + n - 1) / n), n * nt, line_lds_bytes(Q, NC, QF, sizeof(T), false, n), s>>>(
+            b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, target, (T *)op->d_evec,
+            op->d_tpos, two ? op->d_geo_turn + 1 : op->d_elem_sys, two ? op->d_geo_turn + 1 : op->d_sys_active, nullptr, nullptr, nullptr, nullptr, nullptr,
+            nullptr, op->d_trow, op->d_tcount);
+      }
+    } else if (points) {
       if constexpr (Q * Q * Q <= 256)
         hex_apply_points_kernel<P, Q, NC, QF, T><<<(unsigned)grid, epb * Q * Q * Q, lds, s>>>(
             b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, target,
@@ -279,19 +303,20 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
 
 template <int P, int Q, int NC, int QF, typename T>
 void launch_geo_lines(const CeedMi355Operator_private *op, int64_t b, int64_t e, int scatter, const void *u, void *v, const double *kappa_src,
-                      hipStream_t s) {
+                      bool two, hipStream_t s) {
+  const int32_t *elem_sys = two ? op->d_geo_turn : op->d_elem_sys, *sys_active = two ? op->d_geo_turn : op->d_sys_active;
   if constexpr (P == 2 && NC == 1 && QF == kQfDiffusion) {
     if (scatter < kScatterLast && e - b >= elements_min<Q, T>()) {
       hex_apply_elements_kernel<P, Q, T><<<(unsigned)((e - b + kElemThreads - 1) / kElemThreads), kElemThreads, 0, s>>>(
-          b, e, scatter, op->d_offsets, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec, op->d_tpos, op->d_elem_sys, op->d_sys_active,
-          op->d_geo, op->d_geo_pts);
+          b, e, scatter, op->d_offsets, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec, op->d_tpos, elem_sys, sys_active, op->d_geo,
+          op->d_geo_pts);
       return;
     }
   }
   const int64_t epb = op->epb, grid = (e - b + epb - 1) / epb;
   hex_apply_lines_kernel<P, Q, NC, QF, T, false, true><<<(unsigned)grid, (unsigned)(epb * Q * Q), line_lds_bytes(Q, NC, QF, sizeof(T), true, (int)epb), s>>>(
       b, e, scatter, op->d_offsets, op->comp_stride, (const T *)op->d_qdata, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec,
-      op->d_tpos, op->d_elem_sys, op->d_sys_active, nullptr, op->d_geo, op->d_geo_pts, op->d_perm, kappa_src, (T *)op->d_qdata, op->d_trow, op->d_tcount);
+      op->d_tpos, elem_sys, sys_active, nullptr, op->d_geo, op->d_geo_pts, op->d_perm, kappa_src, (T *)op->d_qdata, op->d_trow, op->d_tcount);
 }
 
 // Dispatch over the instantiated (P, Q) pairs: P = 2..9, Q in {P, P+1}.

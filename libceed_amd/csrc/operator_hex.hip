@@ -267,6 +267,23 @@ __global__ void __launch_bounds__(256) geo_qdata(int64_t num_elem, int Q, int qf
   }
 }
 
+// The plan's stored factors are no longer its trilinear geometry's: for the graphs captured while they were
+__global__ void mark_replaced(int32_t *turn) { turn[0] = 0, turn[1] = 1; }
+
+int factors_replaced(CeedMi355Operator op, hipStream_t s) {
+  if (!op->d_geo_turn) return CEED_MI355_SUCCESS;
+  mark_replaced<<<1, 1, 0, s>>>(op->d_geo_turn);
+  MI355_LAUNCH_CHECK();
+  return CEED_MI355_SUCCESS;
+}
+
+bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st == hipStreamCaptureStatusActive;
+  (void)hipGetLastError();
+  return false;
+}
+
 // Whether a mesh basis of two nodes is the linear one, (1 -+ xi)/2 at every point with slopes -+1/2
 bool linear_mesh_basis(int Q, const double *B, const double *G) {
   for (int q = 0; q < Q; q++)
@@ -362,6 +379,7 @@ int plan_default_epb(const CeedMi355Operator op, int layout) {
 // The factors of the plan are from now on a trilinear geometry's (valid) or
 // the caller's; a launch nobody chose follows.
 void set_geo_valid(CeedMi355Operator op, bool valid) {
+  valid = valid && !op->qdata_in_graph;
   if (op->geo_valid == valid) return;
   op->geo_valid = valid;
   if (op->own_launch || op->scatter == CEED_MI355_PLAN_SEGMENT) return;
@@ -908,12 +926,15 @@ extern "C" int CeedMi355OperatorBuildQData(CeedMi355Operator op, int build, int3
   int ierr;
   const int64_t blk = elem_block(op);
   bool                trilinear = false;
-  std::vector<double> pts(2 * Q);  // read by the copy below until the synchronisation
+  std::vector<double>  pts(2 * Q);  // pts, turn: read by the copies below until the synchronisation
+  const int32_t        turn[2] = {1, 0};
   if (PM == 2 && linear_mesh_basis(Q, mesh_interp_1d_host, mesh_grad_1d_host)) {
     for (int q = 0; q < Q; q++) pts[q] = mesh_interp_1d_host[2 * q + 1] - mesh_interp_1d_host[2 * q], pts[Q + q] = q_weight_1d_host[q];
     if (!op->d_geo) MI355_HIP(hipMalloc(&op->d_geo, sizeof(double) * mi355::kGeoStride * ((size_t)op->num_elem + 1)));
-    if (!op->d_geo_pts) MI355_HIP(hipMalloc(&op->d_geo_pts, sizeof(double) * 2 * Q));
-    MI355_HIP(hipMemcpyAsync(op->d_geo_pts, pts.data(), sizeof(double) * 2 * Q, hipMemcpyHostToDevice, s));
+    if (!op->d_geo_pts) MI355_HIP(hipMalloc(&op->d_geo_pts, sizeof(double) * pts.size()));
+    if (!op->d_geo_turn) MI355_HIP(hipMalloc(&op->d_geo_turn, sizeof(turn)));
+    MI355_HIP(hipMemcpyAsync(op->d_geo_pts, pts.data(), sizeof(double) * pts.size(), hipMemcpyHostToDevice, s));
+    MI355_HIP(hipMemcpyAsync(op->d_geo_turn, turn, sizeof(turn), hipMemcpyHostToDevice, s));
     const int64_t q3 = (int64_t)Q * Q * Q;
     geo_coefficients<<<mi355_blocks(op->num_elem * 3, 256), 256, 0, s>>>(op->num_elem, d_mo, mesh_comp_stride, coords, op->d_geo);
     if (op->scalar_type == CEED_MI355_FP64)
@@ -925,6 +946,7 @@ extern "C" int CeedMi355OperatorBuildQData(CeedMi355Operator op, int build, int3
   } else if (op->scalar_type == CEED_MI355_FP64)
     ierr = dispatch_build<double>(Q, build, op->num_elem, PM, d_mo, mesh_comp_stride, coords, d_mats, blk, (double *)op->d_qdata, s);
   else ierr = dispatch_build<float>(Q, build, op->num_elem, PM, d_mo, mesh_comp_stride, coords, d_mats, blk, (float *)op->d_qdata, s);
+  if (!ierr && !trilinear) ierr = factors_replaced(op, s);
   MI355_HIP(hipStreamSynchronize(s));
   (void)hipFree(d_mo);
   (void)hipFree(d_mats);
@@ -947,8 +969,11 @@ extern "C" int CeedMi355OperatorSetQData(CeedMi355Operator op, const void *q_dat
   const int64_t blk = elem_block(op);
   hipStream_t   s   = (hipStream_t)stream;
   MI355_CHECK(per == blk || op->qf == kQfDiffusionKappa, CEED_MI355_ERROR_BACKEND, "layout mismatch");
-  if (op->qf != kQfDiffusionKappa) set_geo_valid(op, false);  // the caller's factors from here on
-  if (op->qf != kQfDiffusionKappa) {
+  if (op->qf != kQfDiffusionKappa) {  // the caller's factors from here on
+    if (is_capturing(s)) op->qdata_in_graph = true;
+    set_geo_valid(op, false);
+    const int err = factors_replaced(op, s);
+    if (err) return err;
     if (op->scalar_type == CEED_MI355_FP64)
       permute_elements<double, double><<<mi355_blocks(op->num_elem * per, 256), 256, 0, s>>>(op->num_elem, per, op->d_perm, 1,
                                                                                              (const double *)q_data, (double *)op->d_qdata);
@@ -1031,12 +1056,15 @@ thread_local const double *t_kappa = nullptr;  // set for the time of one ApplyK
 
 const double *mi355::kappa_of_apply() { return t_kappa; }
 
+bool mi355::into_callers_graph(const CeedMi355Operator_private *op, hipStream_t s) { return !op->solver_graph && is_capturing(s); }
+
 extern "C" int CeedMi355OperatorApplyKappa(CeedMi355Operator op, const double *kappa, const void *u, void *v, void *stream) {
   MI355_CHECK(op && op->qf == kQfDiffusionKappa && (kappa || op->num_elem == 0), CEED_MI355_ERROR_BACKEND,
               "ApplyKappa needs a kappa-diffusion operator and kappa");
   // the line kernel that recomputes the factors takes kappa from the caller
-  // and keeps it on the way, unless it may skip elements (stopped systems)
-  if (!mi355::plan_recomputes(op) || op->d_elem_sys) {
+  // and keeps it on the way, unless it may skip elements (stopped systems) or
+  // is one of two kernels in a caller's graph
+  if (!mi355::plan_recomputes(op) || op->d_elem_sys || mi355::into_callers_graph(op, (hipStream_t)stream)) {
     const int err = CeedMi355OperatorSetKappa(op, kappa, stream);
     return err ? err : CeedMi355OperatorApply(op, u, v, stream);
   }
@@ -1239,6 +1267,7 @@ extern "C" int CeedMi355OperatorDestroy(CeedMi355Operator *op) {
   (void)hipFree((*op)->d_seg_start);
   (void)hipFree((*op)->d_geo);
   (void)hipFree((*op)->d_geo_pts);
+  (void)hipFree((*op)->d_geo_turn);
   delete *op;
   *op = nullptr;
   return CEED_MI355_SUCCESS;
