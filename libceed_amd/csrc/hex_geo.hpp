@@ -53,12 +53,18 @@ __device__ __forceinline__ double geo_dot(const double (&a)[3], const double (&b
   return __builtin_fma(a[2], b[2], __builtin_fma(a[1], b[1], a[0] * b[0]));
 }
 
-// 1 / x to within two units in the last place: the hardware's reciprocal and
-// two Newton steps (5 instructions; the IEEE division takes 11)
-__device__ __forceinline__ double geo_rcp(double x) {
+// w / x with 1 / x to within two units in the last place: the hardware's
+// reciprocal and two Newton steps, which turn the infinite reciprocal of 0 into
+// NaN, so the last instruction puts the division's own result where x or w is 0,
+// infinite or NaN (7 instructions; the IEEE division takes 11).  An element of
+// no volume then has the factors the division gives it, infinite or NaN
+// (without that instruction NaN throughout, and p=1 512k elements 161 us
+// against 162, p=4 8M DoFs 242.0 against 242.6).
+__device__ __forceinline__ double geo_div(double w, double x) {
   double r = __builtin_amdgcn_rcp(x);
   r        = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
-  return __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+  r        = __builtin_fma(__builtin_fma(-x, r, 1.0), r, r);
+  return __builtin_amdgcn_div_fixup(w * r, x, w);
 }
 
 // w (d/dxi x d/deta) . d/dzeta = w det J  (Mass3DBuild)
@@ -76,7 +82,7 @@ __device__ __forceinline__ void geo_poisson(const double (&a)[3], const double (
   geo_cross(b, c, A0);
   geo_cross(c, a, A1);
   geo_cross(a, b, A2);
-  const double qw = w * geo_rcp(geo_dot(a, A0));
+  const double qw = geo_div(w, geo_dot(a, A0));
   s[0] = qw * geo_dot(A0, A0);
   s[1] = qw * geo_dot(A1, A1);
   s[2] = qw * geo_dot(A2, A2);
