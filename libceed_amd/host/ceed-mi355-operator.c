@@ -34,14 +34,6 @@
 
 #include "ceed-mi355-backend.h"
 
-/* A kernel library without these entry points leaves their operators on the
- * generic path. */
-#pragma weak CeedMi355OperatorCreateHexJitFields
-#pragma weak CeedMi355OperatorSetQDataComponents
-#pragma weak CeedMi355PointOperatorCreate
-#pragma weak CeedMi355PointOperatorApply
-#pragma weak CeedMi355PointOperatorDestroy
-
 typedef struct {
   bool     is_set_up, fused, jit;
   /* fused path */
@@ -61,6 +53,17 @@ typedef struct {
   bool     in_valid[CEED_FIELD_MAX];
 } OperatorData;
 
+/* Whether a restriction has the backend's strides; libCEED answers
+ * CeedElemRestrictionHasBackendStrides for strided restrictions only and
+ * raises an error for the others. */
+static int has_backend_strides(CeedElemRestriction rstr, bool *backend) {
+  CeedRestrictionType type;
+  *backend = false;
+  CeedCallBackend(CeedElemRestrictionGetType(rstr, &type));
+  if (type == CEED_RESTRICTION_STRIDED) CeedCallBackend(CeedElemRestrictionHasBackendStrides(rstr, backend));
+  return CEED_ERROR_SUCCESS;
+}
+
 /* E-vector of qdata in [elem][comp][qpt]: the field's L-vector itself when its
  * restriction has the backend strides, else a temporary restricted copy. */
 static int qdata_evector(Ceed ceed, CeedElemRestriction rstr, CeedVector vec, const double **e, double **temp) {
@@ -68,7 +71,7 @@ static int qdata_evector(Ceed ceed, CeedElemRestriction rstr, CeedVector vec, co
   CeedScalar *dl;
   *temp = NULL;
   CeedCallBackend(CeedMi355VectorDevice(vec, false, &dl));
-  CeedCallBackend(CeedElemRestrictionHasBackendStrides(rstr, &backend));
+  CeedCallBackend(has_backend_strides(rstr, &backend));
   if (backend) {
     *e = dl;
     return CEED_ERROR_SUCCESS;
@@ -280,7 +283,6 @@ static int try_fused_jit(CeedOperator op, OperatorData *d) {
       ok = q_elem == Q * Q * Q && q_nc == d->passive_size[k] && q_ne == num_elem;
       CeedCallBackend(CeedElemRestrictionDestroy(&rq));
     }
-    if (num_passive > 1 && !(CeedMi355OperatorCreateHexJitFields && CeedMi355OperatorSetQDataComponents)) ok = 0;
     if (ok) {
       const CeedScalar *interp, *grad;
       const CeedInt    *offsets;
@@ -367,8 +369,7 @@ static int try_points(CeedOperator op, OperatorData *d) {
   int32_t             in_kinds[CEED_FIELD_MAX], in_sizes[CEED_FIELD_MAX];
   bool                ok;
 
-  if ((env && !strcmp(env, "0")) || !CeedMi355PointOperatorCreate || !CeedMi355PointOperatorApply || !CeedMi355PointOperatorDestroy)
-    return CEED_ERROR_SUCCESS;
+  if (env && !strcmp(env, "0")) return CEED_ERROR_SUCCESS;
   CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
   CeedCallBackend(CeedOperatorGetQFunction(op, &qf));
   CeedCallBackend(CeedQFunctionGetSourcePath(qf, &path));
@@ -393,7 +394,7 @@ static int try_points(CeedOperator op, OperatorData *d) {
     CeedCallBackend(CeedQFunctionFieldGetEvalMode(is_in ? qf_in[i] : qf_out[i], &mode));
     CeedCallBackend(CeedQFunctionFieldGetSize(is_in ? qf_in[i] : qf_out[i], &size));
     if (rstr != CEED_ELEMRESTRICTION_NONE) {
-      CeedCallBackend(CeedElemRestrictionHasBackendStrides(rstr, &backend));
+      CeedCallBackend(has_backend_strides(rstr, &backend));
       CeedCallBackend(CeedElemRestrictionGetElementSize(rstr, &elem_size));
       CeedCallBackend(CeedElemRestrictionGetNumComponents(rstr, &rstr_comp));
     }

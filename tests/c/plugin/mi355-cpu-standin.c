@@ -5,9 +5,11 @@
  * arithmetic is the oracle's (oracle/ceed_oracle.c, the restatement of
  * /cpu/self/ref/serial); user QFunctions are compiled from their source file
  * with the host C compiler and loaded with dlopen, where the real library
- * compiles them with hipRTC.  Run-time fused kernels (CeedMi355OperatorCreateHexJit)
- * report CEED_MI355_ERROR_UNSUPPORTED, so operators with user QFunctions take
- * the backend's staged path, which the stand-in covers call by call.
+ * compiles them with hipRTC.  Run-time fused kernels
+ * (CeedMi355OperatorCreateHexJit, ...JitFields) report
+ * CEED_MI355_ERROR_UNSUPPORTED, so operators with user QFunctions take the
+ * backend's staged path, which the stand-in covers call by call; operators
+ * whose output stays at the quadrature points run (CeedMi355PointOperator).
  *
  * STANDIN_CEED_INCLUDE names the directory holding ceed/types.h for the
  * QFunction compiles; STANDIN_LOG (optional) receives one line per entry
@@ -308,6 +310,22 @@ int CeedMi355OperatorCreateHexJit(const char *source_path, const char *function_
   return fail(CEED_MI355_ERROR_UNSUPPORTED, "the stand-in has no run-time fused kernels");
 }
 
+int CeedMi355OperatorCreateHexJitFields(const char *source_path, const char *function_name, int32_t num_in, const int32_t *in_kinds_host,
+                                        const int32_t *in_sizes_host, int32_t num_out, const int32_t *out_kinds_host, int32_t num_elem,
+                                        int32_t P_1d, int32_t Q_1d, const double *interp_1d_host, const double *grad_1d_host,
+                                        const int32_t *offsets_host, int64_t l_size, int flags, CeedMi355Operator *op) {
+  (void)source_path, (void)function_name, (void)num_in, (void)in_kinds_host, (void)in_sizes_host, (void)num_out, (void)out_kinds_host;
+  (void)num_elem, (void)P_1d, (void)Q_1d, (void)interp_1d_host, (void)grad_1d_host, (void)offsets_host, (void)l_size, (void)flags;
+  trace("OperatorCreateHexJitFields");
+  *op = NULL;
+  return fail(CEED_MI355_ERROR_UNSUPPORTED, "the stand-in has no run-time fused kernels");
+}
+
+int CeedMi355OperatorSetQDataComponents(CeedMi355Operator op, int32_t first, int32_t num, const void *q_data, void *stream) {
+  (void)op, (void)first, (void)num, (void)q_data, (void)stream;
+  return fail(CEED_MI355_ERROR_UNSUPPORTED, "the stand-in has no run-time fused kernels");
+}
+
 int CeedMi355OperatorSetContext(CeedMi355Operator op, void *ctx_device) {
   (void)op, (void)ctx_device;
   return CEED_MI355_SUCCESS;
@@ -359,5 +377,81 @@ int CeedMi355OperatorDestroy(CeedMi355Operator *op) {
   if (*op) free((*op)->offsets), free((*op)->interp), free((*op)->grad), free((*op)->q_weight), free((*op)->q_data);
   free(*op);
   *op = NULL;
+  return CEED_MI355_SUCCESS;
+}
+
+/* ---- values at the quadrature points, element by element ----------------- */
+struct CeedMi355PointOperator_private {
+  CeedMi355QFunction qf;
+  int                num_in, kinds[16], sizes[16], out_size, num_comp, num_elem, P, Q, comp_stride;
+  int32_t           *offsets;
+  double            *interp, *grad, *q_weight;
+};
+
+int CeedMi355PointOperatorCreate(const char *source_path, const char *function_name, int32_t num_in, const int32_t *in_kinds_host,
+                                 const int32_t *in_sizes_host, int32_t out_size, int32_t num_comp, int32_t num_elem, int32_t P_1d, int32_t Q_1d,
+                                 const double *interp_1d_host, const double *grad_1d_host, const double *q_weight_1d_host,
+                                 const int32_t *offsets_host, int32_t comp_stride, int64_t l_size, CeedMi355PointOperator *op) {
+  (void)l_size;
+  trace("PointOperatorCreate");
+  *op = NULL;
+  CeedMi355PointOperator o    = calloc(1, sizeof(*o));
+  const int32_t          outs = out_size;
+  const int              ierr = CeedMi355QFunctionCompile(source_path, function_name, num_in, in_sizes_host, 1, &outs, &o->qf);
+  if (ierr) {
+    free(o);
+    return ierr;
+  }
+  const size_t es = (size_t)P_1d * P_1d * P_1d;
+  o->num_in = num_in, o->out_size = out_size, o->num_comp = num_comp, o->num_elem = num_elem, o->P = P_1d, o->Q = Q_1d, o->comp_stride = comp_stride;
+  for (int i = 0; i < num_in; i++) o->kinds[i] = in_kinds_host[i], o->sizes[i] = in_sizes_host[i];
+  o->offsets = malloc(sizeof(int32_t) * (num_elem * es + 1));
+  memcpy(o->offsets, offsets_host, sizeof(int32_t) * num_elem * es);
+  o->interp   = malloc(sizeof(double) * P_1d * Q_1d);
+  o->grad     = malloc(sizeof(double) * P_1d * Q_1d);
+  o->q_weight = calloc(Q_1d, sizeof(double));
+  memcpy(o->interp, interp_1d_host, sizeof(double) * P_1d * Q_1d);
+  memcpy(o->grad, grad_1d_host, sizeof(double) * P_1d * Q_1d);
+  if (q_weight_1d_host) memcpy(o->q_weight, q_weight_1d_host, sizeof(double) * Q_1d);
+  *op = o;
+  return CEED_MI355_SUCCESS;
+}
+
+int CeedMi355PointOperatorApply(CeedMi355PointOperator op, void *ctx_device, const double *u, const double *const *passive_host, double *v, int add,
+                                void *stream) {
+  (void)stream;
+  trace("PointOperatorApply");
+  const int nq = op->Q * op->Q * op->Q, es = op->P * op->P * op->P, nc = op->num_comp;
+  double   *e_u = malloc(sizeof(double) * es * nc), *res = malloc(sizeof(double) * op->out_size * nq), *buf[16] = {NULL};
+  int       ierr = CEED_MI355_SUCCESS;
+  for (int i = 0; i < op->num_in; i++) buf[i] = malloc(sizeof(double) * op->sizes[i] * nq);
+  for (int e = 0; e < op->num_elem && !ierr; e++) {
+    const double *in[16];
+    double       *out[1] = {res};
+    orc_restriction_offset(1, es, nc, op->comp_stride, op->offsets + (size_t)e * es, 0, u, e_u);
+    for (int i = 0, p = 0; i < op->num_in; i++) {
+      in[i] = buf[i];
+      if (op->kinds[i] == CEED_MI355_FIELD_PASSIVE) memcpy(buf[i], passive_host[p++] + (size_t)e * op->sizes[i] * nq, sizeof(double) * op->sizes[i] * nq);
+      else if (orc_basis_apply(3, op->kinds[i] == CEED_MI355_FIELD_WEIGHT ? 1 : nc, op->P, op->Q, op->interp, op->grad, op->q_weight, 1, 0,
+                               op->kinds[i] == CEED_MI355_FIELD_WEIGHT ? ORC_EVAL_WEIGHT : op->kinds[i] == CEED_MI355_FIELD_GRAD ? ORC_EVAL_GRAD : ORC_EVAL_INTERP,
+                               0, op->kinds[i] == CEED_MI355_FIELD_WEIGHT ? NULL : e_u, buf[i]))
+        ierr = fail(CEED_MI355_ERROR_BACKEND, "basis apply failed");
+    }
+    if (!ierr && op->qf->f(ctx_device, nq, in, out)) ierr = fail(CEED_MI355_ERROR_BACKEND, "QFunction returned an error");
+    double *dst = v + (size_t)e * op->out_size * nq;
+    for (int k = 0; k < op->out_size * nq && !ierr; k++) dst[k] = add ? dst[k] + res[k] : res[k];
+  }
+  for (int i = 0; i < op->num_in; i++) free(buf[i]);
+  free(e_u), free(res);
+  return ierr;
+}
+
+int CeedMi355PointOperatorDestroy(CeedMi355PointOperator *op) {
+  if (op && *op) {
+    CeedMi355QFunctionDestroy(&(*op)->qf);
+    free((*op)->offsets), free((*op)->interp), free((*op)->grad), free((*op)->q_weight);
+    free(*op);
+    *op = NULL;
+  }
   return CEED_MI355_SUCCESS;
 }
