@@ -295,7 +295,10 @@ static int try_fused_jit(CeedOperator op, OperatorData *d) {
                                  : CeedMi355OperatorCreateHexJit(path, name, num_in, in_kinds, num_out, out_kinds, q_comp, num_elem, P, Q, interp,
                                                                  grad, offsets, d->l_size, 0, &d->hex);
       CeedCallBackend(CeedElemRestrictionRestoreOffsets(ru, &offsets));
-      if (ierr == CEED_MI355_ERROR_UNSUPPORTED) ok = 0;
+      /* a QFunction that does not compile within the fused kernel (a macro of
+       * its source named like something there) may still compile by itself:
+       * the staged path, which reports what is wrong where it is not that */
+      if (ierr == CEED_MI355_ERROR_UNSUPPORTED || ierr == CEED_MI355_ERROR_BACKEND) ok = 0;
       else CeedCallBackend(CeedMi355Check(ceed, ierr));
     }
   } else {
@@ -456,7 +459,8 @@ static int try_points(CeedOperator op, OperatorData *d) {
       const int ierr = CeedMi355PointOperatorCreate(path, name, num_in, in_kinds, in_sizes, out_size, num_comp, num_elem, P, Q, interp, grad, weights,
                                                     offsets, comp_stride, l_size, &d->points);
       CeedCallBackend(CeedElemRestrictionRestoreOffsets(ru, &offsets));
-      if (ierr != CEED_MI355_ERROR_UNSUPPORTED) CeedCallBackend(CeedMi355Check(ceed, ierr));
+      /* (as for fused plans: where it does not compile, the staged path) */
+      if (ierr != CEED_MI355_ERROR_UNSUPPORTED && ierr != CEED_MI355_ERROR_BACKEND) CeedCallBackend(CeedMi355Check(ceed, ierr));
     }
   }
   d->num_passive = num_passive;
