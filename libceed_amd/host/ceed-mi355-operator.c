@@ -41,10 +41,13 @@ typedef struct {
   CeedSize          l_size;
   CeedInt           num_passive; /* passive inputs held in the plan: their fields, in order, and sizes */
   CeedInt           passive_field[CEED_FIELD_MAX], passive_size[CEED_FIELD_MAX];
+  uint64_t          passive_state[CEED_FIELD_MAX];
+  bool              passive_valid[CEED_FIELD_MAX];
   /* values at the quadrature points (CeedMi355PointOperator) */
   CeedMi355PointOperator points;
   CeedSize               points_size; /* E-vector length of the output */
   /* generic path */
+  bool     is_staged; /* generic_setup has run */
   CeedInt  num_in, num_out, num_elem, Q;
   double  *e_in[CEED_FIELD_MAX], *q_in[CEED_FIELD_MAX];
   double  *e_out[CEED_FIELD_MAX], *q_out[CEED_FIELD_MAX];
@@ -335,7 +338,7 @@ static int fused_sync_qdata(CeedOperator op, OperatorData *d) {
     uint64_t            state;
     CeedCallBackend(CeedOperatorFieldGetVector(in[d->passive_field[k]], &vq));
     CeedCallBackend(CeedVectorGetState(vq, &state));
-    if (!d->in_valid[k] || state != d->in_state[k]) {
+    if (!d->passive_valid[k] || state != d->passive_state[k]) {
       const double *e;
       double       *temp;
       CeedCallBackend(CeedOperatorFieldGetElemRestriction(in[d->passive_field[k]], &rq));
@@ -344,8 +347,8 @@ static int fused_sync_qdata(CeedOperator op, OperatorData *d) {
       else CeedCallBackend(CeedMi355Check(ceed, CeedMi355OperatorSetQData(d->hex, e, NULL)));
       if (temp) CeedMi355Free(temp);
       CeedCallBackend(CeedElemRestrictionDestroy(&rq));
-      d->in_state[k] = state;
-      d->in_valid[k] = true;
+      d->passive_state[k] = state;
+      d->passive_valid[k] = true;
     }
     CeedCallBackend(CeedVectorDestroy(&vq));
   }
@@ -522,6 +525,7 @@ static int generic_setup(CeedOperator op, OperatorData *d) {
   CeedInt            num_in, num_out;
   CeedOperatorField *in, *out;
   CeedQFunctionField *qf_in, *qf_out;
+  if (d->is_staged) return CEED_ERROR_SUCCESS;
   CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
   CeedCallBackend(CeedOperatorGetQFunction(op, &qf));
   CeedCallBackend(CeedOperatorGetFields(op, &num_in, &in, &num_out, &out));
@@ -563,6 +567,7 @@ static int generic_setup(CeedOperator op, OperatorData *d) {
     CeedCallBackend(CeedElemRestrictionDestroy(&rstr));
     CeedCallBackend(CeedBasisDestroy(&basis));
   }
+  d->is_staged = true;
   CeedCallBackend(CeedQFunctionDestroy(&qf));
   CeedCallBackend(CeedDestroy(&ceed));
   return CEED_ERROR_SUCCESS;
@@ -670,14 +675,35 @@ static int setup(CeedOperator op, OperatorData *d) {
   return CEED_ERROR_SUCCESS;
 }
 
+/* Whether this apply is staged: no kernel has the operator's shape, or (values
+ * at the quadrature points, several passive fields) the output is also an
+ * input, all of which the staged path reads before it writes. */
+static int runs_staged(CeedOperator op, OperatorData *d, CeedVector in, CeedVector out, bool *staged) {
+  CeedOperatorField *fields;
+  *staged = !d->fused && !d->points;
+  if (*staged || (!d->points && d->num_passive < 2)) return CEED_ERROR_SUCCESS;
+  *staged = out == CEED_VECTOR_NONE || out == in;
+  CeedCallBackend(CeedOperatorGetFields(op, NULL, &fields, NULL, NULL));
+  for (CeedInt k = 0; !*staged && k < d->num_passive; k++) {
+    CeedVector vec;
+    CeedCallBackend(CeedOperatorFieldGetVector(fields[d->passive_field[k]], &vec));
+    *staged = vec == out;
+    CeedCallBackend(CeedVectorDestroy(&vec));
+  }
+  if (*staged) CeedCallBackend(generic_setup(op, d));
+  return CEED_ERROR_SUCCESS;
+}
+
 static int OperatorApplyAdd(CeedOperator op, CeedVector in, CeedVector out, CeedRequest *request) {
   OperatorData *d;
   Ceed          ceed;
+  bool          staged;
   (void)request;
   CeedCallBackend(CeedOperatorGetData(op, &d));
   CeedCallBackend(setup(op, d));
-  if (d->points && out != CEED_VECTOR_NONE) return points_apply(op, d, in, out, true);
-  if (!d->fused) return generic_apply_add(op, d, in, out);
+  CeedCallBackend(runs_staged(op, d, in, out, &staged));
+  if (staged) return generic_apply_add(op, d, in, out);
+  if (d->points) return points_apply(op, d, in, out, true);
   CeedScalar *du, *dv;
   CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
   CeedCallBackend(fused_sync_qdata(op, d));
@@ -693,13 +719,15 @@ static int OperatorApply(CeedOperator op, CeedVector in, CeedVector out, CeedReq
   OperatorData *d;
   Ceed          ceed;
   CeedSize      out_len;
+  bool          staged;
   CeedCallBackend(CeedOperatorGetData(op, &d));
   CeedCallBackend(setup(op, d));
+  CeedCallBackend(runs_staged(op, d, in, out, &staged));
   if (out != CEED_VECTOR_NONE) CeedCallBackend(CeedVectorGetLength(out, &out_len));
-  if (d->points && out != CEED_VECTOR_NONE && out_len == d->points_size) return points_apply(op, d, in, out, false);
+  if (d->points && !staged && out_len == d->points_size) return points_apply(op, d, in, out, false);
   /* the fused plan overwrites its whole L-vector; a longer output (or the
    * generic path) is zeroed first and accumulated into */
-  if (!d->fused || out == CEED_VECTOR_NONE || out_len != d->l_size) {
+  if (staged || d->points || out == CEED_VECTOR_NONE || out_len != d->l_size) {
     if (out != CEED_VECTOR_NONE) CeedCallBackend(CeedVectorSetValue(out, 0.0));
     return OperatorApplyAdd(op, in, out, request);
   }

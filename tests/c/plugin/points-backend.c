@@ -7,8 +7,9 @@
  * The operators are those of tests/qfunctions/t-points.h on two trilinear
  * hexes: values at the quadrature points (mixed_at_points_3), and a nodal
  * result with three passive fields, one of them on an offset restriction
- * (three_passive).  Usage: points-backend <t-points.h>; prints the sums of
- * Apply and of ApplyAdd of each.
+ * (three_passive); each also with an output that is one of its inputs.
+ * Usage: points-backend <t-points.h>; prints the sums of Apply and of ApplyAdd
+ * of each.
  */
 #include <ceed.h>
 #include <ceed/backend.h>
@@ -128,6 +129,7 @@ int main(int argc, char **argv) {
     CHECK(CeedOperatorSetField(op, "g", rg, CEED_BASIS_NONE, g));
     CHECK(CeedOperatorSetField(op, "out", rf, CEED_BASIS_NONE, CEED_VECTOR_ACTIVE));
     apply_both("points", op, u, out);
+    apply_both("points-in-place", op, u, f); /* the output is also a passive input */
     CHECK(CeedOperatorDestroy(&op));
     CHECK(CeedQFunctionContextDestroy(&ctx));
     CHECK(CeedQFunctionDestroy(&qf));
@@ -166,6 +168,7 @@ int main(int argc, char **argv) {
     CHECK(CeedOperatorSetField(op, "dv", ru, basis, CEED_VECTOR_ACTIVE));
     CHECK(CeedOperatorSetField(op, "v", ru, basis, CEED_VECTOR_ACTIVE));
     apply_both("passive", op, u, out);
+    apply_both("passive-in-place", op, out, out);
     CHECK(CeedOperatorDestroy(&op));
     CHECK(CeedQFunctionDestroy(&qf));
     CHECK(CeedBasisDestroy(&basis));

@@ -39,6 +39,6 @@ def test_paths_agree(program, tmp_path):
     staged, staged_calls = run(program, tmp_path, CEED_MI355_FUSE_QFUNCTIONS="0")
     assert "PointOperatorApply" in fused_calls and "OperatorCreateHexJitFields" in fused_calls
     assert "PointOperatorCreate" not in staged_calls and "OperatorCreateHexJitFields" not in staged_calls
-    assert fused.keys() == staged.keys() and len(fused) == 4
+    assert fused.keys() == staged.keys() and len(fused) == 8
     for k in fused:  # sums of at most 108 values of either path, formed in the same order but for the fused contractions
         assert fused[k] == pytest.approx(staged[k], rel=1e-13), k
