@@ -67,8 +67,8 @@ def time_gpu(fn, steps: int, warmup: int):
 
 
 LAYOUT_NAMES = ["columns", "lines", "points"]  # the fused kernel's thread layouts, by their index in the library
-# (order 1 on many elements: hex_apply_elements_kernel in the lines' place)
-KERNEL_OF_LAYOUT = ["hex_apply_kernel", "hex_apply_lines_kernel", "hex_apply_points_kernel"]
+KERNEL_NAMES = {"columns": "hex_apply_kernel", "lines": "hex_apply_lines_kernel", "points": "hex_apply_points_kernel",
+                "elements": "hex_apply_elements_kernel", "brick": "hex_apply_brick_kernel"}
 
 
 def run_case(p: int, dofs: float, dtype, steps: int, warmup: int, seed: int = 0, scatter: str = "auto", epb: int = 0, num_comp: int = 1,
@@ -98,11 +98,13 @@ def run_case(p: int, dofs: float, dtype, steps: int, warmup: int, seed: int = 0,
     mode = {"tmap": "transpose map", "color": "element colours", "split": "multiplicity split", "atomic": "atomics",
             "brick": "element bricks", "segment": "element segments"}[op.scatter_mode()]
     F = alg_flops(m.num_elem, P, Q, ncomp=num_comp)
-    kname = KERNEL_OF_LAYOUT[layout]
+    kernel, gather = op.kernel()
+    kname = KERNEL_NAMES[kernel]
     res = {
         "p": p, "n": n, "dofs": num_comp * m.num_nodes, "num_comp": num_comp, "elements": m.num_elem,
-        "scatter": mode, "layout": LAYOUT_NAMES[layout], "elems_per_block": epb,
-        "kernels": {"transpose map": f"one apply = {kname} + transpose_gather_kernel (E^T by the transpose offset map)",
+        "scatter": mode, "layout": LAYOUT_NAMES[layout], "elems_per_block": epb, "kernel": kernel,
+        "kernels": {"transpose map": f"one apply = {kname} + transpose_gather_kernel (E^T by the transpose offset map)" if gather else
+                    f"one apply = {kname} (E^T by the transpose offset map, summed by the last contribution to arrive)",
                     "multiplicity split": f"one apply = zero fill + {kname} + split_gather_kernel (E^T: atomic adds for entries of "
                                           "at most two contributions, the ordered transpose map for the rest)",
                     "atomics": f"one apply = zero fill + {kname} (E^T by atomic adds)",

@@ -241,6 +241,20 @@ int CeedMi355OperatorSetLaunch(CeedMi355Operator op, int32_t elems_per_block);
 int CeedMi355OperatorSetLayout(CeedMi355Operator op, int32_t layout, int32_t elems_per_block);
 /* Current thread layout and elements per workgroup (either pointer may be NULL). */
 int CeedMi355OperatorGetLaunch(CeedMi355Operator op, int32_t *layout, int32_t *elems_per_block);
+/* The kernel Apply runs with the current launch, and whether E^T is finished by
+ * a launch of its own after it (either pointer may be NULL): that of the
+ * thread layout, the brick plans', or one thread per element, which takes the
+ * line layout's place for recomputed diffusion factors at P_1d = 2 on many
+ * elements of a launch (of several, the largest counts here) unless the caller
+ * has set the elements per workgroup. */
+enum {
+  CEED_MI355_KERNEL_COLUMNS  = 0,
+  CEED_MI355_KERNEL_LINES    = 1,
+  CEED_MI355_KERNEL_POINTS   = 2,
+  CEED_MI355_KERNEL_ELEMENTS = 3,
+  CEED_MI355_KERNEL_BRICK    = 4
+};
+int CeedMi355OperatorGetKernel(CeedMi355Operator op, int32_t *kernel, int32_t *gather);
 /* 1 if Apply recomputes the geometric factors from the elements' trilinear
  * maps with the current launch (it then reads 168 bytes per element of them),
  * 0 if it reads the stored ones. */

@@ -38,6 +38,14 @@ int CeedRegister_Mi355(void);
  * counterpart of CeedInit_Hip_ref (backends/hip-ref/ceed-hip-ref.c:43-73). */
 int CeedInit_Mi355(const char *resource, Ceed ceed);
 
+/* The path the applies of a (not composite) operator of this backend take:
+ * "fused" (a gallery operator's plan), "fused-qfunction" (a plan with the
+ * QFunction compiled into it at run time), "points" (one run-time compiled
+ * kernel for values at the quadrature points) or "staged" (restriction, basis
+ * and QFunction kernels one after the other).  Compiles what is not compiled
+ * yet.  An apply whose output is one of its inputs may still run staged. */
+int CeedMi355OperatorGetPath(CeedOperator op, const char **path);
+
 #ifdef __cplusplus
 }
 #endif

@@ -41,6 +41,7 @@ SIGNATURES = {
     "CeedMi355PointOperatorApply": (c_int, [vp, vp, vp, vp, vp, c_int, vp]),
     "CeedMi355PointOperatorDestroy": (c_int, [C.POINTER(vp)]),
     "CeedMi355OperatorSetContext": (c_int, [vp, vp]),
+    "CeedMi355OperatorGetPath": (c_int, [vp, C.POINTER(C.c_char_p)]),
     "CeedMi355OperatorBuildQData": (c_int, [vp, c_int, c_i32, vp, vp, vp, vp, c_i32, vp, vp]),
     "CeedMi355OperatorSetQData": (c_int, [vp, vp, vp]),
     "CeedMi355OperatorGetQData": (c_int, [vp, vp, vp]),
@@ -79,6 +80,7 @@ SIGNATURES = {
     "CeedMi355OperatorSetLayout": (c_int, [vp, c_i32, c_i32]),
     "CeedMi355OperatorRecomputesFactors": (c_int, [vp, vp]),
     "CeedMi355OperatorGetLaunch": (c_int, [vp, vp, vp]),
+    "CeedMi355OperatorGetKernel": (c_int, [vp, vp, vp]),
     "CeedRegister_Mi355": (c_int, []),
     "CeedInit_Mi355": (c_int, [C.c_char_p, vp]),
 }

@@ -573,6 +573,12 @@ class Operator(_Object):
     def check(self):
         self._ceed._call("CeedOperatorCheckReady", self._pointer)
 
+    def path(self) -> str:
+        """What its applies run: "fused", "fused-qfunction", "points" or "staged" (CeedMi355OperatorGetPath)."""
+        path = C.c_char_p()
+        self._ceed._call("CeedMi355OperatorGetPath", self._pointer, C.byref(path))
+        return path.value.decode()
+
     def apply(self, u, v):
         up = VECTOR_NONE._pointer if u is None else u._pointer
         self._ceed._call("CeedOperatorApply", self._pointer, up, v._pointer, None)

@@ -25,10 +25,7 @@ namespace mi355 {
 // 12.2, 125k 17.2 / 15.0; FP32 Q=3 74k 17.5 / 19.7, 125k 25.9 / 23.2; eight
 // colours, each a launch: FP64 Q=3 71k each 133 / 139, 121k each 202 / 164, and
 // FP64 Q=2 23k each 51 / 50, 47k each 77 / 60.
-template <int Q, typename T>
-constexpr int64_t elements_min() {
-  return Q == 2 && sizeof(T) == 8 ? 32768 : 98304;
-}
+constexpr int64_t elements_min(int Q, int sb) { return Q == 2 && sb == 8 ? 32768 : 98304; }
 constexpr int kElemThreads = 64;
 constexpr int kElemGeo     = kGeoStride + 1;  // an odd stride in LDS
 

@@ -137,6 +137,7 @@ struct CeedMi355Operator_private {
   int     epb;
   int     layout     = 0;      // mi355::kLayoutColumns or kLayoutLines
   bool    own_launch = false;  // layout and epb were set by the caller or the environment: kept when the factors change kind
+  bool    line_only  = false;  // the line kernel also where one thread per element would take a launch (hex_elements.hpp): the caller set its count, or the autotuner found it faster
   bool    covers_all = false;  // every L entry is reached by some element: Apply needs no zero fill
   int     scatter    = 0;      // CEED_MI355_PLAN_* E^T mode: 0 transpose map, COLOR, SPLIT, ATOMIC, BRICK, SEGMENT
   // transpose offset map (scatter == 0): contribution (elem, comp, node) is
@@ -219,6 +220,16 @@ inline bool plan_recomputes(const CeedMi355Operator_private *op) {
          line_lds_bytes(op->Q, op->num_comp, op->qf, op->scalar_bytes, true, op->epb) <= (size_t)kMaxLdsBytes;
 }
 
+// A launch over n elements takes one thread per element (hex_elements.hpp)
+inline bool elements_take(const CeedMi355Operator_private *op, int64_t n) {
+  return op->P == 2 && op->num_comp == 1 && op->qf == kQfDiffusion && !op->line_only && n >= elements_min(op->Q, op->scalar_bytes);
+}
+
+// The plan's E^T is summed in the apply's own launch (line_last)
+inline bool plan_sums_last(const CeedMi355Operator_private *op) {
+  return op->scatter == 0 && op->layout == kLayoutLines && op->d_tcount && (op->num_elem + op->epb - 1) / op->epb <= kLastWorkgroups && !op->d_elem_sys;
+}
+
 template <int P, int Q, int NC, int QF, typename T>
 int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s) {
   const int    nt     = Q * Q;
@@ -263,7 +274,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
   // kScatterLast: frozen systems' contributions never arrive, a dot product
   // wants the gather, and where u and v overlap all of u is read first
   const size_t l_bytes = sizeof(T) * (size_t)op->l_size;
-  const bool   last    = tmap && lines && op->d_tcount && (op->num_elem + epb - 1) / epb <= kLastWorkgroups && !op->d_elem_sys && !gather_dot_wanted() &&
+  const bool   last    = plan_sums_last(op) && !gather_dot_wanted() &&
                     ((const char *)u + l_bytes <= (const char *)v || (const char *)v + l_bytes <= (const char *)u);
   for (size_t c = 0; c + 1 < op->color_start.size(); c++) {
     const int64_t b = op->color_start[c], e = op->color_start[c + 1];
@@ -306,7 +317,7 @@ void launch_geo_lines(const CeedMi355Operator_private *op, int64_t b, int64_t e,
                       bool two, hipStream_t s) {
   const int32_t *elem_sys = two ? op->d_geo_turn : op->d_elem_sys, *sys_active = two ? op->d_geo_turn : op->d_sys_active;
   if constexpr (P == 2 && NC == 1 && QF == kQfDiffusion) {
-    if (scatter < kScatterLast && e - b >= elements_min<Q, T>()) {
+    if (scatter < kScatterLast && elements_take(op, e - b)) {
       hex_apply_elements_kernel<P, Q, T><<<(unsigned)((e - b + kElemThreads - 1) / kElemThreads), kElemThreads, 0, s>>>(
           b, e, scatter, op->d_offsets, (const T *)op->d_mats, (const T *)u, (T *)v, (T *)op->d_evec, op->d_tpos, elem_sys, sys_active, op->d_geo,
           op->d_geo_pts);

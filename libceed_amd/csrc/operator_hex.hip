@@ -335,22 +335,26 @@ int color_elements(const int32_t *offsets, int64_t num_elem, int es, int nc, int
   return CEED_MI355_SUCCESS;
 }
 
-// Autotuner results: (thread layout, elements per workgroup) by (P, Q,
-// num_comp, pointwise operator, scalar type, E^T mode, recomputed factors).
-std::mutex                                                          g_tune_mutex;
-std::map<std::tuple<int, int, int, int, int, int, bool>, std::pair<int, int>> g_tuned;
+// Autotuner results by (P, Q, num_comp, pointwise operator, scalar type, E^T
+// mode, recomputed factors).
+struct Launch {
+  int  layout, epb;
+  bool line_only;
+};
+std::mutex                                                       g_tune_mutex;
+std::map<std::tuple<int, int, int, int, int, int, bool>, Launch> g_tuned;
 
 std::tuple<int, int, int, int, int, int, bool> tune_key(const CeedMi355Operator op) {
   return std::make_tuple(op->P, op->Q, op->num_comp, op->qf, op->scalar_type, op->scatter, op->geo_valid);
 }
 
-bool tuned_launch(const CeedMi355Operator op, int *layout, int *epb) {
+void set_launch(CeedMi355Operator op, const Launch &l) { op->layout = l.layout, op->epb = l.epb, op->line_only = l.line_only; }
+
+// Take the autotuner's launch for plans of this kind, if there is one
+void tuned_launch(CeedMi355Operator op) {
   std::lock_guard<std::mutex> lock(g_tune_mutex);
   auto                        it = g_tuned.find(tune_key(op));
-  if (it == g_tuned.end()) return false;
-  *layout = it->second.first;
-  *epb    = it->second.second;
-  return true;
+  if (it != g_tuned.end()) set_launch(op, it->second);
 }
 
 // A known layout the plan's kernels exist in (run-time compiled QFunctions:
@@ -383,10 +387,10 @@ void set_geo_valid(CeedMi355Operator op, bool valid) {
   if (op->geo_valid == valid) return;
   op->geo_valid = valid;
   if (op->own_launch || op->scatter == CEED_MI355_PLAN_SEGMENT) return;
-  op->layout = mi355::kLayoutLines;
-  op->epb    = plan_default_epb(op, op->layout);
-  int layout, epb;
-  if (tuned_launch(op, &layout, &epb)) op->layout = layout, op->epb = epb;
+  op->layout    = mi355::kLayoutLines;
+  op->epb       = plan_default_epb(op, op->layout);
+  op->line_only = false;
+  tuned_launch(op);
 }
 
 // A launch the plan can take: segment plans have one (the line layout with an
@@ -707,10 +711,7 @@ int mi355::create_plan(int qf, int scalar_type, int32_t num_comp, int32_t num_el
   // with its default workgroup size; CEED_MI355_LAYOUT / CEED_MI355_EPB override
   op->layout = mi355::kLayoutLines;
   op->epb    = plan_default_epb(op, op->layout);
-  {
-    int layout, epb;
-    if (tuned_launch(op, &layout, &epb)) op->layout = layout, op->epb = epb;
-  }
+  tuned_launch(op);
   if (const char *env = getenv("CEED_MI355_LAYOUT")) {
     const int l = atoi(env);
     if (layout_exists(Q_1d, qf, l)) op->own_launch = true, op->layout = l, op->epb = mi355::default_epb(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, l);
@@ -719,7 +720,7 @@ int mi355::create_plan(int qf, int scalar_type, int32_t num_comp, int32_t num_el
     op->layout = mi355::kLayoutLines, op->epb = mi355::default_epb(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, op->layout);
   if (const char *env = getenv("CEED_MI355_EPB")) {
     const int v = atoi(env);
-    if (admissible(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, op->layout, v)) op->own_launch = true, op->epb = v;
+    if (admissible(P_1d, Q_1d, qf, num_comp, op->scalar_bytes, op->layout, v)) op->own_launch = op->line_only = true, op->epb = v;
   }
 
   const int            es = P_1d * P_1d * P_1d;
@@ -1109,7 +1110,7 @@ extern "C" int CeedMi355OperatorSetLaunch(CeedMi355Operator op, int32_t elems_pe
   MI355_CHECK(plan_admissible(op, op->layout, elems_per_block), CEED_MI355_ERROR_BACKEND,
               "%d elements per workgroup do not fit (at most 256 threads and 160 KiB of LDS for P=%d Q=%d)", elems_per_block, op->P, op->Q);
   op->epb        = elems_per_block;
-  op->own_launch = true;
+  op->own_launch = op->line_only = true;
   return CEED_MI355_SUCCESS;
 }
 
@@ -1128,6 +1129,7 @@ extern "C" int CeedMi355OperatorSetLayout(CeedMi355Operator op, int32_t layout, 
   op->layout     = layout;
   op->epb        = epb;
   op->own_launch = true;
+  op->line_only  = elems_per_block > 0;
   return CEED_MI355_SUCCESS;
 }
 
@@ -1141,6 +1143,21 @@ extern "C" int CeedMi355OperatorGetLaunch(CeedMi355Operator op, int32_t *layout,
   MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
   if (layout) *layout = op->layout;
   if (elems_per_block) *elems_per_block = op->epb;
+  return CEED_MI355_SUCCESS;
+}
+
+extern "C" int CeedMi355OperatorGetKernel(CeedMi355Operator op, int32_t *kernel, int32_t *gather) {
+  MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
+  int64_t most = 0;  // elements of the largest launch
+  for (size_t c = 0; c + 1 < op->color_start.size(); c++) most = std::max<int64_t>(most, op->color_start[c + 1] - op->color_start[c]);
+  if (kernel)
+    *kernel = op->scatter == CEED_MI355_PLAN_BRICK                             ? CEED_MI355_KERNEL_BRICK
+              : mi355::plan_recomputes(op) && mi355::elements_take(op, most) ? CEED_MI355_KERNEL_ELEMENTS
+              : op->layout == mi355::kLayoutLines                             ? CEED_MI355_KERNEL_LINES
+              : op->layout == mi355::kLayoutPoints                            ? CEED_MI355_KERNEL_POINTS
+                                                                              : CEED_MI355_KERNEL_COLUMNS;
+  if (gather)
+    *gather = (op->scatter == 0 && !mi355::plan_sums_last(op)) || op->scatter == CEED_MI355_PLAN_SPLIT || op->scatter == CEED_MI355_PLAN_BRICK;
   return CEED_MI355_SUCCESS;
 }
 
@@ -1170,15 +1187,14 @@ extern "C" int CeedMi355OperatorAutotune(CeedMi355Operator op, int32_t reps, int
   }
   if (op->scalar_type == CEED_MI355_FP64) tune_fill<double><<<mi355_blocks(op->l_size, 256, 4096), 256, 0, s>>>(op->l_size, (double *)u);
   else tune_fill<float><<<mi355_blocks(op->l_size, 256, 4096), 256, 0, s>>>(op->l_size, (float *)u);
-  const int start = op->epb, start_layout = op->layout;
-  int       best = start, best_layout = start_layout;
-  float     bms  = 1e30f;
+  const Launch start{op->layout, op->epb, op->line_only};
+  Launch       best = start;
+  float        bms  = 1e30f;
   int       err  = hipGetLastError() == hipSuccess ? CEED_MI355_SUCCESS : CEED_MI355_ERROR_BACKEND;
   if (err) mi355::set_error("autotune: the fill of the scratch input failed to launch");
   // ms per apply of one launch shape: a warm-up apply, then n timed applies
-  auto time_launch = [&](int layout, int epb, int n, float *ms) -> int {
-    op->layout = layout;
-    op->epb    = epb;
+  auto time_launch = [&](const Launch &l, int n, float *ms) -> int {
+    set_launch(op, l);
     int e      = CeedMi355OperatorApply(op, u, v, s);
     if (e) return e;
     MI355_HIP(hipEventRecord(t0, s));
@@ -1191,16 +1207,25 @@ extern "C" int CeedMi355OperatorAutotune(CeedMi355Operator op, int32_t reps, int
     return CEED_MI355_SUCCESS;
   };
   struct Cand {
-    float ms;
-    int   layout, epb;
+    float  ms;
+    Launch l;
   };
   std::vector<Cand> cands;
+  auto try_launch = [&](const Launch &l) {
+    float ms = 0;
+    err = time_launch(l, reps, &ms);
+    if (!err) cands.push_back({ms, l});
+  };
+  // one thread per element where it may take the plan's launches, beside the
+  // line kernel with each count (a smaller plan leaves it open for larger ones)
+  set_launch(op, {mi355::kLayoutLines, op->scatter == CEED_MI355_PLAN_SEGMENT ? op->seg_max : plan_default_epb(op, mi355::kLayoutLines), false});
+  int32_t kernel = 0;
+  if (!err) err = CeedMi355OperatorGetKernel(op, &kernel, nullptr);
+  const bool elements = kernel == CEED_MI355_KERNEL_ELEMENTS;
+  if (!err && elements) try_launch({op->layout, op->epb, false});
   for (int layout = mi355::kLayoutColumns; layout <= mi355::kLayoutPoints && !err; layout++) {
     for (int epb = 1; epb * mi355::layout_threads(op->Q, layout) <= mi355::max_threads(layout) && !err; epb++) {
-      if (!plan_admissible(op, layout, epb)) continue;
-      float ms = 0;
-      err = time_launch(layout, epb, reps, &ms);
-      if (!err) cands.push_back({ms, layout, epb});
+      if (plan_admissible(op, layout, epb)) try_launch({layout, epb, elements});
     }
   }
   // launches within a few per cent of each other swap places from one timing
@@ -1211,21 +1236,20 @@ extern "C" int CeedMi355OperatorAutotune(CeedMi355Operator op, int32_t reps, int
   for (int round = 0; round < 2 && cands.size() > 1 && !err; round++)
     for (Cand &c : cands) {
       float ms = 0;
-      err = time_launch(c.layout, c.epb, 2 * reps, &ms);
+      err = time_launch(c.l, 2 * reps, &ms);
       if (err) break;
       c.ms = std::min(c.ms, ms);
     }
   for (const Cand &c : cands)
-    if (c.ms < bms) bms = c.ms, best = c.epb, best_layout = c.layout;
-  op->epb    = err ? start : best;
-  op->layout = err ? start_layout : best_layout;
+    if (c.ms < bms) bms = c.ms, best = c.l;
+  set_launch(op, err ? start : best);
   release();
   if (err) return err;
   {
     std::lock_guard<std::mutex> lock(g_tune_mutex);
-    g_tuned[tune_key(op)] = std::make_pair(best_layout, best);
+    g_tuned[tune_key(op)] = best;
   }
-  if (best_epb) *best_epb = best;
+  if (best_epb) *best_epb = best.epb;
   if (best_ms) *best_ms = bms;
   return CEED_MI355_SUCCESS;
 }

@@ -742,6 +742,22 @@ static int OperatorApply(CeedOperator op, CeedVector in, CeedVector out, CeedReq
   return CEED_ERROR_SUCCESS;
 }
 
+/* Name of the path the operator's applies take (include/ceed-mi355.h) */
+int CeedMi355OperatorGetPath(CeedOperator op, const char **path) {
+  OperatorData *d;
+  Ceed          ceed;
+  bool          is_composite;
+  CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
+  CeedCallBackend(CeedOperatorIsComposite(op, &is_composite));
+  CeedCheck(!is_composite, ceed, CEED_ERROR_MINOR, "a composite operator has a path for each of its sub-operators");
+  CeedCallBackend(CeedDestroy(&ceed));
+  CeedCallBackend(CeedOperatorCheckReady(op));
+  CeedCallBackend(CeedOperatorGetData(op, &d));
+  CeedCallBackend(setup(op, d));
+  *path = d->jit ? "fused-qfunction" : d->fused ? "fused" : d->points ? "points" : "staged";
+  return CEED_ERROR_SUCCESS;
+}
+
 /* Diagonal of the operator (Jacobi preconditioning): the fused plan's
  * diagonal kernel; the staged path has no diagonal assembly. */
 static int assemble_diagonal(CeedOperator op, CeedVector assembled, bool add) {

@@ -244,6 +244,12 @@ class HexOperator:
         call("CeedMi355OperatorGetLaunch", self._h, C.byref(layout), C.byref(epb))
         return layout.value, epb.value
 
+    def kernel(self) -> tuple[str, bool]:
+        """The kernel apply runs with the current launch, and whether E^T is finished by a launch of its own after it."""
+        kernel, gather = C.c_int32(), C.c_int32()
+        call("CeedMi355OperatorGetKernel", self._h, C.byref(kernel), C.byref(gather))
+        return ("columns", "lines", "points", "elements", "brick")[kernel.value], bool(gather.value)
+
     def autotune(self, reps: int = 5) -> tuple[int, float]:
         """Pick the fastest (thread layout, elements per workgroup) for this plan; returns (epb, ms per apply)."""
         best, ms = C.c_int32(), C.c_double()
