@@ -267,6 +267,12 @@ __global__ void __launch_bounds__(256) geo_qdata(int64_t num_elem, int Q, int qf
   }
 }
 
+// Device memory of one call
+struct TempBuffer {
+  void *p = nullptr;
+  ~TempBuffer() { (void)hipFree(p); }
+};
+
 // The plan's stored factors are no longer its trilinear geometry's: for the graphs captured while they were
 __global__ void mark_replaced(int32_t *turn) { turn[0] = 0, turn[1] = 1; }
 
@@ -430,7 +436,7 @@ int build_transpose_map(CeedMi355Operator op, const int32_t *offsets) {
   MI355_HIP(hipMemcpy(op->d_tpos, pos.data(), sizeof(int32_t) * pos.size(), hipMemcpyHostToDevice));
   // line_last: every L entry has a contribution (the gather also zeroes the
   // others), and the elements fit its workgroups at the most there can be in one
-  bool last = mi355::line_takes_last(op->P, op->num_comp) && op->num_elem <= mi355::kLastWorkgroups * (256 / (op->Q * op->Q));
+  bool last = op->qf != kQfJit && mi355::line_takes_last(op->P, op->num_comp) && op->num_elem <= mi355::kLastWorkgroups * (256 / (op->Q * op->Q));
   for (int64_t t = 0; t < op->l_size && last; t++) last = row[t] < row[t + 1];
   if (last) {
     MI355_HIP(hipMalloc(&op->d_tcount, sizeof(int32_t) * (size_t)op->l_size));
@@ -918,40 +924,57 @@ extern "C" int CeedMi355OperatorBuildQData(CeedMi355Operator op, int build, int3
   memcpy(mats.data(), mesh_interp_1d_host, sizeof(double) * Q * PM);
   mi355::collocated_grad(PM, Q, mesh_interp_1d_host, mesh_grad_1d_host, &mats[Q * PM]);
   memcpy(&mats[Q * PM + Q * Q], q_weight_1d_host, sizeof(double) * Q);
-  int32_t *d_mo   = nullptr;
-  double  *d_mats = nullptr;
-  MI355_HIP(hipMalloc(&d_mo, sizeof(int32_t) * (mo.size() + 1)));
-  MI355_HIP(hipMalloc(&d_mats, sizeof(double) * mats.size()));
-  MI355_HIP(hipMemcpyAsync(d_mo, mo.data(), sizeof(int32_t) * mo.size(), hipMemcpyHostToDevice, s));
-  MI355_HIP(hipMemcpyAsync(d_mats, mats.data(), sizeof(double) * mats.size(), hipMemcpyHostToDevice, s));
-  int ierr;
   const int64_t blk = elem_block(op);
-  bool                trilinear = false;
-  std::vector<double>  pts(2 * Q);  // pts, turn: read by the copies below until the synchronisation
-  const int32_t        turn[2] = {1, 0};
-  if (PM == 2 && linear_mesh_basis(Q, mesh_interp_1d_host, mesh_grad_1d_host)) {
+  // a linear mesh basis: the elements' trilinear maps, kept where the plan's applies recompute the factors from them
+  const bool            linear    = PM == 2 && linear_mesh_basis(Q, mesh_interp_1d_host, mesh_grad_1d_host);
+  mi355::GeoLinesFn     geo_lines = op->scalar_type == CEED_MI355_FP64 ? mi355::pick_geo_f64(op->P, Q, op->num_comp, op->qf)
+                                                                       : mi355::pick_geo_f32(op->P, Q, op->num_comp, op->qf);
+  const bool            trilinear = linear && geo_lines && mi355::geo_pays(Q, op->qf, op->num_comp, op->scalar_bytes);
+  std::vector<double>   pts(2 * Q);  // pts, turn: read by the copies below until the synchronisation
+  const int32_t         turn[2] = {1, 0};
+  const size_t          geo_bytes = sizeof(double) * mi355::kGeoStride * ((size_t)op->num_elem + 1), pts_bytes = sizeof(double) * pts.size();
+  TempBuffer            mo_buf, mats_buf, geo_buf, pts_buf;
+  // from here on a failure leaves a plan that reads whatever factors it holds, not one that recomputes half-written ones
+  const bool was_valid = op->geo_valid;
+  op->geo_valid        = false;
+  MI355_HIP(hipMalloc(&mo_buf.p, sizeof(int32_t) * (mo.size() + 1)));
+  MI355_HIP(hipMemcpyAsync(mo_buf.p, mo.data(), sizeof(int32_t) * mo.size(), hipMemcpyHostToDevice, s));
+  const int32_t *d_mo = (const int32_t *)mo_buf.p;
+  if (linear) {
     for (int q = 0; q < Q; q++) pts[q] = mesh_interp_1d_host[2 * q + 1] - mesh_interp_1d_host[2 * q], pts[Q + q] = q_weight_1d_host[q];
-    if (!op->d_geo) MI355_HIP(hipMalloc(&op->d_geo, sizeof(double) * mi355::kGeoStride * ((size_t)op->num_elem + 1)));
-    if (!op->d_geo_pts) MI355_HIP(hipMalloc(&op->d_geo_pts, sizeof(double) * pts.size()));
-    if (!op->d_geo_turn) MI355_HIP(hipMalloc(&op->d_geo_turn, sizeof(turn)));
-    MI355_HIP(hipMemcpyAsync(op->d_geo_pts, pts.data(), sizeof(double) * pts.size(), hipMemcpyHostToDevice, s));
-    MI355_HIP(hipMemcpyAsync(op->d_geo_turn, turn, sizeof(turn), hipMemcpyHostToDevice, s));
+    if (trilinear) {
+      if (!op->d_geo) MI355_HIP(hipMalloc(&op->d_geo, geo_bytes));
+      if (!op->d_geo_pts) MI355_HIP(hipMalloc(&op->d_geo_pts, pts_bytes));
+      if (!op->d_geo_turn) MI355_HIP(hipMalloc(&op->d_geo_turn, sizeof(turn)));
+      MI355_HIP(hipMemcpyAsync(op->d_geo_turn, turn, sizeof(turn), hipMemcpyHostToDevice, s));
+      op->geo_lines = geo_lines;
+    } else {
+      MI355_HIP(hipMalloc(&geo_buf.p, geo_bytes));
+      MI355_HIP(hipMalloc(&pts_buf.p, pts_bytes));
+    }
+    double *d_geo = trilinear ? op->d_geo : (double *)geo_buf.p, *d_pts = trilinear ? op->d_geo_pts : (double *)pts_buf.p;
+    MI355_HIP(hipMemcpyAsync(d_pts, pts.data(), pts_bytes, hipMemcpyHostToDevice, s));
     const int64_t q3 = (int64_t)Q * Q * Q;
-    geo_coefficients<<<mi355_blocks(op->num_elem * 3, 256), 256, 0, s>>>(op->num_elem, d_mo, mesh_comp_stride, coords, op->d_geo);
+    geo_coefficients<<<mi355_blocks(op->num_elem * 3, 256), 256, 0, s>>>(op->num_elem, d_mo, mesh_comp_stride, coords, d_geo);
     if (op->scalar_type == CEED_MI355_FP64)
-      geo_qdata<double><<<mi355_blocks(op->num_elem * q3, 256), 256, 0, s>>>(op->num_elem, Q, build == 0, blk, op->d_geo, op->d_geo_pts, (double *)op->d_qdata);
-    else geo_qdata<float><<<mi355_blocks(op->num_elem * q3, 256), 256, 0, s>>>(op->num_elem, Q, build == 0, blk, op->d_geo, op->d_geo_pts, (float *)op->d_qdata);
-    ierr          = hipGetLastError() == hipSuccess ? CEED_MI355_SUCCESS : CEED_MI355_ERROR_BACKEND;
-    op->geo_lines = op->scalar_type == CEED_MI355_FP64 ? mi355::pick_geo_f64(op->P, Q, op->num_comp, op->qf) : mi355::pick_geo_f32(op->P, Q, op->num_comp, op->qf);
-    trilinear     = ierr == CEED_MI355_SUCCESS && op->geo_lines && mi355::geo_pays(Q, op->qf, op->num_comp, op->scalar_bytes);
-  } else if (op->scalar_type == CEED_MI355_FP64)
-    ierr = dispatch_build<double>(Q, build, op->num_elem, PM, d_mo, mesh_comp_stride, coords, d_mats, blk, (double *)op->d_qdata, s);
-  else ierr = dispatch_build<float>(Q, build, op->num_elem, PM, d_mo, mesh_comp_stride, coords, d_mats, blk, (float *)op->d_qdata, s);
-  if (!ierr && !trilinear) ierr = factors_replaced(op, s);
+      geo_qdata<double><<<mi355_blocks(op->num_elem * q3, 256), 256, 0, s>>>(op->num_elem, Q, build == 0, blk, d_geo, d_pts, (double *)op->d_qdata);
+    else geo_qdata<float><<<mi355_blocks(op->num_elem * q3, 256), 256, 0, s>>>(op->num_elem, Q, build == 0, blk, d_geo, d_pts, (float *)op->d_qdata);
+    MI355_LAUNCH_CHECK();
+  } else {
+    MI355_HIP(hipMalloc(&mats_buf.p, sizeof(double) * mats.size()));
+    MI355_HIP(hipMemcpyAsync(mats_buf.p, mats.data(), sizeof(double) * mats.size(), hipMemcpyHostToDevice, s));
+    const double *d_mats = (const double *)mats_buf.p;
+    const int     ierr   = op->scalar_type == CEED_MI355_FP64
+                               ? dispatch_build<double>(Q, build, op->num_elem, PM, d_mo, mesh_comp_stride, coords, d_mats, blk, (double *)op->d_qdata, s)
+                               : dispatch_build<float>(Q, build, op->num_elem, PM, d_mo, mesh_comp_stride, coords, d_mats, blk, (float *)op->d_qdata, s);
+    if (ierr) return ierr;
+  }
+  if (!trilinear) {
+    const int ierr = factors_replaced(op, s);
+    if (ierr) return ierr;
+  }
   MI355_HIP(hipStreamSynchronize(s));
-  (void)hipFree(d_mo);
-  (void)hipFree(d_mats);
-  if (ierr) return ierr;
+  op->geo_valid = was_valid;
   set_geo_valid(op, trilinear);
   if (op->qf == kQfDiffusionKappa) {
     // kappa slot defaults to 1 until CeedMi355OperatorSetKappa
