@@ -376,12 +376,16 @@ bool admissible(int P, int Q, int qf, int num_comp, int scalar_bytes, int layout
 
 int plan_default_epb(const CeedMi355Operator op, int layout) {
   if (layout == mi355::kLayoutLines && op->geo_valid) return mi355::geo_default_epb(op->Q);
-  // three components work three times as long on an element's factors: with
-  // the transpose map, whose one launch fills the GPU, full wavefronts beat
-  // small workgroups (MI355X, 2-4M DoFs, us per apply: Q = 5 5 elements 74.9,
-  // 2 elements 79.7, with colours 138 and 126; Q = 7 5 elements 125, one 131)
-  if (layout == mi355::kLayoutLines && op->num_comp == 3 && op->scalar_bytes == 8 && op->qf == kQfDiffusion && op->scatter == 0 &&
-      (op->Q == 5 || op->Q == 7))
+  // three components work three times as long on an element's factors: at
+  // Q = 5 with the transpose map, once its one launch fills the GPU several
+  // times over, full wavefronts beat small workgroups (MI355X, us per apply, 2
+  // elements / 5: P = 4 2197 elements 16.8 / 16.7, 12167 46.5 / 48.6, 17576 63.3
+  // / 63.0, 24389 82.3 / 78.5, 46656 146 / 131, 110592 327 / 320; P = 5 2744
+  // elements 23.1 / 24.6, 10648 54.3 / 54.0, 19683 85.6 / 85.1; in colours two are
+  // better).  Not at Q = 7 (one / 5: 512 elements 21.9 / 25.7, 2744 42.5 / 48.5,
+  // 8000 103 / 108, 10648 130 / 127, 24389 292 / 296).
+  if (layout == mi355::kLayoutLines && op->num_comp == 3 && op->scalar_bytes == 8 && op->qf == kQfDiffusion && op->scatter == 0 && op->Q == 5 &&
+      op->num_elem >= 16384)
     return 5;
   return mi355::default_epb(op->P, op->Q, op->qf, op->num_comp, op->scalar_bytes, layout);
 }

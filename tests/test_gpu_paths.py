@@ -124,3 +124,12 @@ def test_operator_paths(cuda, monkeypatch, name, passive_strides, path):
     assert make().path() == path
     monkeypatch.setenv("CEED_MI355_FUSE_QFUNCTIONS", "0")
     assert make().path() == ("fused" if path == "fused" else "staged")
+
+
+@pytest.mark.parametrize("n,p,Q,epb", [(25, 3, 5, 2), (26, 3, 5, 5), (4, 5, 7, 1)])
+def test_three_component_workgroups(cuda, n, p, Q, epb):
+    """Stored factors, three components, transpose map: full wavefronts at Q = 5 from 16384 elements, not at Q = 7."""
+    m = hex_mesh(n, p, seed=1)
+    op = ops.HexOperator(ops.QF_DIFFUSION, m.offsets, m.num_elem, p + 1, Q, 3 * m.num_nodes, num_comp=3, comp_stride=m.num_nodes, scatter="tmap")
+    op.set_layout(ops.LAYOUT_LINES)
+    assert op.launch() == (ops.LAYOUT_LINES, epb)
