@@ -81,7 +81,7 @@ constexpr int max_threads(int) { return 256; }
 int default_epb(int P, int Q, int qf, int num_comp, int scalar_bytes, int layout);
 // Whether a plan of this kind recomputes trilinear geometric factors in the
 // line kernel, and its elements per workgroup then (operator_hex.hip).
-bool geo_pays(int Q, int qf, int num_comp, int scalar_bytes);
+bool geo_pays(int P, int Q, int qf, int num_comp, int scalar_bytes);
 int  geo_default_epb(int Q);
 int lds_bytes(int P, int Q, int qf, int num_comp, int epb, int scalar_bytes, int layout);
 // Threads and LDS bytes of the brick kernel's workgroup for a brick of ns

@@ -45,12 +45,19 @@ int64_t brick_lds_bytes(int P, int Q, int qf, int scalar_bytes, const int *shape
 // same, which costs as much as it saves at Q = 8 (0.069 / 0.069) and Q = 10
 // (0.084 / 0.082), not at Q = 7 (0.093 / 0.082) or Q = 9 (0.087 / 0.077),
 // whose elements fill the wavefronts less well; three components share one
-// read of the factors (Q = 4: 0.210 / 0.214; Q = 3 0.654 / 0.620, Q = 5
-// 0.128 / 0.112, Q = 8 0.109 / 0.098).
-bool geo_pays(int Q, int qf, int num_comp, int scalar_bytes) {
+// read of the factors: in FP64 only Q = 4 gains nothing (0.203 / 0.204; Q = 3
+// 0.657 / 0.579, Q = 5 0.143 / 0.127, Q = 7 0.130 / 0.114, Q = 8 0.119 / 0.105),
+// in FP32 (us, P = Q - 1, at 0.5M, 4M and 24M DoFs in their default E^T) Q = 3
+// 471 / 417 (4M), Q = 5 19.5 / 20.8, 88 / 93, 448 / 447, Q = 6 20.8 / 21.8, 76 /
+// 77, 394 / 400, Q = 7 21.9 / 25.8, 82 / 84, 441 / 433, Q = 8 23.8 / 24.6, 71 / 70,
+// 369 / 377, Q = 9 27.2 / 27.6, 85 / 82, 417 / 398, Q = 10 30.8 / 31.6, 94 / 92,
+// 477 / 465, and with P = Q (4M and 24M) Q = 5 58 / 55, 306 / 280, Q = 6 59 / 57,
+// 350 / 328, Q = 7 60 / 63, 327 / 323, Q = 8 58 / 56 (4M).
+bool geo_pays(int P, int Q, int qf, int num_comp, int scalar_bytes) {
   if (qf != kQfDiffusion && qf != kQfDiffusionKappa) return false;
-  if (scalar_bytes == 4 && num_comp == 1) return Q != 8 && Q != 10;
-  return num_comp == 1 || Q != 4;
+  if (scalar_bytes == 8) return num_comp == 1 || Q != 4;
+  if (num_comp == 1) return Q != 8 && Q != 10;
+  return Q <= 3 || Q >= 9 || (P == Q && (Q == 5 || Q == 6));
 }
 
 // Elements per workgroup with recomputed factors: the count of at most 256
@@ -933,7 +940,7 @@ extern "C" int CeedMi355OperatorBuildQData(CeedMi355Operator op, int build, int3
   const bool            linear    = PM == 2 && linear_mesh_basis(Q, mesh_interp_1d_host, mesh_grad_1d_host);
   mi355::GeoLinesFn     geo_lines = op->scalar_type == CEED_MI355_FP64 ? mi355::pick_geo_f64(op->P, Q, op->num_comp, op->qf)
                                                                        : mi355::pick_geo_f32(op->P, Q, op->num_comp, op->qf);
-  const bool            trilinear = linear && geo_lines && mi355::geo_pays(Q, op->qf, op->num_comp, op->scalar_bytes);
+  const bool            trilinear = linear && geo_lines && mi355::geo_pays(op->P, Q, op->qf, op->num_comp, op->scalar_bytes);
   std::vector<double>   pts(2 * Q);  // pts, turn: read by the copies below until the synchronisation
   const int32_t         turn[2] = {1, 0};
   const size_t          geo_bytes = sizeof(double) * mi355::kGeoStride * ((size_t)op->num_elem + 1), pts_bytes = sizeof(double) * pts.size();

@@ -21,7 +21,9 @@ QF_FILE = Path(__file__).resolve().parent / "qfunctions" / "t-points.h"
 @pytest.mark.parametrize("kind,nc,p,Q,fp32,recomputes", [
     (1, 1, 1, 2, False, True), (1, 1, 4, 6, False, True), (1, 1, 6, 8, False, True), (1, 1, 8, 10, False, True), (1, 1, 5, 7, True, True),
     (1, 1, 6, 8, True, False), (1, 3, 2, 3, False, True), (1, 3, 3, 4, False, False), (1, 3, 6, 8, False, True), (2, 1, 3, 4, False, True),
-    (0, 1, 3, 5, False, False)])
+    (0, 1, 3, 5, False, False), (1, 3, 2, 3, True, True), (1, 3, 3, 4, True, False), (1, 3, 3, 5, True, False), (1, 3, 4, 5, True, True),
+    (1, 3, 4, 6, True, False), (1, 3, 5, 6, True, True), (1, 3, 6, 7, True, False), (1, 3, 7, 8, True, False), (1, 3, 7, 9, True, True),
+    (1, 3, 8, 10, True, True)])
 def test_recomputed_or_stored(cuda, kind, nc, p, Q, fp32, recomputes):
     m = hex_mesh(2, p, seed=1)
     op = ops.HexOperator.from_mesh(kind, m, Q=Q, num_comp=nc, dtype=torch.float32 if fp32 else torch.float64, scatter="tmap")
@@ -32,8 +34,13 @@ def test_recomputed_or_stored(cuda, kind, nc, p, Q, fp32, recomputes):
     op.set_layout(ops.LAYOUT_LINES, 1)
     assert op.recomputes_factors() == recomputes
     if kind != 2:
+        u = torch.from_numpy(np.random.default_rng(p).uniform(-1, 1, nc * m.num_nodes)).to(op.dtype).cuda()
+        v, w = torch.empty_like(u), torch.empty_like(u)
+        op.apply(u, v)
         op.set_qdata(op.get_qdata())
         assert not op.recomputes_factors()
+        op.apply(u, w)
+        assert torch.equal(v, w)
     for scatter in ("brick", "segment") if kind != 2 else ():
         assert not ops.HexOperator.from_mesh(kind, m, Q=Q, num_comp=nc, dtype=op.dtype, scatter=scatter).recomputes_factors()
 
