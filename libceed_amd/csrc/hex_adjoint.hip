@@ -513,7 +513,7 @@ int launch_adjoint(const CeedMi355Operator_private *op, const double *u, const d
                                                                     (const double *)op->d_mats, u, lam, v, (double *)op->d_evec, op->d_tpos, g);
   }
   MI355_LAUNCH_CHECK();
-  if (tmap) return transpose_gather(op, v, 1, s);
+  if (tmap) return transpose_gather(op, v, 1, nullptr, s);
   if (op->scatter == CEED_MI355_PLAN_SPLIT) return split_finish(op, v, 1, s);
   return CEED_MI355_SUCCESS;
 }

@@ -297,7 +297,7 @@ int launch_diag(const CeedMi355Operator_private *op, void *v, int add, hipStream
     const int err = launch_diag_elements<P, Q, T>(op, b, e, scatter, target, s);
     if (err) return err;
   }
-  if (tmap) return transpose_gather(op, v, !add, s);
+  if (tmap) return transpose_gather(op, v, !add, nullptr, s);
   if (split) return split_finish(op, v, !add, s);
   return CEED_MI355_SUCCESS;
 }

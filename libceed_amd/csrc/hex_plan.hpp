@@ -33,13 +33,21 @@ using GeoLinesFn = void (*)(const CeedMi355Operator_private *op, int64_t b, int6
 // one kernel / both: p=2 2k DoFs 7.6 / 9.1, p=3 0.9M 37.2 / 39.9, p=1 0.5M 77 /
 // 86, p=4 8M in eight colours 214 / 235.
 bool into_callers_graph(const CeedMi355Operator_private *op, hipStream_t s);
-// Kappa of the apply running on this thread (CeedMi355OperatorApplyKappa), nullptr for the plan's own.
-const double *kappa_of_apply();
-// The apply running on this thread wants its transpose_gather to form a dot product (apply_dot).
-bool gather_dot_wanted();
-using ApplyFn = int (*)(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s);
+// A dot product the gather forms on the way (apply_dot): the partial sums of u . v, nb of them, and *to = *from
+struct GatherDot {
+  const void   *u       = nullptr;
+  double       *partial = nullptr, *to = nullptr;
+  const double *from    = nullptr;
+  int           nb      = 0;
+};
+// What one apply may ask for beside v = A u
+struct ApplyExtras {
+  const double *kappa = nullptr;  // the caller's kappa, read and kept in the plan (the line kernel that recomputes the factors only)
+  GatherDot    *dot   = nullptr;  // formed where the apply overwrites v and ends in transpose_gather, which then sets nb
+};
+using ApplyFn = int (*)(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, const ApplyExtras &x, hipStream_t s);
 // v (=|+=) E^T evec by the plan's transpose map (operator_hex.hip)
-int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, hipStream_t s);
+int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, GatherDot *dot, hipStream_t s);
 // v = A u and, where the apply ends in transpose_gather, the partial sums of
 // u . v into partial (*nb of them, at most kDotBlocks), with *to = *from done
 // on the way; *nb = 0 where it does not (nothing but the apply is done then).
@@ -231,7 +239,7 @@ inline bool plan_sums_last(const CeedMi355Operator_private *op) {
 }
 
 template <int P, int Q, int NC, int QF, typename T>
-int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s) {
+int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, const ApplyExtras &x, hipStream_t s) {
   const int    nt     = Q * Q;
   const int    epb    = op->epb;
   const bool   lines  = op->layout == kLayoutLines;
@@ -274,7 +282,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
   // kScatterLast: frozen systems' contributions never arrive, a dot product
   // wants the gather, and where u and v overlap all of u is read first
   const size_t l_bytes = sizeof(T) * (size_t)op->l_size;
-  const bool   last    = plan_sums_last(op) && !gather_dot_wanted() &&
+  const bool   last    = plan_sums_last(op) && !x.dot &&
                     ((const char *)u + l_bytes <= (const char *)v || (const char *)v + l_bytes <= (const char *)u);
   for (size_t c = 0; c + 1 < op->color_start.size(); c++) {
     const int64_t b = op->color_start[c], e = op->color_start[c + 1];
@@ -285,7 +293,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
                                  : split ? kScatterSplit
                                          : (op->scatter == CEED_MI355_PLAN_ATOMIC ? kScatterAtomic : (overwrite ? kScatterOverwrite : kScatterAdd));
     if (lines) {
-      if (geo) op->geo_lines(op, b, e, scatter, u, target, kappa_of_apply(), two, s);
+      if (geo) op->geo_lines(op, b, e, scatter, u, target, x.kappa, two, s);
       if (!geo || two) {
         // (beside the recomputing kernel it mostly returns at once, the faster the fewer its workgroups)
         const int n = two && line_lds_bytes(Q, NC, QF, sizeof(T), false, 256 / nt) <= (size_t)kMaxLdsBytes ? 256 / nt : epb;
@@ -307,7 +315,7 @@ int launch_hex_apply(const CeedMi355Operator_private *op, const void *u, void *v
                                                                             op->d_tpos, op->d_elem_sys, op->d_sys_active);
   }
   MI355_LAUNCH_CHECK();
-  if (tmap && !last) return transpose_gather(op, v, overwrite, s);
+  if (tmap && !last) return transpose_gather(op, v, overwrite, x.dot, s);
   if (split) return split_finish(op, v, overwrite, s);
   return CEED_MI355_SUCCESS;
 }

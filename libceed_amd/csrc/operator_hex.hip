@@ -558,15 +558,6 @@ __global__ void __launch_bounds__(256) transpose_gather_dot_kernel(int64_t l_siz
   if (threadIdx.x == 0) partial[blockIdx.x] = sum[0];
 }
 
-// What apply_dot asks of the transpose_gather its apply ends in, on its own thread
-struct GatherDot {
-  const void   *u = nullptr;
-  double       *partial = nullptr, *to = nullptr;
-  const double *from = nullptr;
-  int           nb   = 0;
-};
-thread_local GatherDot *t_gather_dot = nullptr;
-
 // The same over chunks of L entries, one block per chunk; chunks of inactive
 // systems (batched solvers) are left out
 template <typename T>
@@ -610,9 +601,7 @@ int split_finish(const CeedMi355Operator_private *op, void *v, int overwrite, hi
   return CEED_MI355_SUCCESS;
 }
 
-bool gather_dot_wanted() { return t_gather_dot != nullptr; }
-
-int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, hipStream_t s) {
+int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite, GatherDot *dot, hipStream_t s) {
   if (op->d_gather_chunk_begin && op->d_sys_active && op->gather_num_chunks > 0) {
     const unsigned nb = (unsigned)op->gather_num_chunks;
     if (op->scalar_type == CEED_MI355_FP64)
@@ -624,8 +613,8 @@ int transpose_gather(const CeedMi355Operator_private *op, void *v, int overwrite
     MI355_LAUNCH_CHECK();
     return CEED_MI355_SUCCESS;
   }
-  if (t_gather_dot && overwrite) {
-    GatherDot &d = *t_gather_dot;
+  if (dot && overwrite) {
+    GatherDot &d = *dot;
     d.nb         = mi355_blocks(op->l_size, 256, kDotBlocks);
     if (op->scalar_type == CEED_MI355_FP64)
       transpose_gather_dot_kernel<double><<<d.nb, 256, 0, s>>>(op->l_size, op->d_trow, (const double *)op->d_evec, (const double *)d.u, (double *)v,
@@ -1086,10 +1075,33 @@ extern "C" int CeedMi355OperatorSetKappa(CeedMi355Operator op, const double *kap
 }
 
 namespace {
-thread_local const double *t_kappa = nullptr;  // set for the time of one ApplyKappa
+int apply_overwrite(CeedMi355Operator op, const void *u, void *v, const mi355::ApplyExtras &x, hipStream_t s) {
+  // first-touch entries are overwritten by the kernel; entries no element reaches are zeroed here
+  if (!op->covers_all || op->num_elem == 0) {
+    if (op->scalar_type == CEED_MI355_FP64)
+      fill_kernel<double><<<mi355_blocks(op->l_size, 256, 4096), 256, 0, s>>>(op->l_size, 0.0, (double *)v);
+    else fill_kernel<float><<<mi355_blocks(op->l_size, 256, 4096), 256, 0, s>>>(op->l_size, 0.0f, (float *)v);
+    MI355_LAUNCH_CHECK();
+  }
+  if (op->num_elem == 0) return CEED_MI355_SUCCESS;
+  return op->apply(op, u, v, 1, x, s);
+}
 }  // namespace
 
-const double *mi355::kappa_of_apply() { return t_kappa; }
+extern "C" int CeedMi355OperatorApply(CeedMi355Operator op, const void *u, void *v, void *stream) {
+  MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
+  return apply_overwrite(op, u, v, {}, (hipStream_t)stream);
+}
+
+int mi355::apply_dot(CeedMi355Operator op, const void *u, void *v, double *partial, double *to, const double *from, int *nb, hipStream_t s) {
+  GatherDot d;
+  d.u = u, d.partial = partial, d.to = to, d.from = from;
+  ApplyExtras x;
+  x.dot          = &d;
+  const int ierr = apply_overwrite(op, u, v, x, s);
+  *nb            = d.nb;
+  return ierr;
+}
 
 bool mi355::into_callers_graph(const CeedMi355Operator_private *op, hipStream_t s) { return !op->solver_graph && is_capturing(s); }
 
@@ -1103,40 +1115,15 @@ extern "C" int CeedMi355OperatorApplyKappa(CeedMi355Operator op, const double *k
     const int err = CeedMi355OperatorSetKappa(op, kappa, stream);
     return err ? err : CeedMi355OperatorApply(op, u, v, stream);
   }
-  t_kappa        = kappa;
-  const int ierr = CeedMi355OperatorApply(op, u, v, stream);
-  t_kappa        = nullptr;
-  return ierr;
+  mi355::ApplyExtras x;
+  x.kappa = kappa;
+  return apply_overwrite(op, u, v, x, (hipStream_t)stream);
 }
 
 extern "C" int CeedMi355OperatorApplyAdd(CeedMi355Operator op, const void *u, void *v, void *stream) {
   MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
   if (op->num_elem == 0) return CEED_MI355_SUCCESS;
-  return op->apply(op, u, v, 0, (hipStream_t)stream);
-}
-
-extern "C" int CeedMi355OperatorApply(CeedMi355Operator op, const void *u, void *v, void *stream) {
-  MI355_CHECK(op, CEED_MI355_ERROR_MAJOR, "null operator");
-  hipStream_t s = (hipStream_t)stream;
-  // first-touch entries are overwritten by the kernel; entries no element reaches are zeroed here
-  if (!op->covers_all || op->num_elem == 0) {
-    if (op->scalar_type == CEED_MI355_FP64)
-      fill_kernel<double><<<mi355_blocks(op->l_size, 256, 4096), 256, 0, s>>>(op->l_size, 0.0, (double *)v);
-    else fill_kernel<float><<<mi355_blocks(op->l_size, 256, 4096), 256, 0, s>>>(op->l_size, 0.0f, (float *)v);
-    MI355_LAUNCH_CHECK();
-  }
-  if (op->num_elem == 0) return CEED_MI355_SUCCESS;
-  return op->apply(op, u, v, 1, s);
-}
-
-int mi355::apply_dot(CeedMi355Operator op, const void *u, void *v, double *partial, double *to, const double *from, int *nb, hipStream_t s) {
-  GatherDot d;
-  d.u = u, d.partial = partial, d.to = to, d.from = from;
-  t_gather_dot   = &d;
-  const int ierr = CeedMi355OperatorApply(op, u, v, s);
-  t_gather_dot   = nullptr;
-  *nb            = d.nb;
-  return ierr;
+  return op->apply(op, u, v, 0, {}, (hipStream_t)stream);
 }
 
 extern "C" int CeedMi355OperatorSetLaunch(CeedMi355Operator op, int32_t elems_per_block) {

@@ -392,7 +392,7 @@ std::string slab_strides(int Q) {
   return to_string(mi355::line_row_stride(Q, 8)) + ", " + to_string(mi355::line_plane_stride(Q, 8));
 }
 
-int launch_jit(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, hipStream_t s) {
+int launch_jit(const CeedMi355Operator_private *op, const void *u, void *v, int overwrite, const mi355::ApplyExtras &x, hipStream_t s) {
   const int    Q = op->Q, nt = Q * Q, epb = op->epb;
   const size_t lds  = sizeof(double) * (size_t)epb * 2 * mi355::line_slab_entries(Q, 8);
   const bool   tmap = op->scatter == 0, split = op->scatter == CEED_MI355_PLAN_SPLIT;
@@ -415,7 +415,7 @@ int launch_jit(const CeedMi355Operator_private *op, const void *u, void *v, int 
     void          *args[] = {&eb, &ee, &scatter, &offsets, &q_data, &mats, &uu, &vv, &evec, &tpos, &elem_sys, &sys_active, &ctx};
     MI355_HIP(hipModuleLaunchKernel(op->jit->kernel, (unsigned)grid, 1, 1, epb * nt, 1, 1, (unsigned)lds, s, args, nullptr));
   }
-  if (tmap) return mi355::transpose_gather(op, v, overwrite, s);
+  if (tmap) return mi355::transpose_gather(op, v, overwrite, x.dot, s);
   if (split) return mi355::split_finish(op, v, overwrite, s);
   return CEED_MI355_SUCCESS;
 }
