@@ -768,6 +768,7 @@ static int assemble_diagonal(CeedOperator op, CeedVector assembled, bool add) {
   CeedCallBackend(setup(op, d));
   CeedCallBackend(CeedOperatorGetCeed(op, &ceed));
   CeedCheck(d->fused && !d->jit, ceed, CEED_ERROR_UNSUPPORTED, "diagonal assembly needs a gallery mass or diffusion operator on 3D tensor hexes");
+  CeedCallBackend(fused_sync_qdata(op, d));
   CeedCallBackend(CeedVectorGetArray(assembled, CEED_MEM_DEVICE, &da));
   CeedCallBackend(CeedMi355Check(ceed, CeedMi355OperatorAssembleDiagonal(d->hex, da, add, NULL)));
   CeedCallBackend(CeedVectorRestoreArray(assembled, &da));
