@@ -15,6 +15,8 @@ void set_error(const char *fmt, ...) {
   va_end(ap);
 }
 
+void touch_thread_storage() { asm volatile("" : : "r"(last_error)); }
+
 }  // namespace mi355
 
 extern "C" const char *CeedMi355GetLastError(void) { return mi355::last_error; }
