@@ -39,7 +39,7 @@ FP64_PEAK_TFLOPS = 78.6    # MI355X FP64 vector/matrix, vendor datasheet
 
 def alg_bytes(N: int, E: int, P: int, Q: int, ncomp: int = 1, qcomp: int = 6, s: int = 8, recomputed: bool = False) -> int:
     """Read u + write v + read q_data + read int32 offsets (each stream counted once); with the factors recomputed
-    the 21 doubles of the element's map in place of q_data."""
+    the 21 doubles of the element's map that matter in place of q_data (24 are stored and loaded)."""
     return s * ncomp * N * 2 + (8 * 21 * E if recomputed else s * qcomp * E * Q ** 3) + 4 * E * P ** 3
 
 
@@ -72,7 +72,7 @@ KERNEL_NAMES = {"columns": "hex_apply_kernel", "lines": "hex_apply_lines_kernel"
 
 
 def run_case(p: int, dofs: float, dtype, steps: int, warmup: int, seed: int = 0, scatter: str = "auto", epb: int = 0, num_comp: int = 1,
-             layout: int = 1):
+             layout: int = 1, stored: bool = False):
     import torch
 
     from libceed_amd import ops
@@ -85,8 +85,12 @@ def run_case(p: int, dofs: float, dtype, steps: int, warmup: int, seed: int = 0,
     g = torch.Generator(device="cuda").manual_seed(seed)
     u = (torch.rand(num_comp * m.num_nodes, dtype=torch.float64, device="cuda", generator=g) * 2 - 1).to(dtype)
     v = torch.zeros_like(u)
-    if epb:
+    if stored:
+        op.set_qdata(op.get_qdata())  # the caller's factors, which the plan reads
+    if epb > 0:
         op.set_layout(layout, epb)
+    elif epb < 0:
+        op.set_layout(layout)
     else:
         op.autotune(5)  # the library's (thread layout, elements per workgroup) tuner; results are bitwise the same for all
     layout, epb = op.launch()
@@ -514,7 +518,7 @@ def cpu_baseline(p: int = 4, n: int = 50, seconds: float = 10.0) -> dict | None:
 
 def measured_traffic(head: dict, dtype: str, num_comp: int):
     """HBM bytes per apply from the committed rocprofv3 counter summary of this workload (same order, size,
-    arithmetic, components, E^T mode and layout), and where it comes from.  A summary of another number of
+    arithmetic, components, E^T mode, layout and kind of factors), and where it comes from.  A summary of another number of
     elements per workgroup is used when none of this launch exists, and says so: it changes the order of the
     memory accesses, not the bytes the plan reads and writes."""
     best = None
@@ -526,6 +530,8 @@ def measured_traffic(head: dict, dtype: str, num_comp: int):
         w = d.get("workload", {})
         if (w.get("p"), w.get("dofs"), w.get("dtype"), w.get("scatter"), w.get("num_comp", 1), w.get("layout")) != (
                 head["p"], head["dofs"], dtype, head["scatter"], num_comp, head["layout"]):
+            continue
+        if w.get("factors") != head["factors"]:
             continue
         same = (w.get("layout"), w.get("elems_per_block")) == (head["layout"], head["elems_per_block"])
         src = d.get("source", f.name) + ("" if same else f" (launch {w.get('layout')} x {w.get('elems_per_block')}; this run's launch "
@@ -555,7 +561,10 @@ def main() -> None:
     ap.add_argument("--ncomp", type=int, default=1, choices=[1, 3],
                     help="components of the headline operator (the metric is scalar; 3 is the vector variant, for profiling)")
     ap.add_argument("--epb", type=int, default=0,
-                    help="elements per workgroup of the headline plan (default: autotuned; fixed values are for profiling)")
+                    help="elements per workgroup of the headline plan (default: autotuned; -1: the library's default; fixed values are "
+                         "for profiling)")
+    ap.add_argument("--stored", action="store_true",
+                    help="hand the headline plan its factors with set_qdata, so that it reads them (for profiling)")
     ap.add_argument("--layout", choices=LAYOUT_NAMES, default="lines",
                     help="thread layout of the headline plan when --epb is given")
     ap.add_argument("--copy-calibration", action="store_true",
@@ -582,7 +591,7 @@ def main() -> None:
                           "sum_bytes_read": 4 * nbytes, "ms_per_sum": ms_read, "GBs_read": 4 * nbytes / (ms_read * 1e-3) / 1e9}), flush=True)
         return
     head = run_case(args.p, args.dofs, torch.float64 if args.dtype == "f64" else torch.float32, args.steps, args.warmup, scatter=args.scatter,
-                    epb=args.epb, layout=LAYOUT_NAMES.index(args.layout), num_comp=args.ncomp)
+                    epb=args.epb, layout=LAYOUT_NAMES.index(args.layout), num_comp=args.ncomp, stored=args.stored)
     sweep = {}
     if not args.no_sweep:
         for p in range(1, 9):

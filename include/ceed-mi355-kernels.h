@@ -225,7 +225,10 @@ int CeedMi355OperatorApplyAdjointKappa(CeedMi355Operator op, const double *kappa
 int CeedMi355OperatorAssembleDiagonal(CeedMi355Operator op, void *diag, int add, void *stream);
 /* v += A u  (CeedOperatorApplyAdd, interface/ceed-operator.c:2313-2340). */
 int CeedMi355OperatorApplyAdd(CeedMi355Operator op, const void *u, void *v, void *stream);
-/* v  = A u  (CeedOperatorApply, interface/ceed-operator.c:2271-2294). */
+/* v  = A u  (CeedOperatorApply, interface/ceed-operator.c:2271-2294).  Applies,
+ * adjoints and diagonals of one plan must not overlap in time on several
+ * streams: they share the plan's E-vector or scratch (E^T modes other than
+ * colours and atomics), and small plans the counts of their contributions. */
 int CeedMi355OperatorApply(CeedMi355Operator op, const void *u, void *v, void *stream);
 /* Elements per workgroup of the fused kernel (1 <= epb, epb * Q^2 <= 256
  * threads, LDS <= 160 KiB, the gfx950 workgroup limit). */
@@ -256,7 +259,8 @@ enum {
 };
 int CeedMi355OperatorGetKernel(CeedMi355Operator op, int32_t *kernel, int32_t *gather);
 /* 1 if Apply recomputes the geometric factors from the elements' trilinear
- * maps with the current launch (it then reads 168 bytes per element of them),
+ * maps with the current launch (it then reads 192 bytes per element of them, 168
+ * of which matter),
  * 0 if it reads the stored ones. */
 int CeedMi355OperatorRecomputesFactors(CeedMi355Operator op, int32_t *yes);
 /* Autotuner (the reference has none: its hip-shared/hip-gen backends fix the

@@ -1,7 +1,7 @@
 // One thread per element, for the lowest order: with two nodes per direction
 // an element's whole diffusion apply fits one thread's registers, so there is
 // nothing to exchange through LDS and nothing to wait for (the line kernel at
-// Q = 3 runs nine threads per element through fourteen barriers and issues 4400
+// Q = 3 runs nine threads per element through eleven barriers and issues 4400
 // instructions per element, this one 2900).  The geometric factors come from
 // the element's trilinear map, whose coefficients a wavefront stages through
 // LDS (coalesced; a thread's own 21 then lie on an odd stride).  Bound by FP64

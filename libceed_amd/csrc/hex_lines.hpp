@@ -22,7 +22,9 @@
 // elements (geo_default_epb) and the in-place slabs count: MI355X, FP64
 // diffusion, 8M DoFs, ms per apply, stored factors / recomputed / recomputed
 // with the lines in place: p=2 0.621 / 0.462 / 0.445, p=4 0.357 / 0.254 /
-// 0.222, p=6 0.252 / 0.229 / 0.180, p=8 0.283 / 0.231 / 0.199.
+// 0.222, p=6 0.252 / 0.229 / 0.180, p=8 0.283 / 0.231 / 0.199 (applies one after
+// the other on one pair of vectors, with a spread of 3% between machines; on vectors and
+// plans that change from apply to apply p=4 takes 0.232 to 0.243).
 //
 // Thread t of an element's Q*Q threads plays these roles:
 //   column (qx, qy) = (t % Q, t / Q)                     z-contractions, pointwise D
@@ -30,8 +32,9 @@
 //   x-line of nodes (y, z) = (t % P, t / P), t < P*P     B_x, B_x^T
 //   y-line (qx, z) = (t % Q, t / Q), t < Q*P              B_y, B_y^T
 //   x-line (qy, qz) and y-line (qx, qz) = (t % Q, t / Q)  the collocated derivatives
-// Slabs are [z][y][x] with strides (Q*Q, Q, 1), padded at Q = 7, 8 against LDS
-// bank conflicts (line_row_stride, line_plane_stride).  A line's thread reads
+// Slabs are [z][y][x] with strides (Q*Q, Q, 1), padded against LDS bank
+// conflicts in FP64 at Q = 3, 4, 7 and 8 and in FP32 at Q = 8 (line_row_stride,
+// line_plane_stride, line_elem_pad).  A line's thread reads
 // all of it before it writes and no other thread touches it in that phase, so
 // lines are contracted in place: mass needs one slab per element, diffusion
 // two (the y-lines of the derivative are read before and written after the
