@@ -42,11 +42,10 @@ __global__ void __launch_bounds__(256, (P <= 5 ? 4 : 1)) hex_diag_kernel(int64_t
                                                        const int32_t *__restrict__ offsets, int32_t comp_stride, const T *__restrict__ q_data,
                                                        const T *__restrict__ mats, const double *__restrict__ geo,
                                                        const double *__restrict__ geo_pts, T *__restrict__ v, T *__restrict__ evec,
-                                                       const int32_t *__restrict__ tpos, const int32_t *__restrict__ turn) {
+                                                       const int32_t *__restrict__ tpos) {
   constexpr int NT = Q * Q, P3 = P * P * P, Q3 = Q * Q * Q, QP = Q * P, QC = QfTraits<QF>::kComps, NS = diag_slabs(QF), NA = QF == kQfMass ? 1 : 6;
   constexpr int SR = line_row_stride(Q, sizeof(T)), SP = line_plane_stride(Q, sizeof(T)), SLAB = P * SP;
   extern __shared__ __align__(16) unsigned char lds_raw[];
-  if (turn && !*turn) return;  // in a caller's graph, where the other of the two kernels runs
   const int     epb = blockDim.x / NT, le = threadIdx.x / NT, t = threadIdx.x - le * NT;
   T            *A  = reinterpret_cast<T *>(lds_raw) + (size_t)le * NS * SLAB;
   auto          at = [](int k, int z, int y, int x) { return k * SLAB + z * SP + y * SR + x; };
@@ -251,17 +250,17 @@ int launch_diag_elements(const CeedMi355Operator_private *op, int64_t b, int64_t
 #define MI355_DIAG_LAUNCH(QF, GEO)                                                                                                        \
   hex_diag_kernel<P, Q, QF, GEO, T><<<grid, nt, epb * per, s>>>(b, e, scatter, op->num_comp, op->d_offsets, op->comp_stride,              \
                                                                 (const T *)op->d_qdata, (const T *)op->d_mats, op->d_geo, op->d_geo_pts, v, \
-                                                                (T *)op->d_evec, op->d_tpos, two ? op->d_geo_turn + !GEO : nullptr)
-  const bool two = op->geo_valid && into_callers_graph(op, s), stored = !op->geo_valid || two;
-  if (op->qf == kQfMass) {
-    MI355_DIAG_LAUNCH(kQfMass, false);
-  } else if (op->qf == kQfDiffusion) {
-    if (op->geo_valid) MI355_DIAG_LAUNCH(kQfDiffusion, true);
-    if (stored) MI355_DIAG_LAUNCH(kQfDiffusion, false);
-  } else {
-    if (op->geo_valid) MI355_DIAG_LAUNCH(kQfDiffusionKappa, true);
-    if (stored) MI355_DIAG_LAUNCH(kQfDiffusionKappa, false);
-  }
+                                                                (T *)op->d_evec, op->d_tpos)
+  // (a graph of the caller's may be replayed after the plan's factors have changed kind: it takes the kernel that
+  // reads them, which are the geometry's while that is the plan's, and every replay follows the plan; two kernels by
+  // turns as in the apply cost the calls outside graphs 0.2 us of 13 at p=6, 48 elements, one more test in each.
+  // MI355X, FP64, 1M DoFs, us recomputed / read: p=1 208 / 504, p=2 60 / 83, p=4 40 / 53, p=8 45 / 46)
+  const bool geo = op->geo_valid && !into_callers_graph(op, s);
+  if (op->qf == kQfMass) MI355_DIAG_LAUNCH(kQfMass, false);
+  else if (op->qf == kQfDiffusion && geo) MI355_DIAG_LAUNCH(kQfDiffusion, true);
+  else if (op->qf == kQfDiffusion) MI355_DIAG_LAUNCH(kQfDiffusion, false);
+  else if (geo) MI355_DIAG_LAUNCH(kQfDiffusionKappa, true);
+  else MI355_DIAG_LAUNCH(kQfDiffusionKappa, false);
 #undef MI355_DIAG_LAUNCH
   MI355_LAUNCH_CHECK();
   return CEED_MI355_SUCCESS;
@@ -322,6 +321,7 @@ extern "C" int CeedMi355OperatorAssembleDiagonal(CeedMi355Operator op, void *dia
   MI355_CHECK(op->qf == mi355::kQfMass || op->qf == mi355::kQfDiffusion || op->qf == mi355::kQfDiffusionKappa, CEED_MI355_ERROR_UNSUPPORTED,
               "diagonal assembly needs a mass or diffusion plan");
   if (op->num_elem == 0) return CEED_MI355_SUCCESS;
+  mi355::touch_thread_storage();
   if (op->scatter == CEED_MI355_PLAN_BRICK && !op->d_evec)  // element-major E-vector of the brick plan's diagonal, made once
     MI355_HIP(hipMalloc(&op->d_evec, (size_t)op->scalar_bytes * ((size_t)op->num_elem * op->num_comp * op->P * op->P * op->P + 1)));
   auto fn = op->scalar_type == CEED_MI355_FP64 ? mi355::pick_diag<double>(op->P, op->Q) : mi355::pick_diag<float>(op->P, op->Q);

@@ -13,7 +13,7 @@ namespace mi355 {
 void set_error(const char *fmt, ...);
 
 // Take the address of this library's thread-local storage (2 ns), which every
-// apply does.  Until a thread has done so since the library was loaded, glibc
+// apply, adjoint and diagonal does.  Until a thread has done so since the library was loaded, glibc
 // sends its accesses to all other libraries' thread-local storage through a
 // slow path (the thread's table of modules is older than the newest module), and
 // the interpreter and torch around a small apply make many: from Python 8.8 us
